@@ -1,0 +1,146 @@
+"""GPU parity of the basin sweep (batched TFCE maxima through the basins of a
+map's local maxima) against the C oracle, at the sizes and values where it can
+go wrong: workgroup edges of the vertex passes, every LDS size of the basin
+sweep and the element-wise sweep behind it, ties, NaN, infinities, one sign,
+empty images, images without neighbours.
+
+Bar: bit-exact float32 for H = 2, E = 1 (each increment is one correctly
+rounded product, summed in level order); E = 0.5 goes through the sqrt table
+on both sides, 4 ulp.
+"""
+import sys
+
+import numpy as np
+import pytest
+
+from oracle import tfce as otfce
+from tfce_mediation_amd import adjacency, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+def grid6(shape):
+    m = np.zeros([s + 2 for s in shape], bool)
+    m[1:-1, 1:-1, 1:-1] = True
+    return adjacency.voxel_csr(m, 6)
+
+
+def first_of_ico5(n):
+    """The first n vertices of an order-5 icosphere (short and empty rows among them)."""
+    return adjacency.induced_subgraph(*synth.icosphere_csr(5), np.arange(10242) < n)
+
+
+def smoothed(csr, x, passes):
+    rp, col = csr
+    deg = np.diff(rp).astype(np.int64)
+    src = np.repeat(np.arange(len(deg)), deg)
+    for _ in range(passes):
+        x = (x + np.bincount(src, weights=x[col], minlength=len(deg))) / (deg + 1)
+    return x / x.std()
+
+
+def check(csr, maps, E, signs=3):
+    import torch
+    from tfce_mediation_amd.tfce import Adjacency, SurfaceSet
+    rp, col = csr
+    V = len(rp) - 1
+    ss = SurfaceSet([Adjacency(csr, 2.0, E)], [0])
+    d = torch.from_numpy(np.ascontiguousarray(maps, dtype=np.float32)).cuda()
+    out, raw, own, st = ss.batch(d, signs, want_raw=True, want_own=True, want_status=True)
+    out, raw, own, st = (t[0].cpu().numpy() for t in (out, raw, own, st))
+    for p in range(len(maps)):
+        for k, sgn in enumerate({1: (1,), 2: (-1,), 3: (1, -1)}[signs]):
+            x = (np.float32(sgn) * maps[p]).astype(np.float32)
+            top = np.float32(np.nanmax(x)) if not np.isnan(x).all() else np.float32(-np.inf)
+            assert own[p, k] == top, (p, k, own[p, k], top)
+            if not np.isfinite(top) or top <= 0:
+                assert raw[p, k] == 0
+                continue
+            # NaN never joins a cluster; the oracle's maximum must not see it
+            y = np.where(np.isnan(x), np.float32(-1.0), x)
+            enh, levels, _ = otfce.tfce(rp, col, y, 2.0, E, exact_pow=True)
+            assert st[p, k] == levels
+            exp = np.float32(enh.max() * np.float32(top / np.float32(100)))
+            if E == 1.0:
+                assert raw[p, k] == enh.max() and out[p, k] == exp, (V, p, k, raw[p, k], enh.max())
+            else:
+                assert abs(int(np.float32(out[p, k]).view(np.int32)) - int(exp.view(np.int32))) <= 4
+    return out
+
+
+GRAPHS = {
+    "one": lambda: (np.zeros(2, np.int32), np.zeros(0, np.int32)),
+    "first_4096": lambda: first_of_ico5(4096),
+    "first_4097": lambda: first_of_ico5(4097),
+    "ico5": lambda: synth.icosphere_csr(5),
+    "ico6_cut": lambda: adjacency.induced_subgraph(*synth.icosphere_csr(6), synth.icosphere(6)[0][:, 2] < 0.8),
+    "ico5_holes": lambda: adjacency.induced_subgraph(*synth.icosphere_csr(5),
+                                                     np.random.default_rng(3).random(10242) < 0.6),
+    "grid6": lambda: grid6((17, 23, 12)),
+}
+
+
+@pytest.mark.parametrize("E", [1.0, 0.5])
+@pytest.mark.parametrize("gname", sorted(GRAPHS))
+def test_values_and_sizes(gname, E):
+    csr = GRAPHS[gname]()
+    V = len(csr[0]) - 1
+    rng = np.random.default_rng(11)
+    noise = rng.standard_normal((4, V))
+    maps = [noise[0], smoothed(csr, noise[1], 4) if V > 1 else noise[1],
+            np.round(2 * noise[2]) / 2,                  # ties everywhere
+            np.abs(noise[3]) + 0.01,                     # one sign, nothing in the other image
+            np.zeros(V), np.full(V, 1.5),                # no levels; one level value
+            np.where(rng.random(V) < 0.1, np.nan, noise[0]),
+            np.minimum(noise[1], 0.0), 1e-30 * noise[2]]
+    maps.append(np.where(np.arange(V) == V // 2, 149 * 2.0 ** -149, 0.0))  # subnormal: up to 150 levels
+    maps = np.stack(maps).astype(np.float32)
+    say(f"[gpu] basin sweep {gname} V={V} E={E}")
+    both = check(csr, maps, E)
+    one = check(csr, maps, E, signs=2)
+    np.testing.assert_array_equal(one[:, 0], both[:, 1])
+    np.testing.assert_array_equal(check(csr, maps, E, signs=1)[:, 0], both[:, 0])
+
+
+# white noise has one local maximum per seven elements: 1,500 and 5,900 basins
+# per image on icospheres, 7,500, 23,400 (16-bit parents) and, 6-connected,
+# more than the sweep holds (the element-wise sweep takes those images)
+@pytest.mark.parametrize("gname,csr", [("ico5", lambda: synth.icosphere_csr(5)), ("ico6", lambda: synth.icosphere_csr(6)),
+                                       ("grid6_52k", lambda: grid6((36, 38, 38))), ("ico7", lambda: synth.icosphere_csr(7)),
+                                       ("grid6_238k", lambda: grid6((62, 62, 62)))])
+def test_basin_counts(gname, csr):
+    csr = csr()
+    V = len(csr[0]) - 1
+    say(f"[gpu] basin sweep, white noise {gname} V={V}")
+    maps = np.random.default_rng(5).standard_normal((3, V)).astype(np.float32)
+    maps[1] = smoothed(csr, maps[1].astype(np.float64), 2)
+    check(csr, maps, 1.0)
+
+
+def test_uneven_set_and_shared_thresholds():
+    """Surfaces of several sizes in one set, a number of maps that is no
+    multiple of eight, thresholds of the largest surface for all."""
+    import torch
+    from tfce_mediation_amd.tfce import Adjacency, SurfaceSet
+    csrs = [synth.icosphere_csr(4), first_of_ico5(5001), synth.icosphere_csr(6), grid6((9, 8, 7))]
+    offsets = np.concatenate([[0], np.cumsum([len(c[0]) - 1 for c in csrs])])
+    maps = np.random.default_rng(7).standard_normal((13, int(offsets[-1]))).astype(np.float32)
+    d = torch.from_numpy(maps).cuda()
+    ss = SurfaceSet([Adjacency(c, 2.0, 1.0) for c in csrs], offsets[:-1])
+    out = ss.batch(d, 3).cpu().numpy()
+    shared, raw = (t.cpu().numpy() for t in ss.batch(d, 3, shared_thresholds=True, want_raw=True)[:2])
+    for s, (rp, col) in enumerate(csrs):
+        for p in (0, 7, 8, 12):
+            x = maps[p, offsets[s]:offsets[s + 1]]
+            enh, _, _ = otfce.tfce(rp, col, x, 2.0, 1.0, exact_pow=True)
+            assert out[s, p, 0] == np.float32(enh.max() * np.float32(x.max() / np.float32(100)))
+    rp, col = adjacency.merge_csr(csrs)
+    for p in (0, 9, 12):
+        enh, _, _ = otfce.tfce(rp, col, -maps[p], 2.0, 1.0, exact_pow=True)
+        for s in range(len(csrs)):
+            assert raw[s, p, 1] == enh[offsets[s]:offsets[s + 1]].max()

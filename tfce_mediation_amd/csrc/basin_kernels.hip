@@ -1,0 +1,853 @@
+// Basin sweep: the TFCE maxima of a batch of maps through the basins of each
+// map's local maxima.
+//
+// Order a map's active elements by (value descending, index ascending).  Adding
+// them one by one, an element with no earlier neighbour starts a component (a
+// local maximum, the root of a basin); one whose earlier neighbours are
+// mutually connected through its own neighbourhood only extends the component
+// they are in; one whose earlier neighbours fall into several arcs (a saddle)
+// joins what those arcs belong to.  An element points at its largest
+// neighbour, so following the pointers ends at the basin's maximum, and a
+// component of a superlevel set is a set of basins: the union-find of a map
+// runs over its basins and only at its saddles.  On maps smoothed five times
+// an order-7 icosphere has 2,600 maxima and about twice that in saddles for 163,842
+// vertices, so the union-find, which in the element-wise sweep is random
+// global memory for every element, fits LDS.  Components at every threshold,
+// their sizes and the float increments are those of fast_tfce.hpp:11-95.
+//
+//   basin_prepare  one workgroup per map: the maxima of +map and -map, the
+//                  threshold tables of the two images (one read of the map);
+//   basin_assign   4,096 elements per workgroup: level, pointer, local maxima
+//                  (numbered within the workgroup), saddle pairs;
+//   basin_scan     one workgroup per map: level starts, basin numbers;
+//   basin_resolve  4,096 elements per workgroup: pointers followed to the
+//                  basin, basin numbers written in level order, saddle pairs
+//                  as basin pairs in level order (pairs of one basin dropped);
+//   basin_sweep    one workgroup per image: the levels over the basins in LDS.
+// The vertex passes are streaming kernels over every workgroup slot of the GPU
+// (the element-wise sweeps hold one image per workgroup for all its levels).
+// Elements of the + and the - image are disjoint (x > T >= 0 against
+// -x > T >= 0), so one pass over a map serves both.
+#include <algorithm>
+#include <type_traits>
+
+#include "tfce_device.h"
+#include "tfce_internal.h"
+
+namespace tfcehip {
+
+namespace {
+
+constexpr int kThreads = 256;
+constexpr int kPer = kBasinBlock / kThreads;  // elements per thread of the vertex passes
+constexpr int kRound = 4;                     // elements per thread in flight
+constexpr uint16_t kInactive = 0xffff;
+
+// Basins per image of the LDS sizes: eight, four, two and one workgroup
+// (kBasinMax12) per compute unit at 12 bytes a basin, one at 6 (kBasinMax).
+// An image's levels are a chain of short steps, so images side by side on a
+// compute unit, not threads per image, fill it: 2,640-basin images took 398 us
+// a launch of 1,024 with four workgroups of 256 threads per compute unit, 493
+// with four of 512.
+constexpr int kBasinTiny = 1696, kBasinSmall = 3400, kBasinMid = 6800, kBasinMax12 = 13600;
+
+// Local unit of a workgroup of the vertex passes.  Consecutive workgroups go
+// round the eight XCDs; the workgroups of one map stay on one XCD, so its L2
+// holds the map and its pointers while they are gathered from.
+struct BlockRef {
+  int s, lp, j;
+};
+__device__ __forceinline__ BlockRef decode_block(const BasinArgs& a, int s0, int s1) {
+  const int64_t first = (int64_t)a.surfs[s0].basin.blk0;
+  int64_t b = (int64_t)blockIdx.x + first * a.pc;
+  int s = s0;
+  while (s + 1 < s1 && b >= (int64_t)a.surfs[s + 1].basin.blk0 * a.pc) ++s;
+  b -= (int64_t)a.surfs[s].basin.blk0 * a.pc;
+  const int nb = a.surfs[s].basin.nblk;
+  const int64_t whole = (int64_t)(a.pc / 8) * 8 * nb;
+  BlockRef r;
+  r.s = s;
+  if (b < whole) {
+    r.lp = (int)(b / (8 * nb)) * 8 + (int)(b & 7);
+    r.j = (int)((b % (8 * nb)) >> 3);
+  } else {
+    const int rest = a.pc & 7;
+    b -= whole;
+    r.lp = (a.pc & ~7) + (int)(b % rest);
+    r.j = (int)(b / rest);
+  }
+  return r;
+}
+
+__device__ __forceinline__ int64_t unit_of(const BasinArgs& a, int s, int lp) {
+  return (int64_t)lp * (a.n_surf - a.s_first) + (s - a.s_first);
+}
+// global item of local unit (s, lp) and sign slot g
+__device__ __forceinline__ int64_t item_of(const BasinArgs& a, int s, int lp, int g) {
+  return ((int64_t)s * a.n_maps + a.p0 + lp) * a.n_signs + g;
+}
+
+// One workgroup per map of the chunk: own maximum of each sign, threshold
+// tables (as tfce_prepare_kernel), cleared counters.
+__global__ __launch_bounds__(1024) void basin_prepare_kernel(BasinArgs a) {
+  __shared__ float s_red[2][16];
+  __shared__ int s_L[2];
+  const int n_bs = a.n_surf - a.s_first;
+  const int s = a.s_first + blockIdx.x % n_bs, lp = blockIdx.x / n_bs;
+  const SurfDev S = a.surfs[s];
+  const int V = S.V, tid = threadIdx.x;
+  const float* x = a.maps + (int64_t)(a.p0 + lp) * a.map_stride + S.offset;
+  float hi[4], lo[4];  // maxima of +x and of -x, NaN dropped by fmaxf
+#pragma unroll
+  for (int j = 0; j < 4; ++j) hi[j] = lo[j] = -INFINITY;
+  int v = tid;
+  for (; v + 3 * 1024 < V; v += 4 * 1024) {
+    float xv[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) xv[j] = x[v + j * 1024];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      hi[j] = fmaxf(hi[j], xv[j]);
+      lo[j] = fmaxf(lo[j], -xv[j]);
+    }
+  }
+  for (; v < V; v += 1024) {
+    hi[0] = fmaxf(hi[0], x[v]);
+    lo[0] = fmaxf(lo[0], -x[v]);
+  }
+  const float wh = wave_max(fmaxf(fmaxf(hi[0], hi[1]), fmaxf(hi[2], hi[3])));
+  const float wl = wave_max(fmaxf(fmaxf(lo[0], lo[1]), fmaxf(lo[2], lo[3])));
+  if ((tid & 63) == 0) {
+    s_red[0][tid >> 6] = wh;
+    s_red[1][tid >> 6] = wl;
+  }
+  int32_t* u = a.unit + unit_of(a, s, lp) * kBasinUnitWords;
+  for (int i = tid; i < kBasinUnitWords; i += 1024) u[i] = 0;
+  __syncthreads();
+  if (tid < a.n_signs) {
+    const int side = (a.n_signs == 2) ? tid : (a.sign0 < 0.0f ? 1 : 0);
+    float m = s_red[side][0];
+    for (int i = 1; i < 16; ++i) m = fmaxf(m, s_red[side][i]);
+    const int64_t item = item_of(a, s, lp, tid);
+    int32_t* rec = a.prep + item * kPrepWords;
+    float* T = reinterpret_cast<float*>(rec + kPrepT);
+    const float T0 = a.ext_T0 ? a.ext_T0[item] : ((S.flags & kSurfZeroInLevels) ? fmaxf(m, 0.0f) : m);
+    const float dT = __fdiv_rn(T0, 100.0f);
+    int L = 0, status = 0;
+    if (T0 >= 0.0f) {
+      if (!(dT > 0.0f)) {
+        status = kStatusDegenerate;
+      } else {
+        for (float t = T0; t >= 0.0f; t = __fsub_rn(t, dT)) {
+          if (L == kMaxLevels) { status = kStatusTooManyLevels; break; }
+          T[L++] = t;
+        }
+      }
+    }
+    rec[kPrepL] = status < 0 ? status : L;
+    rec[kPrepOwn] = __float_as_int(m);
+    rec[kPrepT0] = __float_as_int(T0);
+    rec[kPrepDT] = __float_as_int(dT);
+    s_L[tid] = L;
+  }
+  __syncthreads();
+  for (int g = 0; g < a.n_signs; ++g) {
+    int32_t* rec = a.prep + item_of(a, s, lp, g) * kPrepWords;
+    const float* T = reinterpret_cast<const float*>(rec + kPrepT);
+    float* HH = reinterpret_cast<float*>(rec + kPrepT + kMaxLevels);
+    for (int l = tid; l < s_L[g]; l += 1024) HH[l] = pow_h(T[l], S.H);
+  }
+}
+
+// level_of for an element known to be above the last threshold, the estimate
+// by a multiplication (the table decides, so the level is the same).
+__device__ __forceinline__ int level_of_inv(float xv, const float* s_T, int L, float T0, float inv) {
+  const float est = (T0 - xv) * inv;
+  int l = est < (float)(L - 1) ? max((int)est, 0) : L - 1;  // NaN or too large: the last level
+  while (l > 0 && xv > s_T[l - 1]) --l;
+  while (!(xv > s_T[l])) ++l;
+  return l;
+}
+
+// Arcs of the earlier neighbours of a ring-packed element: bit j of the result
+// is set for the first entry of each arc (mutually linked run of entries of
+// `up` around the ring); a closed ring that is earlier as a whole is one arc
+// (its entry 0).
+__device__ __forceinline__ unsigned ring_arcs(unsigned up, unsigned tail) {
+  const unsigned link = tail & 63u;
+  const int deg = (int)(tail >> 6);
+  // entry j continues its predecessor's arc when both are earlier and linked
+  unsigned cont = up & ((up & link & 31u) << 1);
+  if ((link & 32u) && (up & 1u) && ((up >> (deg - 1)) & 1u)) cont |= 1u;
+  const unsigned first = up & ~cont;
+  return (up && !first) ? 1u : first;
+}
+
+// Vertex pass 1 over ring-packed surfaces [s0, s1).  Bound by the gathers of
+// the six neighbours' values (L2), four elements' rows and values in flight
+// per thread.
+__global__ __launch_bounds__(kThreads) void basin_assign_ring_kernel(BasinArgs a, int s0, int s1) {
+  __shared__ float s_T[2][kBasinLevels];
+  __shared__ int s_hist[2 * kBasinLevels], s_eh[2 * kBasinLevels];
+  __shared__ int s_nmax[2], s_nev;
+  __shared__ int s_word[kBasinBlock];
+  const int tid = threadIdx.x;
+  const BlockRef br = decode_block(a, s0, s1);
+  const SurfDev S = a.surfs[br.s];
+  const int V = S.V;
+  const float* x = a.maps + (int64_t)(a.p0 + br.lp) * a.map_stride + S.offset;
+  int L[2] = {0, 0};
+  float T0[2] = {0.0f, 0.0f}, inv[2] = {1.0f, 1.0f}, last[2] = {INFINITY, INFINITY};
+  float sgn[2] = {a.n_signs == 2 ? 1.0f : a.sign0, -1.0f};
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    if (g >= a.n_signs) break;
+    const int32_t* rec = a.prep + item_of(a, br.s, br.lp, g) * kPrepWords;
+    const int l = rec[kPrepL];
+    L[g] = (l > 0 && l <= kBasinLevels) ? l : 0;
+    T0[g] = __int_as_float(rec[kPrepT0]);
+    inv[g] = 1.0f / __int_as_float(rec[kPrepDT]);
+    for (int i = tid; i < L[g]; i += kThreads) s_T[g][i] = __int_as_float(rec[kPrepT + i]);
+    if (L[g] > 0) last[g] = __int_as_float(rec[kPrepT + L[g] - 1]);
+  }
+  for (int i = tid; i < 2 * kBasinLevels; i += kThreads) s_hist[i] = s_eh[i] = 0;
+  if (tid < 2) s_nmax[tid] = 0;
+  if (tid == 2) s_nev = 0;
+  __syncthreads();
+  const int64_t e0 = (int64_t)br.lp * a.elt_total + S.basin.elt0;
+  int32_t* word = a.word + e0;
+  uint16_t* code = a.code + e0;
+  const int cap = S.basin.cand_blk;
+  uint64_t* cand = a.cand + (int64_t)br.lp * a.cand_total + S.basin.cand0 + (int64_t)br.j * cap;
+  const int4* tab = reinterpret_cast<const int4*>(S.nadj);
+  for (int r = 0; r < kPer / kRound; ++r) {
+    const int vb = br.j * kBasinBlock + r * kRound * kThreads + tid;
+    if (vb - tid >= V) break;
+    float key[kRound];
+    int g[kRound];
+    int4 row[kRound];
+    bool act[kRound];
+#pragma unroll
+    for (int t = 0; t < kRound; ++t) {
+      const int v = vb + t * kThreads;
+      key[t] = v < V ? x[v] : __int_as_float(0x7fc00000);
+    }
+#pragma unroll
+    for (int t = 0; t < kRound; ++t) {
+      g[t] = 0;
+      act[t] = sgn[0] * key[t] > last[0];
+      if (!act[t] && -key[t] > last[1]) {
+        act[t] = true;
+        g[t] = 1;
+      }
+      key[t] *= g[t] ? -1.0f : sgn[0];
+      row[t] = act[t] ? tab[vb + t * kThreads] : make_int4(-1, -1, -1, -1);
+    }
+    float nk[kRound][kRingMaxDeg];
+#pragma unroll
+    for (int t = 0; t < kRound; ++t) {
+      int u[kRingMaxDeg];
+      unsigned tail;
+      ring_fields(row[t], u, tail);
+#pragma unroll
+      for (int j = 0; j < kRingMaxDeg; ++j) nk[t][j] = u[j] != kRingNone ? x[u[j]] : __int_as_float(0x7fc00000);
+    }
+#pragma unroll
+    for (int t = 0; t < kRound; ++t) {
+      const int v = vb + t * kThreads;
+      int u[kRingMaxDeg];
+      unsigned tail;
+      ring_fields(row[t], u, tail);
+      const float s = g[t] ? -1.0f : sgn[0];
+      // the earlier neighbours, the largest of them; equal values (index
+      // order) only where the wave meets any
+      unsigned up = 0;
+      bool tie = false;
+      float bk = key[t];
+      int best = v;
+#pragma unroll
+      for (int j = 0; j < kRingMaxDeg; ++j) {
+        const float k = s * nk[t][j];
+        up |= k > key[t] ? 1u << j : 0u;
+        tie |= k == key[t];
+        best = k > bk ? u[j] : best;
+        bk = fmaxf(bk, k);
+      }
+      if (__any(tie)) {
+#pragma unroll
+        for (int j = 0; j < kRingMaxDeg; ++j)
+          if (s * nk[t][j] == key[t] && u[j] < v) {
+            up |= 1u << j;
+            if (best == v) best = u[j];
+          }
+      }
+      int lev = kNever;
+      if (act[t]) {
+        lev = g[t] * kBasinLevels + level_of_inv(key[t], s_T[g[t]], L[g[t]], T0[g[t]], g[t] ? inv[1] : inv[0]);
+        atomicAdd(&s_hist[lev], 1);
+      }
+      // local maxima numbered within the workgroup, per sign
+      int32_t w = best;
+      if (act[t] && up == 0u) w = ~atomicAdd(&s_nmax[g[t]], 1);
+      if (v < V) code[v] = act[t] ? (uint16_t)lev : kInactive;
+      s_word[(r * kRound + t) * kThreads + tid] = act[t] ? w : kNever;
+      // one pair per further arc: the first arc's first entry and its own
+      const unsigned arcs = ring_arcs(up, tail);
+      const int more = __popc(arcs) - 1;
+      if (more > 0) {
+        int at = atomicAdd(&s_nev, more);
+        atomicAdd(&s_eh[lev], more);
+        int first = -1;
+#pragma unroll
+        for (int j = 0; j < kRingMaxDeg; ++j) {
+          if (!((arcs >> j) & 1u)) continue;
+          if (first < 0) {
+            first = u[j];
+          } else {
+            if (at < cap) cand[at] = (uint64_t)lev | (uint64_t)first << 16 | (uint64_t)u[j] << 40;
+            ++at;
+          }
+        }
+      }
+    }
+  }
+  __syncthreads();
+  // pointers followed as far as they stay in the workgroup's elements: one
+  // that ends at a maximum here becomes that maximum's number
+  const int vb0 = br.j * kBasinBlock;
+  const int here = min(kBasinBlock, V - vb0);
+  for (int i = tid; i < here; i += kThreads) {
+    int w = s_word[i];
+    if (w == kNever) continue;
+    while (w >= vb0 && w < vb0 + kBasinBlock) w = s_word[w - vb0];
+    word[vb0 + i] = w;
+  }
+  int32_t* unit = a.unit + unit_of(a, br.s, br.lp) * kBasinUnitWords;
+  for (int i = tid; i < 2 * kBasinLevels; i += kThreads) {
+    if (s_hist[i]) atomicAdd(&unit[kBasinCur + i], s_hist[i]);
+    if (s_eh[i]) atomicAdd(&unit[kBasinEvCur + i], s_eh[i]);
+  }
+  if (tid < 3) {
+    int32_t* cnt = a.blk + ((int64_t)br.lp * a.blk_total + S.basin.blk0 - a.blk_first + br.j) * 4;
+    cnt[tid] = tid < 2 ? s_nmax[tid] : s_nev;
+  }
+}
+
+// Exclusive scan over the workgroup's kThreads values; total in *tot.
+__device__ __forceinline__ int block_excl_scan(int v, int* s_wave, int* tot) {
+  const int incl = wave_incl_scan(v);
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 63) s_wave[w] = incl;
+  __syncthreads();
+  int base = 0, all = 0;
+#pragma unroll
+  for (int i = 0; i < kThreads / 64; ++i) {
+    if (i < w) base += s_wave[i];
+    all += s_wave[i];
+  }
+  __syncthreads();
+  *tot = all;
+  return base + incl - v;
+}
+
+// One workgroup per map of the chunk: counts to starts.  An image that the
+// LDS sweeps do not take (too many basins, levels or saddle pairs) has its
+// basin count set to -1 and its item appended to the list of the element-wise
+// sweep.
+__global__ __launch_bounds__(kThreads) void basin_scan_kernel(BasinArgs a) {
+  __shared__ int s_wave[kThreads / 64];
+  const int n_bs = a.n_surf - a.s_first;
+  const int s = a.s_first + blockIdx.x % n_bs, lp = blockIdx.x / n_bs, tid = threadIdx.x;
+  const SurfDev S = a.surfs[s];
+  int32_t* u = a.unit + unit_of(a, s, lp) * kBasinUnitWords;
+  int32_t* blk = a.blk + ((int64_t)lp * a.blk_total + S.basin.blk0 - a.blk_first) * 4;
+  int run[2] = {0, 0};
+  int over = 0;
+  for (int b0 = 0; b0 < S.basin.nblk; b0 += kThreads) {
+    const int b = b0 + tid;
+    const int4 c = b < S.basin.nblk ? reinterpret_cast<const int4*>(blk)[b] : make_int4(0, 0, 0, 0);
+    over |= c.z > S.basin.cand_blk;
+    int t0, t1;
+    const int x0 = block_excl_scan(c.x, s_wave, &t0);
+    const int x1 = block_excl_scan(c.y, s_wave, &t1);
+    if (b < S.basin.nblk) {
+      blk[4 * b] = run[0] + x0;
+      blk[4 * b + 1] = run[1] + x1;
+    }
+    run[0] += t0;
+    run[1] += t1;
+  }
+  int start[2] = {0, 0};
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int cur = q ? kBasinEvCur : kBasinCur, st = q ? kBasinEvStart : kBasinStart;
+    int base = 0;
+    for (int i0 = 0; i0 < 2 * kBasinLevels; i0 += kThreads) {
+      const int i = i0 + tid;
+      const int c = i < 2 * kBasinLevels ? u[cur + i] : 0;
+      int tot;
+      const int x0 = block_excl_scan(c, s_wave, &tot) + base;
+      if (i < 2 * kBasinLevels) {
+        u[cur + i] = x0;
+        u[st + i] = x0;
+      }
+      base += tot;
+    }
+    if (tid == 0) u[st + 2 * kBasinLevels] = base;
+    start[q] = base;
+  }
+  over |= start[1] > S.basin.ev_cap;
+  over = __syncthreads_or(over);
+  if (tid < a.n_signs) {
+    const int64_t item = item_of(a, s, lp, tid);
+    // (beyond kBasinMax12 the values lie in the map's half of the candidates)
+    const bool bad = over || a.prep[item * kPrepWords + kPrepL] > kBasinLevels || run[tid] > a.nb_max ||
+                     (run[tid] > kBasinMax12 && run[tid] > (int64_t)S.basin.nblk * S.basin.cand_blk);
+    u[kBasinCount + tid] = bad ? -1 : run[tid];
+    if (bad) a.rest[1 + atomicAdd(&a.rest[0], 1)] = (int32_t)item;
+  }
+}
+
+// Follows N pointers to their basins' maxima: x[j] >= 0 in, the maximum's
+// element out in x[j] and its number within its workgroup in n[j].
+template <int N>
+__device__ __forceinline__ void chase(const int32_t* word, int (&x)[N], int (&n)[N]) {
+  bool go[N];
+  bool any = false;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    go[j] = x[j] >= 0;
+    n[j] = 0;
+    any |= go[j];
+  }
+  while (any) {
+    int p[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) p[j] = go[j] ? word[x[j]] : 0;
+    any = false;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if (!go[j]) continue;
+      if (p[j] < 0) {
+        n[j] = ~p[j];
+        go[j] = false;
+      } else {
+        x[j] = p[j];
+        any = true;
+      }
+    }
+  }
+}
+
+// Vertex pass 2: basins.
+constexpr int kBaseMax = 512;  // workgroups per map whose first basin numbers fit LDS (2M elements)
+
+__global__ __launch_bounds__(kThreads) void basin_resolve_kernel(BasinArgs a) {
+  __shared__ int s_cnt[2 * kBasinLevels];
+  __shared__ int s_base[2 * kBaseMax];
+  const int tid = threadIdx.x;
+  const BlockRef br = decode_block(a, a.s_first, a.n_surf);
+  const SurfDev S = a.surfs[br.s];
+  const int V = S.V;
+  int32_t* unit = a.unit + unit_of(a, br.s, br.lp) * kBasinUnitWords;
+  if (unit[kBasinCount] <= 0 && unit[kBasinCount + 1] <= 0) return;
+  const int64_t e0 = (int64_t)br.lp * a.elt_total + S.basin.elt0;
+  const int32_t* word = a.word + e0;
+  const uint16_t* code = a.code + e0;
+  uint16_t* list = a.list + e0;
+  const int32_t* blk = a.blk + ((int64_t)br.lp * a.blk_total + S.basin.blk0 - a.blk_first) * 4;
+  const int nblk = S.basin.nblk;
+  // basin number of maximum n of the workgroup of element e
+  auto basin = [&](int e, int g, int n) -> int {
+    const int b = e / kBasinBlock;
+    return (b < kBaseMax ? s_base[2 * b + g] : blk[4 * b + g]) + n;
+  };
+  for (int i = tid; i < 2 * kBasinLevels; i += kThreads) s_cnt[i] = 0;
+  for (int i = tid; i < 2 * min(nblk, kBaseMax); i += kThreads) s_base[i] = blk[4 * (i >> 1) + (i & 1)];
+  __syncthreads();
+  const int vb = br.j * kBasinBlock + tid;
+  // rank of every element among the workgroup's elements of its level
+  int cr[kPer];  // level code | rank << 16, -1: inactive
+#pragma unroll
+  for (int t = 0; t < kPer; ++t) {
+    const int v = vb + t * kThreads;
+    cr[t] = v < V ? (int)code[v] : (int)kInactive;
+  }
+#pragma unroll
+  for (int t = 0; t < kPer; ++t) cr[t] = cr[t] == kInactive ? -1 : cr[t] | atomicAdd(&s_cnt[cr[t]], 1) << 16;
+  __syncthreads();
+  for (int i = tid; i < 2 * kBasinLevels; i += kThreads)
+    if (s_cnt[i]) s_cnt[i] = atomicAdd(&unit[kBasinCur + i], s_cnt[i]);
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kPer / kRound; ++r) {
+    int e[kRound], n[kRound];
+#pragma unroll
+    for (int t = 0; t < kRound; ++t) e[t] = cr[r * kRound + t] >= 0 ? vb + (r * kRound + t) * kThreads : -1;
+    chase<kRound>(word, e, n);
+#pragma unroll
+    for (int t = 0; t < kRound; ++t) {
+      const int c = cr[r * kRound + t];
+      if (c < 0) continue;
+      const int lc = c & 0xffff;
+      list[s_cnt[lc] + (c >> 16)] = (uint16_t)basin(e[t], lc >= kBasinLevels ? 1 : 0, n[t]);
+    }
+  }
+  // the workgroup's saddle pairs, placed in level order by one reservation
+  // per level and kThreads pairs (a returning atomic on the level's cursor per
+  // pair took 5 ms of a 512-map launch whose pairs lie in few levels)
+  const int cap = S.basin.cand_blk;
+  const int nev = blk[4 * br.j + 2];
+  const uint64_t* cand = a.cand + (int64_t)br.lp * a.cand_total + S.basin.cand0 + (int64_t)br.j * cap;
+  uint32_t* ev = a.ev + (int64_t)br.lp * a.ev_total + S.basin.ev0;
+  for (int i0 = 0; i0 < nev; i0 += kThreads) {
+    __syncthreads();
+    for (int i = tid; i < 2 * kBasinLevels; i += kThreads) s_cnt[i] = 0;
+    __syncthreads();
+    int lc = -1, rank = 0, p = 0, q = 0;
+    if (i0 + tid < nev) {
+      const uint64_t w = cand[i0 + tid];
+      const int c = (int)(w & 0xffff), g = c >= kBasinLevels ? 1 : 0;
+      int e[2] = {(int)((w >> 16) & 0xffffff), (int)(w >> 40)}, n[2];
+      chase<2>(word, e, n);
+      p = basin(e[0], g, n[0]);
+      q = basin(e[1], g, n[1]);
+      if (p != q) {
+        lc = c;
+        rank = atomicAdd(&s_cnt[c], 1);
+      }
+    }
+    __syncthreads();
+    for (int i = tid; i < 2 * kBasinLevels; i += kThreads)
+      if (s_cnt[i]) s_cnt[i] = atomicAdd(&unit[kBasinEvCur + i], s_cnt[i]);
+    __syncthreads();
+    if (lc >= 0) ev[s_cnt[lc] + rank] = (uint32_t)p | (uint32_t)q << 16;
+  }
+}
+
+// Workgroup barrier for data in LDS: global loads stay in flight across it
+// (__syncthreads would wait for them).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// The basins' parents in LDS: 32 bits each, or 16 (P16) where a surface has
+// more basins than 12 bytes each leave room for.
+template <bool P16>
+struct Parents {
+  typedef typename std::conditional<P16, uint16_t, int>::type type;
+  type* p;
+  __device__ __forceinline__ int get(int c) const {
+    return (int)__hip_atomic_load(p + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __device__ __forceinline__ void set(int c, int v) {
+    __hip_atomic_store(p + c, (type)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  // Hooks root c under v; what c's parent was (c: done).
+  __device__ __forceinline__ int hook(int c, int v) {
+    if constexpr (P16) {
+      uint32_t* w = reinterpret_cast<uint32_t*>(p) + (c >> 1);
+      const int sh = 16 * (c & 1);
+      uint32_t old = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      while (true) {
+        const int now = (int)((old >> sh) & 0xffffu);
+        if (now != c) return now;
+        // fails where the word's other half changed meanwhile, too
+        if (__hip_atomic_compare_exchange_strong(w, &old, (old & ~(0xffffu << sh)) | (uint32_t)v << sh,
+                                                 __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
+          return c;
+      }
+    } else {
+      int seen = c;
+      __hip_atomic_compare_exchange_strong(p + c, &seen, v, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+      return seen;
+    }
+  }
+  // Roots of N basins (x[j] < 0: none), the chains' reads interleaved.
+  template <int N>
+  __device__ __forceinline__ void roots(int (&x)[N]) const {
+    int up[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) up[j] = x[j] >= 0 ? get(x[j]) : x[j];
+    while (true) {
+      bool more = false;
+#pragma unroll
+      for (int j = 0; j < N; ++j) more |= up[j] != x[j];
+      if (!more) return;
+      int q[N];
+#pragma unroll
+      for (int j = 0; j < N; ++j) q[j] = up[j] >= 0 ? get(up[j]) : up[j];
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        x[j] = up[j];
+        up[j] = q[j];
+      }
+    }
+  }
+};
+
+constexpr int kIlp = 4;  // basins or elements in flight per thread
+
+// Adds the wave's active lanes' elements to their roots' sizes: those of the
+// first lane's root as one addition.
+__device__ __forceinline__ void count_wave(int* size, int r) {
+  const int r0 = __builtin_amdgcn_readfirstlane(r);
+  const unsigned long long same = __ballot(r == r0);
+  const bool lead = (int)(threadIdx.x & 63) == __ffsll((long long)same) - 1;
+  if (r != r0 || lead) atomicAdd(&size[r], r != r0 ? 1 : __popcll(same));
+}
+
+// One image per workgroup (basin counts in (nb_lo, nb_hi]): parent, size and
+// value of every basin in LDS.  Two phases per level, each closed by one
+// barrier:
+//   A  the level's saddle pairs hook roots (the larger under the smaller, by
+//      CAS).  Beside it every root gains the previous level's
+//      (float)(size^E * T^H), and a basin whose parent was hooked there moves up
+//      one step;
+//   B  every hooked root hands its size and its value (the larger one stays) to
+//      its final root, and the level's elements add to their roots' sizes.
+// A root's value is the largest TFCE among its members (members gain the same
+// increments once joined, and the earliest element has the most of them), so
+// the largest value over the roots is the image's maximum, bit for bit.
+// Bound by the instructions a wave issues per level, times about 100 levels:
+// an image of the batch has its own workgroup and its levels are a chain, so
+// the number of instructions on that chain counts, not the LDS operations.
+// Hence one basin and one element per thread where that is enough (N = 1) and
+// the level tables in registers, level l in lane l % 64.
+// P16: 16-bit parents and the values in global memory (the map's dead saddle
+// candidates), for images of more basins.
+template <int T, bool P16>
+__global__ __launch_bounds__(T) void basin_sweep_kernel(BasinArgs a, int nb_lo, int nb_hi) {
+  extern __shared__ int s_dyn[];
+  __shared__ float s_red[T / 64];
+  const int n_bs = a.n_surf - a.s_first;
+  const int g = blockIdx.x % a.n_signs;
+  const int s = a.s_first + (blockIdx.x / a.n_signs) % n_bs, lp = blockIdx.x / a.n_signs / n_bs;
+  const int32_t* unit = a.unit + unit_of(a, s, lp) * kBasinUnitWords;
+  const int nb = unit[kBasinCount + g];
+  if (nb <= nb_lo || nb > nb_hi) return;
+  const SurfDev S = a.surfs[s];
+  const int64_t item = item_of(a, s, lp, g);
+  const int32_t* rec = a.prep + item * kPrepWords;
+  const int status = rec[kPrepL];
+  const int L = status > 0 ? status : 0;
+  const int tid = threadIdx.x;
+  // (nb_hi is even)
+  Parents<P16> par{reinterpret_cast<typename Parents<P16>::type*>(s_dyn)};
+  int* size = s_dyn + (P16 ? nb_hi / 2 : nb_hi);
+  float* val = reinterpret_cast<float*>(size + nb_hi);
+  if constexpr (P16)
+    val = reinterpret_cast<float*>(a.cand + (int64_t)lp * a.cand_total + S.basin.cand0) +
+          (int64_t)g * S.basin.nblk * S.basin.cand_blk;
+  auto val_get = [&](int c) -> float {
+    if constexpr (P16) return __hip_atomic_load(val + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else return val[c];
+  };
+  auto val_set = [&](int c, float v) {
+    if constexpr (P16) __hip_atomic_store(val + c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else val[c] = v;
+  };
+  auto level_barrier = [&]() {
+    if constexpr (P16) __syncthreads();
+    else lds_barrier();
+  };
+  for (int c = tid; c < nb; c += T) {
+    par.set(c, c);
+    size[c] = 0;
+    val_set(c, 0.0f);
+  }
+  __syncthreads();
+  const uint16_t* list = a.list + (int64_t)lp * a.elt_total + S.basin.elt0;
+  uint32_t* ev = a.ev + (int64_t)lp * a.ev_total + S.basin.ev0;
+  // gains of level l for basins c0 + j T; a basin that is no root, or not yet
+  // reached, has size 0
+  auto gain = [&](float HH) {
+    if (nb <= T) {
+      const int c = min(tid, nb - 1);
+      const int sz = size[c];
+      const float v = val_get(c);
+      if (sz && tid < nb) val_set(c, v + tfce_inc(sz, HH, S.E, S.sizepow));
+      return;
+    }
+    for (int c0 = tid; c0 < nb; c0 += kIlp * T) {
+      int sz[kIlp];
+      float v[kIlp];
+#pragma unroll
+      for (int j = 0; j < kIlp; ++j) {
+        const int c = min(c0 + j * T, nb - 1);
+        sz[j] = size[c];
+        if (!P16) v[j] = val_get(c);
+      }
+      if (P16) {
+#pragma unroll
+        for (int j = 0; j < kIlp; ++j) v[j] = sz[j] ? val_get(min(c0 + j * T, nb - 1)) : 0.0f;
+      }
+#pragma unroll
+      for (int j = 0; j < kIlp; ++j)
+        if (sz[j] && c0 + j * T < nb) val_set(c0 + j * T, v[j] + tfce_inc(sz[j], HH, S.E, S.sizepow));
+    }
+  };
+  // one step up for basins whose parent was hooked; a basin that is no root
+  // has its parent written by its own thread only
+  auto move_up = [&]() {
+    for (int c0 = tid; c0 < nb; c0 += 2 * T) {
+      const int c1 = min(c0 + T, nb - 1);
+      const int p0 = par.get(c0), p1 = par.get(c1);
+      const int q0 = par.get(p0), q1 = par.get(p1);
+      if (q0 != p0) par.set(c0, q0);
+      if (q1 != p1 && c0 + T < nb) par.set(c1, q1);
+    }
+  };
+  auto hand_over = [&](int c) {
+    const int sz = size[c];
+    int r[1] = {c};
+    par.roots(r);
+    if (sz) {  // 0: a basin reached at this level
+      atomicAdd(&size[r[0]], sz);
+      atomicMax(reinterpret_cast<int*>(val) + r[0], __float_as_int(val_get(c)));
+      size[c] = 0;
+    }
+  };
+  bool moved = false;  // roots were hooked at the last level
+  float HH = 0.0f;     // its T^H
+  for (int lb = 0; lb < L; lb += 64) {
+    const int Lb = min(64, L - lb);
+    const int ll = lb + min(tid & 63, Lb - 1), cl = g * kBasinLevels + ll;
+    const int t_b0 = unit[kBasinStart + cl], t_b1 = unit[kBasinStart + cl + 1];
+    const int t_e0 = unit[kBasinEvStart + cl], t_e1 = unit[kBasinEvCur + cl];
+    const int t_HH = rec[kPrepT + kMaxLevels + ll];
+    // a thread's first element and pair of a level, loaded one level ahead
+    // (indexes clamped into the level; those beyond it are not used)
+    unsigned el_n = 0, ev_n = 0;
+    auto ahead = [&](int b0, int b1, int e0, int e1) {
+      el_n = list[(unsigned)max(min(b0 + tid, b1 - 1), 0)];
+      if (e1 > e0) ev_n = ev[(unsigned)min(e0 + tid, e1 - 1)];
+    };
+    int b0 = __builtin_amdgcn_readlane(t_b0, 0), b1 = __builtin_amdgcn_readlane(t_b1, 0);
+    int e0 = __builtin_amdgcn_readlane(t_e0, 0), e1 = __builtin_amdgcn_readlane(t_e1, 0);
+    ahead(b0, b1, e0, e1);
+    for (int l = 0; l < Lb; ++l) {
+      const int el = (int)el_n;
+      const unsigned evw = ev_n;
+      const int ln = min(l + 1, Lb - 1);
+      const int nb0 = __builtin_amdgcn_readlane(t_b0, ln), nb1 = __builtin_amdgcn_readlane(t_b1, ln);
+      const int ne0 = __builtin_amdgcn_readlane(t_e0, ln), ne1 = __builtin_amdgcn_readlane(t_e1, ln);
+      ahead(nb0, nb1, ne0, ne1);
+      // A
+      int mine = -1;  // the root that this thread's first pair hooked
+      const bool pairs = e1 > e0;
+      if (pairs) {
+        for (int k = e0 + tid; k < e1; k += T) {
+          const uint32_t w = k == e0 + tid ? evw : ev[k];
+          int p = par.get((int)(w & 0xffffu)), q = par.get((int)(w >> 16));
+          int hit = -1;
+          while (p != q) {
+            const int hi = max(p, q), lo = min(p, q);
+            const int seen = par.hook(hi, lo);
+            if (seen == hi) {
+              hit = hi;
+              break;
+            }
+            p = seen;  // hi was no root: its parent (smaller) takes its place
+            q = lo;
+          }
+          // a thread's later pairs leave the root they hooked in their place
+          if (k == e0 + tid) mine = hit;
+          else ev[k] = (uint32_t)(hit + 1);
+        }
+      }
+      gain(HH);
+      if (moved) move_up();
+      moved = pairs;
+      HH = __int_as_float(__builtin_amdgcn_readlane(t_HH, l));
+      level_barrier();
+      // B
+      if (pairs) {
+        if (mine >= 0) hand_over(mine);
+        for (int k = e0 + T + tid; k < e1; k += T) {
+          const int c = (int)ev[k] - 1;
+          if (c >= 0) hand_over(c);
+        }
+      }
+      if (b0 + tid < b1) {
+        int r[1] = {el};
+        par.roots(r);
+        count_wave(size, r[0]);
+      }
+      // more than one element per thread: kIlp at a time
+      for (int k0 = b0 + T + tid; k0 < b1; k0 += kIlp * T) {
+        int r[kIlp];
+#pragma unroll
+        for (int j = 0; j < kIlp; ++j) r[j] = k0 + j * T < b1 ? (int)list[(unsigned)(k0 + j * T)] : -1;
+        par.roots(r);
+#pragma unroll
+        for (int j = 0; j < kIlp; ++j)
+          if (r[j] >= 0) count_wave(size, r[j]);
+      }
+      level_barrier();
+      b0 = nb0;
+      b1 = nb1;
+      e0 = ne0;
+      e1 = ne1;
+    }
+  }
+  if (L > 0) gain(HH);
+  __syncthreads();
+  float best = 0.0f;
+  for (int c = tid; c < nb; c += T) best = fmaxf(best, val_get(c));
+  best = wave_max(best);
+  if ((tid & 63) == 0) s_red[tid >> 6] = best;
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 0; w < T / 64; ++w) best = fmaxf(best, s_red[w]);
+    const float own = __int_as_float(rec[kPrepOwn]);
+    const float smax = (S.flags & kSurfZeroInScale) ? fmaxf(own, 0.0f) : own;
+    a.raw_max[item] = best;
+    if (a.scaled_max) a.scaled_max[item * a.out_mul + a.out_add] = __fmul_rn(best, __fdiv_rn(smax, 100.0f));
+    if (a.own_max) a.own_max[item] = own;
+    if (a.status) a.status[item] = status;
+  }
+}
+
+__global__ void basin_clear_kernel(int32_t* rest, int32_t* queue) {
+  rest[0] = 0;
+  queue[0] = queue[1] = 0;
+}
+
+// Images of at most `hi` basins and more than *lo, which becomes hi.
+template <int T, bool P16>
+hipError_t launch_sweep(const BasinArgs& a, unsigned units, int* lo, int hi, hipStream_t stream) {
+  hi = std::min(hi, (a.nb_max + 1) & ~1);
+  if (hi <= *lo) return hipSuccess;
+  const size_t lds = (size_t)hi * (P16 ? 6 : 12);
+  if (lds > 65536) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(basin_sweep_kernel<T, P16>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL((basin_sweep_kernel<T, P16>), dim3(units * a.n_signs), dim3(T), lds, stream, a, *lo, hi);
+  *lo = hi;
+  return hipSuccess;
+}
+
+}  // namespace
+
+hipError_t launch_basin_batch(const BasinArgs& a, hipStream_t stream) {
+  const int n_bs = a.n_surf - a.s_first;
+  const unsigned units = (unsigned)(n_bs * a.pc);
+  hipLaunchKernelGGL(basin_clear_kernel, dim3(1), dim3(1), 0, stream, a.rest, a.queue);
+  hipLaunchKernelGGL(basin_prepare_kernel, dim3(units), dim3(1024), 0, stream, a);
+  const unsigned blocks = (unsigned)((int64_t)a.blk_total * a.pc);
+  hipLaunchKernelGGL(basin_assign_ring_kernel, dim3(blocks), dim3(kThreads), 0, stream, a, a.s_first, a.n_surf);
+  hipLaunchKernelGGL(basin_scan_kernel, dim3(units), dim3(kThreads), 0, stream, a);
+  hipLaunchKernelGGL(basin_resolve_kernel, dim3(blocks), dim3(kThreads), 0, stream, a);
+  int lo = -1;
+  hipError_t e = launch_sweep<256, false>(a, units, &lo, kBasinTiny, stream);
+  if (e == hipSuccess) e = launch_sweep<256, false>(a, units, &lo, kBasinSmall, stream);
+  if (e == hipSuccess) e = launch_sweep<512, false>(a, units, &lo, kBasinMid, stream);
+  if (e == hipSuccess) e = launch_sweep<1024, false>(a, units, &lo, kBasinMax12, stream);
+  if (e == hipSuccess) e = launch_sweep<1024, true>(a, units, &lo, kBasinMax, stream);
+  if (e != hipSuccess) return e;
+  return hipGetLastError();
+}
+
+}  // namespace tfcehip

@@ -16,6 +16,17 @@
 
 using namespace tfcehip;
 
+// Scratch of the basin sweep per map, summed over the surfaces it takes
+// (launch positions [first, n)).
+struct BasinSpan {
+  int32_t first = 0, n = 0;
+  int32_t blk_first = 0, blk_total = 0;
+  int64_t elt_total = 0, cand_total = 0, ev_total = 0;
+  int32_t nb_max = 0;  // most basins of one image
+  bool all_ring = true;
+  bool sure = true;  // no image of these surfaces can exceed the sweep's limits
+};
+
 struct tfce_adj {
   int32_t V = 0;
   int64_t nnz = 0;
@@ -31,6 +42,10 @@ struct tfce_adj {
   int32_t ell_width = 0;
   double* d_sizepow = nullptr;  // (double)s^E for s in [0, V] when E != 1
   SurfDev* d_surf = nullptr;    // one descriptor, offset 0
+  int32_t basins_max = 0;       // most local maxima an image can have
+  int32_t pairs_max = 0;        // most saddle pairs of one element (basin sweep); 0: not taken
+  int64_t earlier_max = 0;      // most entries that can be earlier than their rows' elements
+  BasinSpan span;               // of the adjacency alone
 };
 
 struct tfce_surfset {
@@ -42,6 +57,8 @@ struct tfce_surfset {
   std::vector<int32_t> user_index;  // launch position -> caller's surface index
   bool all_ring = true;             // every surface ring-packed
   std::vector<uint8_t> lds_ok;      // per launch position: the LDS-resident sweep may take it
+  int32_t n_old = 0;                // launch positions [0, n_old): not the basin sweep's
+  BasinSpan span;                   // the others
   SurfDev* d_surfs = nullptr;
 };
 
@@ -202,6 +219,50 @@ int tfce_set_occupancy(int32_t wgs_per_cu) {
   return 0;
 }
 
+}  // extern "C"
+
+static SurfDev describe(const tfce_adj* a, int64_t offset) {
+  SurfDev sd{};
+  sd.row_ptr = a->d_row_ptr;
+  sd.col = a->d_col;
+  sd.ell = a->d_ell;
+  sd.ell_width = a->ell_width;
+  sd.nadj = a->d_nadj;
+  sd.adjw = a->d_adjw;
+  sd.adjid = a->d_adjid;
+  sd.sizepow = a->d_sizepow;
+  sd.offset = offset;
+  sd.V = a->V;
+  sd.flags = a->flags;
+  sd.H = a->H;
+  sd.E = a->E;
+  return sd;
+}
+
+// Whether the basin sweep takes a surface in MAX mode.
+static bool basin_ok(const tfce_adj* a) { return a->pairs_max > 0; }
+
+// Appends a surface to the basin sweep's scratch layout.
+static void span_add(BasinSpan& p, const tfce_adj* a, SurfDev& sd) {
+  BasinSurf& b = sd.basin;
+  b.blk0 = p.blk_first + p.blk_total;
+  b.nblk = (a->V + kBasinBlock - 1) / kBasinBlock;
+  b.elt0 = p.elt_total;
+  b.cand0 = p.cand_total;
+  b.ev0 = p.ev_total;
+  b.cand_blk = (int32_t)std::min<int64_t>((int64_t)std::min(a->V, kBasinBlock) * a->pairs_max, a->earlier_max + 1);
+  b.ev_cap = (int32_t)std::min<int64_t>(a->earlier_max + 1, (int64_t)b.nblk * b.cand_blk);
+  p.blk_total += b.nblk;
+  p.elt_total += ((int64_t)a->V + 63) & ~(int64_t)63;
+  p.cand_total += (int64_t)b.nblk * b.cand_blk;
+  p.ev_total += (b.ev_cap + 15) & ~15;
+  p.nb_max = std::max(p.nb_max, a->basins_max);
+  p.all_ring = p.all_ring && (a->flags & kSurfRing) != 0;
+  p.sure = p.sure && a->basins_max <= kBasinMax;
+}
+
+extern "C" {
+
 int tfce_adj_create_ex(const int32_t* row_ptr, const int32_t* col, int32_t V, int64_t nnz, float H,
                        float E, uint32_t flags, tfce_adj_t** out) {
   if (!out) return set_error(TFCE_EINVAL, "out is NULL");
@@ -219,6 +280,7 @@ int tfce_adj_create_ex(const int32_t* row_ptr, const int32_t* col, int32_t V, in
     return set_error(TFCE_EINVAL, "unknown adjacency flag");
   // symmetry: every (v,u) has (u,v); self loops and repeats are harmless
   bool symmetric = true;
+  int64_t listed = 0, earlier = 0;
   {
     std::vector<int64_t> fwd, bwd;
     fwd.reserve(nnz);
@@ -230,11 +292,15 @@ int tfce_adj_create_ex(const int32_t* row_ptr, const int32_t* col, int32_t V, in
         fwd.push_back((int64_t)v * V + u);
         bwd.push_back(u * V + v);
       }
+    listed = (int64_t)fwd.size();
     std::sort(fwd.begin(), fwd.end());
     fwd.erase(std::unique(fwd.begin(), fwd.end()), fwd.end());
     std::sort(bwd.begin(), bwd.end());
     bwd.erase(std::unique(bwd.begin(), bwd.end()), bwd.end());
     symmetric = (fwd == bwd);
+    // one end of every edge lists the other as earlier; with repeated entries
+    // any listing may be one
+    earlier = listed == (int64_t)fwd.size() ? listed / 2 : listed;
   }
   tfce_adj* a = new tfce_adj();
   a->V = V;
@@ -243,6 +309,7 @@ int tfce_adj_create_ex(const int32_t* row_ptr, const int32_t* col, int32_t V, in
   a->E = E;
   a->flags = (int32_t)flags | (symmetric ? kSurfSymmetric : 0);
   a->device = current_device();
+  a->earlier_max = earlier;
   auto cleanup = [&](int code, const std::string& m) {
     if (a->d_row_ptr) (void)hipFree(a->d_row_ptr);
     if (a->d_col) (void)hipFree(a->d_col);
@@ -304,6 +371,7 @@ int tfce_adj_create_ex(const int32_t* row_ptr, const int32_t* col, int32_t V, in
           // Each row is then packed into 16 bytes: six 18-bit indices, the
           // link byte from bit 108, the length from bit 114.
           std::vector<uint32_t> packed((size_t)V * 4, 0);
+          int32_t arcs_max = 1, deg_min = kRingMaxDeg;
           for (int32_t v = 0; v < V; ++v) {
             int32_t* row = ell.data() + (size_t)v * width;
             const int deg = row_ptr[v + 1] - row_ptr[v];
@@ -318,6 +386,19 @@ int tfce_adj_create_ex(const int32_t* row_ptr, const int32_t* col, int32_t V, in
             for (int j = 0; j + 1 < deg; ++j)
               if (adjacent(row[j], row[j + 1])) m |= (uint8_t)(1u << j);
             if (deg >= 3 && adjacent(row[deg - 1], row[0])) m |= (uint8_t)(1u << 5);
+            // most arcs any subset of the row falls into: every second entry
+            // of each linked run, entries linked in a closed ring floor(deg/2)
+            int arcs = 0;
+            for (int j = 0, run = 0; j < deg; ++j) {
+              ++run;
+              if (j + 1 == deg || !((m >> j) & 1u)) {
+                arcs += (run + 1) / 2;
+                run = 0;
+              }
+            }
+            if (m == (uint8_t)((1u << (deg > 0 ? deg - 1 : 0)) - 1u | 32u) && deg >= 3) arcs = deg / 2;
+            arcs_max = std::max(arcs_max, arcs);
+            deg_min = std::min(deg_min, deg);
             uint64_t f[kRingMaxDeg];
             for (int j = 0; j < kRingMaxDeg; ++j) f[j] = j < deg ? (uint64_t)row[j] : (uint64_t)kRingNone;
             const uint64_t lo = f[0] | f[1] << 18 | f[2] << 36 | f[3] << 54;
@@ -334,6 +415,12 @@ int tfce_adj_create_ex(const int32_t* row_ptr, const int32_t* col, int32_t V, in
           if ((e = hipMemcpy(a->d_nadj, packed.data(), pbytes, hipMemcpyHostToDevice)) != hipSuccess)
             return cleanup(-(int)e, "upload ring rows");
           a->flags |= kSurfRing;
+          a->pairs_max = std::max(arcs_max - 1, 1);
+          // no two local maxima are adjacent, so an element is next to at most
+          // arcs_max of them, and each is next to deg_min others at least
+          // (self loops and repeated entries: no such count)
+          const bool plain = listed == nnz && 2 * earlier == listed;
+          a->basins_max = (plain && deg_min > 0) ? (int32_t)((int64_t)V * arcs_max / (deg_min + arcs_max)) + 1 : V;
         } else {
           std::vector<uint8_t> nadj((size_t)V * width, 0);
           for (int32_t v = 0; v < V; ++v)
@@ -424,20 +511,11 @@ int tfce_adj_create_ex(const int32_t* row_ptr, const int32_t* col, int32_t V, in
     if ((e = launch_sizepow(a->d_sizepow, V, E, nullptr)) != hipSuccess || (e = hipDeviceSynchronize()) != hipSuccess)
       return cleanup(-(int)e, "sizepow table");
   }
-  SurfDev sd;
-  sd.row_ptr = a->d_row_ptr;
-  sd.col = a->d_col;
-  sd.ell = a->d_ell;
-  sd.ell_width = a->ell_width;
-  sd.nadj = a->d_nadj;
-  sd.adjw = a->d_adjw;
-  sd.adjid = a->d_adjid;
-  sd.sizepow = a->d_sizepow;
-  sd.offset = 0;
-  sd.V = V;
-  sd.flags = a->flags;
-  sd.H = H;
-  sd.E = E;
+  SurfDev sd = describe(a, 0);
+  if (basin_ok(a)) {
+    a->span.n = 1;
+    span_add(a->span, a, sd);
+  }
   if ((e = hipMemcpy(a->d_surf, &sd, sizeof(SurfDev), hipMemcpyHostToDevice)) != hipSuccess)
     return cleanup(-(int)e, "upload surface");
   *out = a;
@@ -559,17 +637,55 @@ static bool lds_eligible(const tfce_adj* a) {
   return (a->flags & kSurfSymmetric) && a->d_ell != nullptr && a->V <= kLdsMaxV && g_lds_sweep;
 }
 
+// The basin sweep's scratch for a chunk of `maps` maps: byte offsets of its
+// arrays.  The chunk is all P maps where that stays within a sixteenth of the
+// device's memory (18 GB of 288), a multiple of eight maps (one per XCD) below
+// that.  The list of leftover items comes last, so that everything before it
+// can serve as the element-wise sweep's slots, one at least.
+struct BasinLayout {
+  int32_t maps = 0;
+  size_t word = 0, code = 0, list = 0, cand = 0, ev = 0, blk = 0, unit = 0, rest = 0, bytes = 0;
+};
+
+static void basin_layout(const BasinSpan& s, int P, int n_signs, size_t slot_bytes, BasinLayout* out) {
+  auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+  const size_t per_map = (size_t)s.elt_total * 8 + (size_t)s.cand_total * 8 + (size_t)s.ev_total * 4 +
+                         (size_t)s.blk_total * 16 + (size_t)s.n * kBasinUnitWords * 4;
+  int64_t maps = (int64_t)(device_memory(current_device()) / 16 / per_map);
+  if (maps > 8) maps &= ~(int64_t)7;
+  maps = std::max<int64_t>(1, std::min<int64_t>(maps, P));
+  BasinLayout l;
+  l.maps = (int32_t)maps;
+  const size_t m = (size_t)maps;
+  l.cand = 0;
+  l.word = l.cand + up(m * s.cand_total * 8);
+  l.ev = l.word + up(m * s.elt_total * 4);
+  l.code = l.ev + up(m * s.ev_total * 4);
+  l.list = l.code + up(m * s.elt_total * 2);
+  l.blk = l.list + up(m * s.elt_total * 2);
+  l.unit = l.blk + up(m * s.blk_total * 16);
+  l.rest = l.unit + up(m * s.n * kBasinUnitWords * 4);
+  if (!s.sure) l.rest = std::max(l.rest, up(slot_bytes));
+  l.bytes = l.rest + up((1 + m * s.n * n_signs) * 4);
+  *out = l;
+}
+
 static int run_batch(const SurfDev* d_surfs, int32_t n_surf, int32_t v_max, int32_t np_w, const float* d_maps,
                      int64_t map_stride, int P, int sign_mask, const float* d_T0,
                      const float* d_vdensity, bool full, float* d_enhn, float min_t, float dh,
                      int32_t labels_level, int32_t* d_labels, float* d_scaled, float* d_raw,
                      float* d_own, int32_t* d_status, hipStream_t stream, int out_mul = 1,
                      int out_add = 0, uint32_t batch_flags = 0, const ExtScratch* ext = nullptr,
-                     bool all_ring = false, int32_t n_lds_surf = 0, bool rest_ring = false) {
+                     bool all_ring = false, int32_t n_lds_surf = 0, bool rest_ring = false,
+                     const BasinSpan* span = nullptr) {
   if (P <= 0) return 0;
   if (sign_mask < 1 || sign_mask > 3) return set_error(TFCE_EINVAL, "sign_mask must be 1, 2 or 3");
   const int n_signs = (sign_mask == 3) ? 2 : 1;
   const int64_t n_items = (int64_t)n_surf * P * n_signs;
+  // the basin sweep: MAX mode with the reference's step, on the stream's scratch
+  const bool basin = span && span->n > 0 && !full && !ext && dh == 0.0f && min_t == 0.0f;
+  const int32_t n_old_surf = basin ? span->first : n_surf;
+  const int64_t n_old = (int64_t)n_old_surf * P * n_signs;
   const int64_t slot_words = tfce_slot_words(v_max, np_w);
   const size_t slot_bytes = (size_t)slot_words * sizeof(int32_t);
   // resident workgroups, each with its own slot; the slots stay within a
@@ -577,14 +693,15 @@ static int run_batch(const SurfDev* d_surfs, int32_t n_surf, int32_t v_max, int3
   const int64_t mem_cap = (int64_t)(device_memory(current_device()) / 4 / slot_bytes);
   // the trailing n_lds_surf surfaces (the smallest) run in the LDS-resident
   // sweep, one 1,024-thread workgroup per compute unit, after the others
-  const int64_t n_lds_items = full ? 0 : (int64_t)std::min(n_lds_surf, n_surf) * P * n_signs;
-  const int64_t n_global = n_items - n_lds_items;
+  const int64_t n_lds_items = full ? 0 : (int64_t)std::min(n_lds_surf, n_old_surf) * P * n_signs;
+  const int64_t n_global = n_old - n_lds_items;
   int grid = (int)std::max<int64_t>(1, std::min<int64_t>(tfce_grid(std::max<int64_t>(n_global, 1)), mem_cap));
   const size_t prep_bytes = (size_t)n_items * kPrepWords * sizeof(int32_t);
   // raw_max is mandatory for the kernel: park it in scratch when not wanted
   const size_t raw_bytes = (size_t)n_items * sizeof(float);
   const size_t t0_bytes = (batch_flags & TFCE_BATCH_SHARED_THRESHOLDS) ? (size_t)n_items * sizeof(float) : 0;
-  char* slots = nullptr;  // grid slots
+  BasinLayout bl;
+  char* slots = nullptr;  // grid slots; then the basin sweep's scratch
   char* rest = nullptr;   // prep records, raw maxima, shared thresholds
   int32_t* queue = nullptr;
   if (ext) {
@@ -602,7 +719,11 @@ static int run_batch(const SurfDev* d_surfs, int32_t n_surf, int32_t v_max, int3
     slots = base + fixed;
   } else {
     Workspace* ws = nullptr;
-    const size_t slots_bytes = (size_t)grid * slot_bytes;
+    size_t slots_bytes = n_old > 0 ? (size_t)grid * slot_bytes : 0;
+    if (basin) {
+      basin_layout(*span, P, n_signs, slot_bytes, &bl);
+      slots_bytes = std::max(slots_bytes, bl.bytes);
+    }
     int rc = workspace_get(stream, slots_bytes + prep_bytes + raw_bytes + t0_bytes + 512, &ws);
     if (rc) return rc;
     slots = reinterpret_cast<char*>(ws->ptr);
@@ -656,13 +777,63 @@ static int run_batch(const SurfDev* d_surfs, int32_t n_surf, int32_t v_max, int3
   if (g_pair_sweep && !full && n_signs == 2 && ring_only && min_t >= 0.0f && n_global >= 2)
     pair_grid = (int)std::max<int64_t>(1, std::min<int64_t>({n_global / 2, (int64_t)grid,
                                                               2 * (int64_t)cu_count(current_device())}));
-  hipError_t e = launch_tfce_batch(a, full, ring_only, grid, n_global, stream, pair_grid);
-  if (e != hipSuccess) return set_error(-(int)e, std::string("tfce launch: ") + hipGetErrorString(e));
+  hipError_t e = hipSuccess;
+  if (n_old > 0) {
+    a.n_items = n_old;
+    e = launch_tfce_batch(a, full, ring_only, grid, n_global, stream, pair_grid);
+    if (e != hipSuccess) return set_error(-(int)e, std::string("tfce launch: ") + hipGetErrorString(e));
+  }
   if (n_lds_items > 0) {
     // one workgroup per compute unit, each taking both signs of a map at a time
     const int lgrid = (int)std::max<int64_t>(1, std::min<int64_t>(n_lds_items / n_signs, cu_count(current_device())));
     e = launch_tfce_lds(a, n_global, lgrid, stream);
     if (e != hipSuccess) return set_error(-(int)e, std::string("tfce LDS launch: ") + hipGetErrorString(e));
+  }
+  if (!basin) return 0;
+  BasinArgs b{};
+  b.surfs = d_surfs;
+  b.n_surf = n_surf;
+  b.s_first = span->first;
+  b.n_maps = P;
+  b.n_signs = n_signs;
+  b.sign0 = a.sign0;
+  b.maps = d_maps;
+  b.map_stride = map_stride;
+  b.ext_T0 = a.ext_T0;
+  b.prep = a.prep;
+  b.nb_max = std::min(kBasinMax, span->nb_max);
+  b.blk_first = span->blk_first;
+  b.blk_total = span->blk_total;
+  b.elt_total = span->elt_total;
+  b.cand_total = span->cand_total;
+  b.ev_total = span->ev_total;
+  b.word = reinterpret_cast<int32_t*>(slots + bl.word);
+  b.code = reinterpret_cast<uint16_t*>(slots + bl.code);
+  b.list = reinterpret_cast<uint16_t*>(slots + bl.list);
+  b.cand = reinterpret_cast<uint64_t*>(slots + bl.cand);
+  b.ev = reinterpret_cast<uint32_t*>(slots + bl.ev);
+  b.blk = reinterpret_cast<int32_t*>(slots + bl.blk);
+  b.unit = reinterpret_cast<int32_t*>(slots + bl.unit);
+  b.rest = reinterpret_cast<int32_t*>(slots + bl.rest);
+  b.queue = queue;
+  b.raw_max = a.raw_max;
+  b.scaled_max = a.scaled_max;
+  b.out_mul = out_mul;
+  b.out_add = out_add;
+  b.own_max = d_own;
+  b.status = d_status;
+  for (b.p0 = 0; b.p0 < P; b.p0 += bl.maps) {
+    b.pc = std::min(bl.maps, P - b.p0);
+    e = launch_basin_batch(b, stream);
+    if (e != hipSuccess) return set_error(-(int)e, std::string("tfce basin launch: ") + hipGetErrorString(e));
+    if (span->sure) continue;
+    // the images with more basins than the LDS holds: element-wise, on slots
+    // that reuse the chunk's scratch (its lists are dead by then)
+    TfceBatchArgs r = a;
+    r.rest = b.rest;
+    const int64_t most = std::min<int64_t>(tfce_grid((int64_t)span->n * b.pc * n_signs), (int64_t)(bl.rest / slot_bytes));
+    e = launch_tfce_rest(r, span->all_ring, (int)std::max<int64_t>(1, most), stream);
+    if (e != hipSuccess) return set_error(-(int)e, std::string("tfce launch: ") + hipGetErrorString(e));
   }
   return 0;
 }
@@ -684,7 +855,7 @@ int batch_max_in(tfce_adj_t* adj, const float* d_maps, int P, int sign_mask, con
   return run_batch(adj->d_surf, 1, adj->V, np_width(adj), d_maps, adj->V, P, sign_mask, nullptr, d_vdensity,
                    d_vdensity != nullptr, nullptr, 0.0f, 0.0f, -1, nullptr, d_max, nullptr, nullptr, nullptr,
                    stream, sign_mask == 3 ? 1 : 2, sign_mask == 2 ? 1 : 0, 0u, ext, (adj->flags & kSurfRing) != 0,
-                   lds_eligible(adj) ? 1 : 0);
+                   lds_eligible(adj) ? 1 : 0, false, &adj->span);
 }
 
 }  // namespace tfcehip
@@ -801,17 +972,18 @@ int tfce_batch_max(tfce_adj_t* adj, const float* d_maps, int P, int sign_mask, c
 
 }  // extern "C"
 
-// Number of trailing surfaces (smallest first from the end) the LDS-resident
-// sweep takes, and whether the others are all ring-packed.
+// Of the surfaces the basin sweep does not take: the number of trailing ones
+// (smallest first from the end) the LDS-resident sweep takes, and whether the
+// others are all ring-packed.
 static int32_t lds_tail(const tfce_surfset* s) {
   if (!g_lds_sweep) return 0;
   int32_t k = 0;
-  while (k < s->n && s->lds_ok[s->n - 1 - k]) ++k;
+  while (k < s->n_old && s->lds_ok[s->n_old - 1 - k]) ++k;
   return k;
 }
 
 static bool big_all_ring(const tfce_surfset* s) {
-  const int32_t n_big = s->n - lds_tail(s);
+  const int32_t n_big = s->n_old - lds_tail(s);
   for (int32_t k = 0; k < n_big; ++k)
     if (!(s->host[k].flags & kSurfRing)) return false;
   return true;
@@ -830,33 +1002,26 @@ int tfce_surfset_create(const tfce_adj_t* const* adjs, int32_t n, const int64_t*
     if (!adjs[i]) { delete s; return set_error(TFCE_EINVAL, "NULL adjacency in set"); }
     idx[i] = i;
   }
-  // launch order: the surfaces the LDS-resident sweep can take last (they form
-  // its item range), largest first within each group (work balance of the
-  // persistent queues)
+  // launch order: the basin sweep's surfaces last; of the others, those the
+  // LDS-resident sweep can take last (each sweep has one item range), largest
+  // first within each group (work balance of the persistent queues)
   auto small = [&](int32_t i) {
     const tfce_adj* a = adjs[i];
     return (a->flags & kSurfSymmetric) && a->d_ell != nullptr && a->V <= kLdsMaxV;
   };
   std::stable_sort(idx.begin(), idx.end(), [&](int32_t a, int32_t b) {
+    if (basin_ok(adjs[a]) != basin_ok(adjs[b])) return !basin_ok(adjs[a]);
     if (small(a) != small(b)) return !small(a);
     return adjs[a]->V > adjs[b]->V;
   });
   for (int32_t k = 0; k < n; ++k) {
     const tfce_adj* a = adjs[idx[k]];
-    SurfDev sd;
-    sd.row_ptr = a->d_row_ptr;
-    sd.col = a->d_col;
-    sd.ell = a->d_ell;
-    sd.ell_width = a->ell_width;
-    sd.nadj = a->d_nadj;
-    sd.adjw = a->d_adjw;
-    sd.adjid = a->d_adjid;
-    sd.sizepow = a->d_sizepow;
-    sd.offset = offsets[idx[k]];
-    sd.V = a->V;
-    sd.flags = a->flags;
-    sd.H = a->H;
-    sd.E = a->E;
+    SurfDev sd = describe(a, offsets[idx[k]]);
+    if (basin_ok(a)) {
+      span_add(s->span, a, sd);
+    } else {
+      s->n_old = k + 1;
+    }
     s->host.push_back(sd);
     s->user_index.push_back(idx[k]);
     s->v_max = std::max(s->v_max, a->V);
@@ -864,6 +1029,8 @@ int tfce_surfset_create(const tfce_adj_t* const* adjs, int32_t n, const int64_t*
     s->all_ring = s->all_ring && (a->flags & kSurfRing) != 0;
     s->lds_ok.push_back(small(idx[k]) ? 1 : 0);
   }
+  s->span.first = s->n_old;
+  s->span.n = n - s->n_old;
   hipError_t e = hipMalloc(&s->d_surfs, sizeof(SurfDev) * n);
   if (e == hipSuccess) e = hipMemcpy(s->d_surfs, s->host.data(), sizeof(SurfDev) * n, hipMemcpyHostToDevice);
   if (e != hipSuccess) {
@@ -890,7 +1057,7 @@ int tfce_batch_ex(const tfce_surfset_t* s, const float* d_maps, int64_t map_stri
     return set_error(TFCE_EINVAL, "unknown batch flag");
   return run_batch(s->d_surfs, s->n, s->v_max, s->np_w, d_maps, map_stride, P, sign_mask, nullptr, d_vdensity,
                    d_vdensity != nullptr, nullptr, 0.0f, 0.0f, -1, nullptr, d_scaled, d_raw, d_own, d_status,
-                   stream, 1, 0, flags, nullptr, s->all_ring, lds_tail(s), big_all_ring(s));
+                   stream, 1, 0, flags, nullptr, s->all_ring, lds_tail(s), big_all_ring(s), &s->span);
 }
 
 int tfce_surfset_order(const tfce_surfset_t* s, int32_t* user_index) {
@@ -905,7 +1072,7 @@ int tfce_batch(const tfce_surfset_t* s, const float* d_maps, int64_t map_stride,
   if (!s || !d_maps || !d_scaled) return set_error(TFCE_EINVAL, "NULL argument");
   return run_batch(s->d_surfs, s->n, s->v_max, s->np_w, d_maps, map_stride, P, sign_mask, d_T0, d_vdensity,
                    d_vdensity != nullptr, nullptr, 0.0f, 0.0f, -1, nullptr, d_scaled, d_raw, d_own, d_status,
-                   stream, 1, 0, 0u, nullptr, s->all_ring, lds_tail(s), big_all_ring(s));
+                   stream, 1, 0, 0u, nullptr, s->all_ring, lds_tail(s), big_all_ring(s), &s->span);
 }
 
 }  // extern "C"

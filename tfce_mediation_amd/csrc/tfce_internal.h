@@ -57,6 +57,32 @@ constexpr int32_t kAdjDictMaxRows = 65535;
 constexpr int32_t kLdsMaxV = 13248;
 constexpr int kLdsMaxLevels = 128;
 
+// Where a surface's part of the basin sweep's scratch lies, per map (see
+// basin_kernels.hip): its first workgroup and number of workgroups of
+// kBasinBlock elements, its first element, the first saddle pair slot of its
+// workgroups and their number per workgroup, the first slot and the number of
+// slots of its sorted pairs.
+struct BasinSurf {
+  int32_t blk0, nblk, cand_blk, ev_cap;
+  int64_t elt0, cand0, ev0;
+};
+constexpr int kBasinBlock = 4096;
+// Levels per image the basin sweep takes.  A step of fl(T0 / 100) gives at
+// most 102 levels for a normal T0 and at most 150 for a subnormal one (T0 =
+// 149 units of 2^-149, step 1).
+constexpr int kBasinLevels = 152;
+// Most basins of one image the sweep takes (6 bytes of LDS each; even).
+constexpr int kBasinMax = 27264;
+// Per-map counters (int32): level starts of the elements and of the saddle
+// pairs (level code = sign slot * kBasinLevels + level), their cursors, the
+// basin count of each sign slot (-1: left to the element-wise sweep).
+constexpr int kBasinStart = 0;
+constexpr int kBasinEvStart = kBasinStart + 2 * kBasinLevels + 1;
+constexpr int kBasinCur = kBasinEvStart + 2 * kBasinLevels + 1;
+constexpr int kBasinEvCur = kBasinCur + 2 * kBasinLevels;
+constexpr int kBasinCount = kBasinEvCur + 2 * kBasinLevels;
+constexpr int kBasinUnitWords = kBasinCount + 4;
+
 struct SurfDev {
   const int32_t* row_ptr;  // V+1
   const int32_t* col;      // nnz (indices local to the surface)
@@ -74,6 +100,7 @@ struct SurfDev {
   int32_t V;
   int32_t flags;
   float H, E;
+  BasinSurf basin;
 };
 
 struct TfceBatchArgs {
@@ -106,6 +133,7 @@ struct TfceBatchArgs {
   int32_t* queue;          // dynamic work counter, zeroed before launch
   int32_t* prep;           // [n_items][kPrepWords] per-item maximum and level tables
   int64_t n_items;
+  const int32_t* rest;     // null, or the items to sweep: rest[0] of them, from rest[1]
 };
 
 // Per-item record written by the prepare kernel (int32 words).
@@ -159,6 +187,41 @@ hipError_t launch_tfce_batch(const TfceBatchArgs& a, bool full, bool ring_only, 
 // (dh == 0): an item with more than kLdsMaxLevels levels gets NaN and
 // status kStatusTooManyLevels.
 hipError_t launch_tfce_lds(const TfceBatchArgs& a, int64_t item0, int grid, hipStream_t stream);
+// Basin sweep of a chunk of maps [p0, p0 + pc) over surfaces [s_first, n_surf).
+struct BasinArgs {
+  const SurfDev* surfs;
+  int32_t n_surf, s_first;
+  int32_t n_maps, p0, pc;
+  int32_t n_signs;
+  float sign0;
+  const float* maps;
+  int64_t map_stride;
+  const float* ext_T0;     // optional [n_items] first thresholds
+  int32_t* prep;           // [n_items][kPrepWords]
+  int32_t nb_max;          // most basins of an image taken here
+  int32_t blk_first, blk_total;  // workgroups of the vertex passes per map
+  int64_t elt_total, cand_total, ev_total;
+  // scratch of the chunk, [pc][...] each
+  int32_t* word;           // [elt_total] pointer of an element, ~number for a local maximum
+  uint16_t* code;          // [elt_total] level code, 0xffff inactive
+  uint16_t* list;          // [elt_total] basins of the elements in level order
+  uint64_t* cand;          // [cand_total] saddle pairs: level code | element << 16 | element << 40
+  uint32_t* ev;            // [ev_total] saddle pairs in level order: basin | basin << 16
+  int32_t* blk;            // [blk_total][4] local maxima of each sign, saddle pairs
+  int32_t* unit;           // [surfaces][kBasinUnitWords]
+  int32_t* rest;           // [1 + items] number and list of the items not taken
+  int32_t* queue;          // work counter of the sweep of those
+  // outputs, as TfceBatchArgs
+  float* raw_max;
+  float* scaled_max;
+  int32_t out_mul, out_add;
+  float* own_max;
+  int32_t* status;
+};
+hipError_t launch_basin_batch(const BasinArgs& a, hipStream_t stream);
+// The element-wise MAX sweep over a list of items whose records are written
+// (a.rest; the work counter already zero).
+hipError_t launch_tfce_rest(const TfceBatchArgs& a, bool ring_only, int grid, hipStream_t stream);
 hipError_t launch_sizepow(double* out, int32_t n, float E, hipStream_t stream);
 hipError_t launch_shared_T0(const TfceBatchArgs& a, float* T0, int zero_in_image, hipStream_t stream);
 hipError_t launch_fill_f32(float* p, int64_t n, float v, hipStream_t stream);

@@ -39,6 +39,7 @@
 // active prefix (FULL).  The sweep kernel carries no transcendental math (T^H
 // comes from the prepare kernel, s^E from a per-adjacency table) so it keeps
 // few registers and many waves resident: it is latency bound.
+#include "tfce_device.h"
 #include "tfce_internal.h"
 
 namespace tfcehip {
@@ -83,20 +84,6 @@ __device__ __forceinline__ int uf_link(int32_t* parent, int32_t* size, int a, in
       return b;
     }
   }
-}
-
-// (float)(s^E * HH) for one component: E == 1 is one correctly rounded float
-// product (exact in double, as fast_tfce.hpp:77 computes it); otherwise the
-// per-adjacency table holds (double)s^E.
-__device__ __forceinline__ float tfce_inc(int size, float HH, float E, const double* sizepow) {
-  if (E == 1.0f) return __fmul_rn((float)size, HH);
-  return __double2float_rn(sizepow[size] * (double)HH);
-}
-
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
 }
 
 // max over the workgroup; NaN inputs are dropped by fmaxf
@@ -230,19 +217,6 @@ __device__ __forceinline__ int4 ring_pack(const int (&q)[kRingMaxDeg], unsigned 
   const uint64_t lo = c(q[0]) | c(q[1]) << 18 | c(q[2]) << 36 | c(q[3]) << 54;
   const uint64_t hi = c(q[3]) >> 10 | c(q[4]) << 8 | c(q[5]) << 26 | (uint64_t)tail << 44;
   return make_int4((int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32));
-}
-
-__device__ __forceinline__ void ring_fields(const int4 w, int (&p)[kRingMaxDeg], unsigned& tail) {
-  const uint64_t lo = (uint64_t)(uint32_t)w.x | (uint64_t)(uint32_t)w.y << 32;
-  const uint64_t hi = (uint64_t)(uint32_t)w.z | (uint64_t)(uint32_t)w.w << 32;
-  const uint64_t M = kRingNone;
-  p[0] = (int)(lo & M);
-  p[1] = (int)((lo >> 18) & M);
-  p[2] = (int)((lo >> 36) & M);
-  p[3] = (int)(((lo >> 54) | (hi << 10)) & M);
-  p[4] = (int)((hi >> 8) & M);
-  p[5] = (int)((hi >> 26) & M);
-  tail = (unsigned)(hi >> 44) & 0x1ffu;
 }
 
 // Positions (kRingNone: inactive or no entry) and the adjacency masks among
@@ -419,30 +393,6 @@ __device__ __forceinline__ int join_roots(int32_t* parent, int32_t* size, int (&
   return tgt;
 }
 
-__device__ __forceinline__ int wave_incl_scan(int v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int t = __shfl_up(v, o, 64);
-    if (lane >= o) v += t;
-  }
-  return v;
-}
-
-// First level l with x > T[l] (T strictly decreasing, L levels), kNever if none.
-__device__ __forceinline__ int level_of(float xv, const float* s_T, int L, float T0, float dT) {
-  if (!(xv > s_T[L - 1])) return kNever;  // also NaN
-  int l = 0;
-  if (xv < T0) {
-    const float g = (T0 - xv) / dT;  // estimate; fixed up against the table below
-    l = g < (float)(L - 1) ? (int)g : L - 1;
-    if (l < 0) l = 0;
-  }
-  while (l > 0 && xv > s_T[l - 1]) --l;
-  while (!(xv > s_T[l])) ++l;
-  return l;
-}
-
 struct ItemRef {
   int s, p;
   float sign;
@@ -456,14 +406,6 @@ __device__ __forceinline__ ItemRef decode_item(const TfceBatchArgs& a, int64_t i
   r.p = rem / a.n_signs;
   r.sign = (a.n_signs == 2) ? ((rem % 2) ? -1.0f : 1.0f) : a.sign0;
   return r;
-}
-
-// fl(T^H), correctly rounded (T*T is exact in double).  The reference calls libm
-// powf, which is one ulp off for ~0.06% of inputs.
-__device__ __forceinline__ float pow_h(float T, float H) {
-  if (H == 2.0f) return __fmul_rn(T, T);
-  if (H == 1.0f) return T;
-  return __double2float_rn(pow((double)T, (double)H));
 }
 
 // One workgroup per item: maximum of sign*map over the surface (NaN ignored),
@@ -543,8 +485,9 @@ __global__ __launch_bounds__(kTfceThreads, FULL ? 3 : 4) void tfce_batch_kernel(
       s_item_hi = (int)(it >> 31);
     }
     __syncthreads();
-    const int64_t item = ((int64_t)s_item_hi << 31) | s_item_lo;
-    if (item >= a.n_items) break;  // uniform across the workgroup
+    int64_t item = ((int64_t)s_item_hi << 31) | s_item_lo;
+    if (item >= (a.rest ? (int64_t)a.rest[0] : a.n_items)) break;  // uniform across the workgroup
+    if (a.rest) item = a.rest[1 + item];
 
     const ItemRef itr = decode_item(a, item);
     const float sign = itr.sign;
@@ -2151,6 +2094,14 @@ hipError_t launch_tfce_batch(const TfceBatchArgs& a, bool full, bool ring_only, 
     hipLaunchKernelGGL((tfce_batch_kernel<false, true>), dim3(grid), dim3(kTfceThreads), 0, stream, g);
   else
     hipLaunchKernelGGL((tfce_batch_kernel<false, false>), dim3(grid), dim3(kTfceThreads), 0, stream, g);
+  return hipGetLastError();
+}
+
+hipError_t launch_tfce_rest(const TfceBatchArgs& a, bool ring_only, int grid, hipStream_t stream) {
+  if (ring_only)
+    hipLaunchKernelGGL((tfce_batch_kernel<false, true>), dim3(grid), dim3(kTfceThreads), 0, stream, a);
+  else
+    hipLaunchKernelGGL((tfce_batch_kernel<false, false>), dim3(grid), dim3(kTfceThreads), 0, stream, a);
   return hipGetLastError();
 }
 
