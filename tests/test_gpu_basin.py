@@ -35,6 +35,33 @@ def first_of_ico5(n):
     return adjacency.induced_subgraph(*synth.icosphere_csr(5), np.arange(10242) < n)
 
 
+def loop(n):
+    i = np.arange(n, dtype=np.int32)
+    nb = np.sort(np.stack([(i - 1) % n, (i + 1) % n], 1), 1).astype(np.int32)
+    return np.arange(0, 2 * n + 1, 2, dtype=np.int32), nb.ravel()
+
+
+def grid26(shape, sub=None):
+    m = np.ones(shape, bool)
+    if sub is not None:
+        m &= np.random.default_rng(sub).random(shape) < 0.6
+    return adjacency.voxel_csr(m, 26)
+
+
+def chords(n, width, seed):
+    """A loop with random chords between elements a few steps apart, lists in
+    random order: up to ``width`` neighbours, unrelated to each other."""
+    rng = np.random.default_rng(seed)
+    nb = [{(i - 1) % n, (i + 1) % n} for i in range(n)]
+    for _ in range(n * (width - 2) // 3):
+        a = int(rng.integers(n))
+        b = (a + int(rng.integers(2, 200))) % n
+        if len(nb[a]) < width and len(nb[b]) < width:
+            nb[a].add(b)
+            nb[b].add(a)
+    return adjacency.to_csr([list(rng.permutation(sorted(s))) for s in nb])
+
+
 def smoothed(csr, x, passes):
     rp, col = csr
     deg = np.diff(rp).astype(np.int64)
@@ -82,6 +109,15 @@ GRAPHS = {
     "ico5_holes": lambda: adjacency.induced_subgraph(*synth.icosphere_csr(5),
                                                      np.random.default_rng(3).random(10242) < 0.6),
     "grid6": lambda: grid6((17, 23, 12)),
+    # fixed-width tables: 4, 8, 12, 16 and 32 entries
+    "loop_4095": lambda: loop(4095),
+    "loop_4097": lambda: loop(4097),
+    "plane8": lambda: grid26((1, 70, 61)),
+    "chords12": lambda: chords(3000, 11, 1),
+    "chords16": lambda: chords(3000, 16, 2),
+    "chords32": lambda: chords(5000, 30, 3),
+    "grid26": lambda: grid26((19, 22, 13)),
+    "grid26_holes": lambda: grid26((21, 22, 17), sub=4),
 }
 
 
@@ -112,7 +148,8 @@ def test_values_and_sizes(gname, E):
 # more than the sweep holds (the element-wise sweep takes those images)
 @pytest.mark.parametrize("gname,csr", [("ico5", lambda: synth.icosphere_csr(5)), ("ico6", lambda: synth.icosphere_csr(6)),
                                        ("grid6_52k", lambda: grid6((36, 38, 38))), ("ico7", lambda: synth.icosphere_csr(7)),
-                                       ("grid6_238k", lambda: grid6((62, 62, 62)))])
+                                       ("grid6_238k", lambda: grid6((62, 62, 62))),
+                                       ("grid26_238k", lambda: grid26((62, 62, 62)))])
 def test_basin_counts(gname, csr):
     csr = csr()
     V = len(csr[0]) - 1
@@ -127,7 +164,8 @@ def test_uneven_set_and_shared_thresholds():
     multiple of eight, thresholds of the largest surface for all."""
     import torch
     from tfce_mediation_amd.tfce import Adjacency, SurfaceSet
-    csrs = [synth.icosphere_csr(4), first_of_ico5(5001), synth.icosphere_csr(6), grid6((9, 8, 7))]
+    csrs = [synth.icosphere_csr(4), first_of_ico5(5001), grid26((14, 9, 11)), synth.icosphere_csr(6), grid6((9, 8, 7)),
+            loop(300)]
     offsets = np.concatenate([[0], np.cumsum([len(c[0]) - 1 for c in csrs])])
     maps = np.random.default_rng(7).standard_normal((13, int(offsets[-1]))).astype(np.float32)
     d = torch.from_numpy(maps).cuda()

@@ -25,6 +25,7 @@ struct BasinSpan {
   int32_t nb_max = 0;  // most basins of one image
   bool all_ring = true;
   bool sure = true;  // no image of these surfaces can exceed the sweep's limits
+  std::vector<BasinGroup> groups;
 };
 
 struct tfce_adj {
@@ -239,8 +240,11 @@ static SurfDev describe(const tfce_adj* a, int64_t offset) {
   return sd;
 }
 
-// Whether the basin sweep takes a surface in MAX mode.
+// Whether the basin sweep takes a surface in MAX mode: symmetric lists in a
+// table (ring-packed or of fixed width).  Others (one-sided lists, lists of
+// more than kEllMaxWidth neighbours) stay with the element-wise sweep.
 static bool basin_ok(const tfce_adj* a) { return a->pairs_max > 0; }
+static int32_t basin_width(const tfce_adj* a) { return (a->flags & kSurfRing) ? 0 : a->ell_width; }
 
 // Appends a surface to the basin sweep's scratch layout.
 static void span_add(BasinSpan& p, const tfce_adj* a, SurfDev& sd) {
@@ -250,7 +254,12 @@ static void span_add(BasinSpan& p, const tfce_adj* a, SurfDev& sd) {
   b.elt0 = p.elt_total;
   b.cand0 = p.cand_total;
   b.ev0 = p.ev_total;
-  b.cand_blk = (int32_t)std::min<int64_t>((int64_t)std::min(a->V, kBasinBlock) * a->pairs_max, a->earlier_max + 1);
+  // an edge is the second or later arc of at most one element.  Wide rows
+  // rarely have a second arc (0.02 per voxel of smoothed 26-connected volumes,
+  // 0.1 of white noise): room for two per element, and an image with more in
+  // one workgroup's elements goes to the element-wise sweep
+  const int64_t all = std::min<int64_t>((int64_t)std::min(a->V, kBasinBlock) * a->pairs_max, a->earlier_max + 1);
+  b.cand_blk = (int32_t)((a->flags & kSurfRing) ? all : std::min<int64_t>(all, 2 * kBasinBlock));
   b.ev_cap = (int32_t)std::min<int64_t>(a->earlier_max + 1, (int64_t)b.nblk * b.cand_blk);
   p.blk_total += b.nblk;
   p.elt_total += ((int64_t)a->V + 63) & ~(int64_t)63;
@@ -258,7 +267,12 @@ static void span_add(BasinSpan& p, const tfce_adj* a, SurfDev& sd) {
   p.ev_total += (b.ev_cap + 15) & ~15;
   p.nb_max = std::max(p.nb_max, a->basins_max);
   p.all_ring = p.all_ring && (a->flags & kSurfRing) != 0;
-  p.sure = p.sure && a->basins_max <= kBasinMax;
+  p.sure = p.sure && a->basins_max <= kBasinMax && b.cand_blk == all;
+  const int32_t at = p.first + p.n++;
+  if (p.groups.empty() || p.groups.back().width != basin_width(a))
+    p.groups.push_back(BasinGroup{basin_width(a), at, at, 0});
+  p.groups.back().s1 = at + 1;
+  p.groups.back().blocks += b.nblk;
 }
 
 extern "C" {
@@ -511,11 +525,12 @@ int tfce_adj_create_ex(const int32_t* row_ptr, const int32_t* col, int32_t V, in
     if ((e = launch_sizepow(a->d_sizepow, V, E, nullptr)) != hipSuccess || (e = hipDeviceSynchronize()) != hipSuccess)
       return cleanup(-(int)e, "sizepow table");
   }
-  SurfDev sd = describe(a, 0);
-  if (basin_ok(a)) {
-    a->span.n = 1;
-    span_add(a->span, a, sd);
+  if (symmetric && a->d_ell && !(a->flags & kSurfRing)) {
+    a->pairs_max = std::max(a->ell_width - 1, 1);
+    a->basins_max = V;
   }
+  SurfDev sd = describe(a, 0);
+  if (basin_ok(a)) span_add(a->span, a, sd);
   if ((e = hipMemcpy(a->d_surf, &sd, sizeof(SurfDev), hipMemcpyHostToDevice)) != hipSuccess)
     return cleanup(-(int)e, "upload surface");
   *out = a;
@@ -824,7 +839,7 @@ static int run_batch(const SurfDev* d_surfs, int32_t n_surf, int32_t v_max, int3
   b.status = d_status;
   for (b.p0 = 0; b.p0 < P; b.p0 += bl.maps) {
     b.pc = std::min(bl.maps, P - b.p0);
-    e = launch_basin_batch(b, stream);
+    e = launch_basin_batch(b, span->groups.data(), (int)span->groups.size(), stream);
     if (e != hipSuccess) return set_error(-(int)e, std::string("tfce basin launch: ") + hipGetErrorString(e));
     if (span->sure) continue;
     // the images with more basins than the LDS holds: element-wise, on slots
@@ -1011,13 +1026,16 @@ int tfce_surfset_create(const tfce_adj_t* const* adjs, int32_t n, const int64_t*
   };
   std::stable_sort(idx.begin(), idx.end(), [&](int32_t a, int32_t b) {
     if (basin_ok(adjs[a]) != basin_ok(adjs[b])) return !basin_ok(adjs[a]);
-    if (small(a) != small(b)) return !small(a);
+    if (basin_ok(adjs[a]) && basin_width(adjs[a]) != basin_width(adjs[b]))
+      return basin_width(adjs[a]) > basin_width(adjs[b]);
+    if (!basin_ok(adjs[a]) && small(a) != small(b)) return !small(a);
     return adjs[a]->V > adjs[b]->V;
   });
   for (int32_t k = 0; k < n; ++k) {
     const tfce_adj* a = adjs[idx[k]];
     SurfDev sd = describe(a, offsets[idx[k]]);
     if (basin_ok(a)) {
+      s->span.first = s->n_old;
       span_add(s->span, a, sd);
     } else {
       s->n_old = k + 1;
@@ -1029,8 +1047,6 @@ int tfce_surfset_create(const tfce_adj_t* const* adjs, int32_t n, const int64_t*
     s->all_ring = s->all_ring && (a->flags & kSurfRing) != 0;
     s->lds_ok.push_back(small(idx[k]) ? 1 : 0);
   }
-  s->span.first = s->n_old;
-  s->span.n = n - s->n_old;
   hipError_t e = hipMalloc(&s->d_surfs, sizeof(SurfDev) * n);
   if (e == hipSuccess) e = hipMemcpy(s->d_surfs, s->host.data(), sizeof(SurfDev) * n, hipMemcpyHostToDevice);
   if (e != hipSuccess) {

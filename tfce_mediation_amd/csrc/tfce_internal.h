@@ -218,7 +218,12 @@ struct BasinArgs {
   float* own_max;
   int32_t* status;
 };
-hipError_t launch_basin_batch(const BasinArgs& a, hipStream_t stream);
+// Consecutive surfaces [s0, s1) of one table form: ring-packed (width 0) or a
+// fixed-width table; `blocks` workgroups of the vertex passes per map.
+struct BasinGroup {
+  int32_t width, s0, s1, blocks;
+};
+hipError_t launch_basin_batch(const BasinArgs& a, const BasinGroup* groups, int n_groups, hipStream_t stream);
 // The element-wise MAX sweep over a list of items whose records are written
 // (a.rest; the work counter already zero).
 hipError_t launch_tfce_rest(const TfceBatchArgs& a, bool ring_only, int grid, hipStream_t stream);
