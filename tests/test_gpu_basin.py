@@ -182,3 +182,60 @@ def test_uneven_set_and_shared_thresholds():
         enh, _, _ = otfce.tfce(rp, col, -maps[p], 2.0, 1.0, exact_pow=True)
         for s in range(len(csrs)):
             assert raw[s, p, 1] == enh[offsets[s]:offsets[s + 1]].max()
+
+
+LARGE = {"ico7_smooth": (lambda: synth.icosphere_csr(7), 4), "ico7_noise": (lambda: synth.icosphere_csr(7), 0),
+         "grid6_238k_noise": (lambda: grid6((62, 62, 62)), 0), "grid26_100k": (lambda: grid26((45, 47, 48)), 1)}
+
+
+@pytest.mark.parametrize("gname", sorted(GRAPHS) + sorted(LARGE))
+def test_images(gname):
+    """Whole images: every element's sum, added to what the caller's buffer
+    holds, in level order from it (large surfaces: the whole-GPU sweep behind
+    the basin sweep takes the image with too many basins)."""
+    import torch
+    from tfce_mediation_amd.tfce import Adjacency
+    csr, passes = LARGE[gname] if gname in LARGE else (GRAPHS[gname], 2)
+    rp, col = csr = csr()
+    V = len(rp) - 1
+    rng = np.random.default_rng(21)
+    say(f"[gpu] basin image {gname} V={V}")
+    adj = Adjacency(csr, 2.0, 1.0)
+    x = rng.standard_normal(V)
+    x = smoothed(csr, x, passes) if V > 1 else x
+    for img in (x, np.round(3 * x) / 3, np.where(rng.random(V) < 0.05, np.nan, -x), np.full(V, -1.0), np.zeros(V)):
+        img = img.astype(np.float32)
+        start = rng.random(V).astype(np.float32)
+        enh = torch.from_numpy(start.copy()).cuda()
+        st = torch.zeros(1, dtype=torch.int32, device="cuda")
+        adj.run_device(torch.from_numpy(img).cuda(), enh, accumulate=True, status=st)
+        got = enh.cpu().numpy()
+        y = np.where(np.isnan(img), np.float32(-1.0), img)
+        if not y.max() > 0:
+            np.testing.assert_array_equal(got, start)
+            continue
+        exp, levels, _ = otfce.tfce(rp, col, y, 2.0, 1.0, exact_pow=True, enhn=start.copy())
+        assert int(st.item()) == levels
+        np.testing.assert_array_equal(got.view(np.uint32), exp.view(np.uint32))
+
+
+@pytest.mark.parametrize("gname", ["one", "ico6_cut", "grid26_holes", "chords12", "loop_4097"])
+def test_weighted_maxima(gname):
+    """Rescaled maxima with element weights, some negative, both signs; images
+    with no active element keep the maximum over zeros."""
+    import torch
+    from tfce_mediation_amd.tfce import Adjacency
+    rp, col = csr = GRAPHS[gname]()
+    V = len(rp) - 1
+    rng = np.random.default_rng(31)
+    maps = np.stack([rng.standard_normal(V), np.abs(rng.standard_normal(V)), np.zeros(V)]).astype(np.float32)
+    vd = (rng.standard_normal(V) + 0.5).astype(np.float32)
+    adj = Adjacency(csr, 2.0, 1.0)
+    out = adj.batch_max(torch.from_numpy(maps).cuda(), 3, vdensity=torch.from_numpy(vd).cuda()).cpu().numpy()
+    for p in range(len(maps)):
+        for k, sgn in enumerate((1, -1)):
+            x = (np.float32(sgn) * maps[p]).astype(np.float32)
+            enh = np.zeros(V, np.float32)
+            if x.max() > 0:
+                enh, _, _ = otfce.tfce(rp, col, x, 2.0, 1.0, exact_pow=True)
+            assert out[p, k] == ((enh * np.float32(x.max() / np.float32(100))) * vd).max()

@@ -39,8 +39,15 @@ namespace tfcehip {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kPer = kBasinBlock / kThreads;  // elements per thread of the vertex passes
-constexpr int kRound = 4;                     // elements per thread in flight
+constexpr int kRound = 4;  // elements per thread in flight
+
+// The vertex passes run with 4,096 or 1,024 elements per workgroup (Q = 1 or
+// 4 workgroups per kBasinBlock): a launch of few maps with the smaller ones, so
+// that it has enough workgroups and a workgroup's chain of rounds is short;
+// a large one with the larger, whose pointers more often end in the
+// workgroup's own elements and whose per-workgroup tables cost less.
+template <int Q>
+constexpr int kBlockOf = kBasinBlock / Q;
 constexpr uint16_t kInactive = 0xffff;
 
 // Basins per image of the LDS sizes: eight, four, two and one workgroup
@@ -57,13 +64,14 @@ constexpr int kBasinTiny = 1696, kBasinSmall = 3400, kBasinMid = 6800, kBasinMax
 struct BlockRef {
   int s, lp, j;
 };
+template <int Q>
 __device__ __forceinline__ BlockRef decode_block(const BasinArgs& a, int s0, int s1) {
-  const int64_t first = (int64_t)a.surfs[s0].basin.blk0;
+  const int64_t first = (int64_t)a.surfs[s0].basin.blk0 * Q;
   int64_t b = (int64_t)blockIdx.x + first * a.pc;
   int s = s0;
-  while (s + 1 < s1 && b >= (int64_t)a.surfs[s + 1].basin.blk0 * a.pc) ++s;
-  b -= (int64_t)a.surfs[s].basin.blk0 * a.pc;
-  const int nb = a.surfs[s].basin.nblk;
+  while (s + 1 < s1 && b >= (int64_t)a.surfs[s + 1].basin.blk0 * Q * a.pc) ++s;
+  b -= (int64_t)a.surfs[s].basin.blk0 * Q * a.pc;
+  const int nb = a.surfs[s].basin.nblk * Q;
   const int64_t whole = (int64_t)(a.pc / 8) * 8 * nb;
   BlockRef r;
   r.s = s;
@@ -87,6 +95,51 @@ __device__ __forceinline__ int64_t item_of(const BasinArgs& a, int s, int lp, in
   return ((int64_t)s * a.n_maps + a.p0 + lp) * a.n_signs + g;
 }
 
+// Maxima of +x and of -x over elements [v0, v1), NaN dropped by fmaxf: this
+// thread's share, four loads in flight.
+template <int T>
+__device__ __forceinline__ void map_maxima(const float* x, int v0, int v1, float& hi, float& lo) {
+  int v = v0 + threadIdx.x;
+  for (; v + 3 * T < v1; v += 4 * T) {
+    float xv[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) xv[j] = x[v + j * T];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      hi = fmaxf(hi, xv[j]);
+      lo = fmaxf(lo, -xv[j]);
+    }
+  }
+  for (; v < v1; v += T) {
+    hi = fmaxf(hi, x[v]);
+    lo = fmaxf(lo, -x[v]);
+  }
+}
+
+// Maxima per workgroup of the vertex passes, for launches of few large maps
+// (one workgroup reads a 163,842-element map in 60 us).
+template <int Q>
+__global__ __launch_bounds__(kThreads) void basin_max_kernel(BasinArgs a) {
+  __shared__ float s_red[2][kThreads / 64];
+  const BlockRef br = decode_block<Q>(a, a.s_first, a.n_surf);
+  const SurfDev S = a.surfs[br.s];
+  const float* x = a.maps + (int64_t)(a.p0 + br.lp) * a.map_stride + S.offset;
+  float hi = -INFINITY, lo = -INFINITY;
+  map_maxima<kThreads>(x, br.j * kBlockOf<Q>, min(S.V, (br.j + 1) * kBlockOf<Q>), hi, lo);
+  hi = wave_max(hi);
+  lo = wave_max(lo);
+  if ((threadIdx.x & 63) == 0) {
+    s_red[0][threadIdx.x >> 6] = hi;
+    s_red[1][threadIdx.x >> 6] = lo;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    float m = s_red[threadIdx.x][0];
+    for (int i = 1; i < kThreads / 64; ++i) m = fmaxf(m, s_red[threadIdx.x][i]);
+    a.part[(((int64_t)br.lp * a.blk_total + S.basin.blk0 - a.blk_first) * Q + br.j) * 4 + threadIdx.x] = m;
+  }
+}
+
 // One workgroup per map of the chunk: own maximum of each sign, threshold
 // tables (as tfce_prepare_kernel), cleared counters.
 __global__ __launch_bounds__(1024) void basin_prepare_kernel(BasinArgs a) {
@@ -96,26 +149,17 @@ __global__ __launch_bounds__(1024) void basin_prepare_kernel(BasinArgs a) {
   const SurfDev S = a.surfs[s];
   const int V = S.V, tid = threadIdx.x;
   const float* x = a.maps + (int64_t)(a.p0 + lp) * a.map_stride + S.offset;
-  float hi[4], lo[4];  // maxima of +x and of -x, NaN dropped by fmaxf
-#pragma unroll
-  for (int j = 0; j < 4; ++j) hi[j] = lo[j] = -INFINITY;
-  int v = tid;
-  for (; v + 3 * 1024 < V; v += 4 * 1024) {
-    float xv[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) xv[j] = x[v + j * 1024];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      hi[j] = fmaxf(hi[j], xv[j]);
-      lo[j] = fmaxf(lo[j], -xv[j]);
+  float hi = -INFINITY, lo = -INFINITY;  // maxima of +x and of -x
+  if (a.part) {
+    const float* part = a.part + ((int64_t)lp * a.blk_total + S.basin.blk0 - a.blk_first) * a.q * 4;
+    for (int b = tid; b < S.basin.nblk * a.q; b += 1024) {
+      hi = fmaxf(hi, part[4 * b]);
+      lo = fmaxf(lo, part[4 * b + 1]);
     }
+  } else {
+    map_maxima<1024>(x, 0, V, hi, lo);
   }
-  for (; v < V; v += 1024) {
-    hi[0] = fmaxf(hi[0], x[v]);
-    lo[0] = fmaxf(lo[0], -x[v]);
-  }
-  const float wh = wave_max(fmaxf(fmaxf(hi[0], hi[1]), fmaxf(hi[2], hi[3])));
-  const float wl = wave_max(fmaxf(fmaxf(lo[0], lo[1]), fmaxf(lo[2], lo[3])));
+  const float wh = wave_max(hi), wl = wave_max(lo);
   if ((tid & 63) == 0) {
     s_red[0][tid >> 6] = wh;
     s_red[1][tid >> 6] = wl;
@@ -184,11 +228,12 @@ __device__ __forceinline__ unsigned ring_arcs(unsigned up, unsigned tail) {
 
 // What a workgroup of vertex pass 1 shares: the two images' thresholds, counts
 // per level of elements and saddle pairs, the pointers of its elements.
+template <int Q>
 struct AssignShared {
   float T[2][kBasinLevels];
   int hist[2 * kBasinLevels], pairs[2 * kBasinLevels];
   int nmax[2], npairs;
-  int word[kBasinBlock];
+  int word[kBlockOf<Q>];
 };
 
 // A workgroup's place and the images' level parameters in registers.
@@ -204,12 +249,19 @@ struct Assign {
   int cap;
 };
 
+// Counters of a workgroup: local maxima of each sign, saddle pairs.
+template <int Q>
+__device__ __forceinline__ int32_t* block_counts(const BasinArgs& a, const SurfDev& S, int lp, int j) {
+  return a.blk + (((int64_t)lp * a.blk_total + S.basin.blk0 - a.blk_first) * Q + j) * 4;
+}
+
+template <int Q>
 __device__ __forceinline__ void assign_begin(const BasinArgs& a, const SurfDev& S, const BlockRef& br, Assign& w,
-                                             AssignShared& sh) {
+                                             AssignShared<Q>& sh) {
   const int tid = threadIdx.x;
   w.br = br;
   w.V = S.V;
-  w.vb0 = br.j * kBasinBlock;
+  w.vb0 = br.j * kBlockOf<Q>;
   w.x = a.maps + (int64_t)(a.p0 + br.lp) * a.map_stride + S.offset;
   w.sgn[0] = a.n_signs == 2 ? 1.0f : a.sign0;
   w.sgn[1] = -1.0f;
@@ -234,7 +286,7 @@ __device__ __forceinline__ void assign_begin(const BasinArgs& a, const SurfDev& 
   const int64_t e0 = (int64_t)br.lp * a.elt_total + S.basin.elt0;
   w.word = a.word + e0;
   w.code = a.code + e0;
-  w.cap = S.basin.cand_blk;
+  w.cap = S.basin.cand_blk / Q;
   w.cand = a.cand + (int64_t)br.lp * a.cand_total + S.basin.cand0 + (int64_t)br.j * w.cap;
   __syncthreads();
 }
@@ -253,14 +305,16 @@ __device__ __forceinline__ bool assign_active(const Assign& w, float xv, int& g,
 }
 
 // Level code of an active element, counted.
-__device__ __forceinline__ int assign_level(const Assign& w, AssignShared& sh, int g, float key) {
+template <int Q>
+__device__ __forceinline__ int assign_level(const Assign& w, AssignShared<Q>& sh, int g, float key) {
   const int lev = g * kBasinLevels + level_of_inv(key, sh.T[g], w.L[g], g ? w.T0[1] : w.T0[0], g ? w.inv[1] : w.inv[0]);
   atomicAdd(&sh.hist[lev], 1);
   return lev;
 }
 
 // Reserves `more` slots for saddle pairs of level code lev; the first of them.
-__device__ __forceinline__ int assign_pairs(AssignShared& sh, int lev, int more) {
+template <int Q>
+__device__ __forceinline__ int assign_pairs(AssignShared<Q>& sh, int lev, int more) {
   atomicAdd(&sh.pairs[lev], more);
   return atomicAdd(&sh.npairs, more);
 }
@@ -271,14 +325,16 @@ __device__ __forceinline__ void put_pair(const Assign& w, int at, int lev, int u
 // Pointers and counts out.  Pointers are followed as far as they stay in the
 // workgroup's elements: one that ends at a maximum here becomes that maximum's
 // number.
-__device__ __forceinline__ void assign_end(const BasinArgs& a, const SurfDev& S, const Assign& w, AssignShared& sh) {
+template <int Q>
+__device__ __forceinline__ void assign_end(const BasinArgs& a, const SurfDev& S, const Assign& w,
+                                           AssignShared<Q>& sh) {
   const int tid = threadIdx.x;
   __syncthreads();
-  const int here = min(kBasinBlock, w.V - w.vb0);
+  const int here = min(kBlockOf<Q>, w.V - w.vb0);
   for (int i = tid; i < here; i += kThreads) {
     int p = sh.word[i];
     if (p == kNever) continue;
-    while (p >= w.vb0 && p < w.vb0 + kBasinBlock) p = sh.word[p - w.vb0];
+    while (p >= w.vb0 && p < w.vb0 + kBlockOf<Q>) p = sh.word[p - w.vb0];
     w.word[w.vb0 + i] = p;
   }
   int32_t* unit = a.unit + unit_of(a, w.br.s, w.br.lp) * kBasinUnitWords;
@@ -286,25 +342,23 @@ __device__ __forceinline__ void assign_end(const BasinArgs& a, const SurfDev& S,
     if (sh.hist[i]) atomicAdd(&unit[kBasinCur + i], sh.hist[i]);
     if (sh.pairs[i]) atomicAdd(&unit[kBasinEvCur + i], sh.pairs[i]);
   }
-  if (tid < 3) {
-    int32_t* cnt = a.blk + ((int64_t)w.br.lp * a.blk_total + S.basin.blk0 - a.blk_first + w.br.j) * 4;
-    cnt[tid] = tid < 2 ? sh.nmax[tid] : sh.npairs;
-  }
+  if (tid < 3) block_counts<Q>(a, S, w.br.lp, w.br.j)[tid] = tid < 2 ? sh.nmax[tid] : sh.npairs;
 }
 
 // Vertex pass 1 over ring-packed surfaces [s0, s1): four elements' rows and
 // values in flight per thread.
+template <int Q>
 __global__ __launch_bounds__(kThreads) void basin_assign_ring_kernel(BasinArgs a, int s0, int s1) {
-  __shared__ AssignShared sh;
+  __shared__ AssignShared<Q> sh;
   const int tid = threadIdx.x;
-  const BlockRef br = decode_block(a, s0, s1);
+  const BlockRef br = decode_block<Q>(a, s0, s1);
   const SurfDev S = a.surfs[br.s];
   Assign w;
   assign_begin(a, S, br, w, sh);
   const float* x = w.x;
   const int V = w.V;
   const int4* tab = reinterpret_cast<const int4*>(S.nadj);
-  for (int r = 0; r < kPer / kRound; ++r) {
+  for (int r = 0; r < kBlockOf<Q> / kThreads / kRound; ++r) {
     const int vb = w.vb0 + r * kRound * kThreads + tid;
     if (vb - tid >= V) break;
     float key[kRound];
@@ -411,17 +465,17 @@ __device__ __forceinline__ unsigned row_arcs(unsigned up, unsigned seed, unsigne
 // the same masks (the interior of a volume); narrower tables by the adjacency
 // bytes within each eight entries (a group seen as two only adds a pair that
 // basin_resolve drops).
-template <int W>
+template <int W, int Q>
 __global__ __launch_bounds__(kThreads) void basin_assign_table_kernel(BasinArgs a, int s0, int s1) {
-  __shared__ AssignShared sh;
+  __shared__ AssignShared<Q> sh;
   const int tid = threadIdx.x;
-  const BlockRef br = decode_block(a, s0, s1);
+  const BlockRef br = decode_block<Q>(a, s0, s1);
   const SurfDev S = a.surfs[br.s];
   Assign w;
   assign_begin(a, S, br, w, sh);
   const float* x = w.x;
   const int V = w.V;
-  for (int r = 0; r < kPer; ++r) {
+  for (int r = 0; r < kBlockOf<Q> / kThreads; ++r) {
     const int v = w.vb0 + r * kThreads + tid;
     if (v - tid >= V) break;
     float key = v < V ? x[v] : __int_as_float(0x7fc00000);
@@ -551,17 +605,18 @@ __global__ __launch_bounds__(kThreads) void basin_scan_kernel(BasinArgs a) {
   const int s = a.s_first + blockIdx.x / a.pc, lp = blockIdx.x % a.pc, tid = threadIdx.x;
   const SurfDev S = a.surfs[s];
   int32_t* u = a.unit + unit_of(a, s, lp) * kBasinUnitWords;
-  int32_t* blk = a.blk + ((int64_t)lp * a.blk_total + S.basin.blk0 - a.blk_first) * 4;
+  int32_t* blk = a.blk + ((int64_t)lp * a.blk_total + S.basin.blk0 - a.blk_first) * a.q * 4;
+  const int nblk = S.basin.nblk * a.q;
   int run[2] = {0, 0};
   int over = 0;
-  for (int b0 = 0; b0 < S.basin.nblk; b0 += kThreads) {
+  for (int b0 = 0; b0 < nblk; b0 += kThreads) {
     const int b = b0 + tid;
-    const int4 c = b < S.basin.nblk ? reinterpret_cast<const int4*>(blk)[b] : make_int4(0, 0, 0, 0);
-    over |= c.z > S.basin.cand_blk;
+    const int4 c = b < nblk ? reinterpret_cast<const int4*>(blk)[b] : make_int4(0, 0, 0, 0);
+    over |= c.z > S.basin.cand_blk / a.q;
     int t0, t1;
     const int x0 = block_excl_scan(c.x, s_wave, &t0);
     const int x1 = block_excl_scan(c.y, s_wave, &t1);
-    if (b < S.basin.nblk) {
+    if (b < nblk) {
       blk[4 * b] = run[0] + x0;
       blk[4 * b + 1] = run[1] + x1;
     }
@@ -592,8 +647,10 @@ __global__ __launch_bounds__(kThreads) void basin_scan_kernel(BasinArgs a) {
   if (tid < a.n_signs) {
     const int64_t item = item_of(a, s, lp, tid);
     // (beyond kBasinMax12 the values lie in the map's half of the candidates)
-    const bool bad = over || a.prep[item * kPrepWords + kPrepL] > kBasinLevels || run[tid] > a.nb_max ||
-                     (run[tid] > kBasinMax12 && run[tid] > (int64_t)S.basin.nblk * S.basin.cand_blk);
+    const int L = a.prep[item * kPrepWords + kPrepL];
+    bool bad = over || L > kBasinLevels || run[tid] > a.nb_max ||
+               (run[tid] > kBasinMax12 && run[tid] > (int64_t)S.basin.nblk * S.basin.cand_blk);
+    if (a.tab) bad = bad || (int64_t)run[tid] * ((L + 7) & ~7) > S.basin.tab_cap;
     u[kBasinCount + tid] = bad ? -1 : run[tid];
     if (bad) a.rest[1 + atomicAdd(&a.rest[0], 1)] = (int32_t)item;
   }
@@ -631,13 +688,15 @@ __device__ __forceinline__ void chase(const int32_t* word, int (&x)[N], int (&n)
 }
 
 // Vertex pass 2: basins.
-constexpr int kBaseMax = 512;  // workgroups per map whose first basin numbers fit LDS (2M elements)
+constexpr int kBaseMax = 512;  // workgroups per map whose first basin numbers fit LDS
 
+template <int Q>
 __global__ __launch_bounds__(kThreads) void basin_resolve_kernel(BasinArgs a) {
+  constexpr int kBlock = kBlockOf<Q>, kPer = kBlock / kThreads;
   __shared__ int s_cnt[2 * kBasinLevels];
   __shared__ int s_base[2 * kBaseMax];
   const int tid = threadIdx.x;
-  const BlockRef br = decode_block(a, a.s_first, a.n_surf);
+  const BlockRef br = decode_block<Q>(a, a.s_first, a.n_surf);
   const SurfDev S = a.surfs[br.s];
   const int V = S.V;
   int32_t* unit = a.unit + unit_of(a, br.s, br.lp) * kBasinUnitWords;
@@ -646,17 +705,17 @@ __global__ __launch_bounds__(kThreads) void basin_resolve_kernel(BasinArgs a) {
   const int32_t* word = a.word + e0;
   const uint16_t* code = a.code + e0;
   uint16_t* list = a.list + e0;
-  const int32_t* blk = a.blk + ((int64_t)br.lp * a.blk_total + S.basin.blk0 - a.blk_first) * 4;
-  const int nblk = S.basin.nblk;
+  const int32_t* blk = block_counts<Q>(a, S, br.lp, 0);
+  const int nblk = S.basin.nblk * Q;
   // basin number of maximum n of the workgroup of element e
   auto basin = [&](int e, int g, int n) -> int {
-    const int b = e / kBasinBlock;
+    const int b = e / kBlock;
     return (b < kBaseMax ? s_base[2 * b + g] : blk[4 * b + g]) + n;
   };
   for (int i = tid; i < 2 * kBasinLevels; i += kThreads) s_cnt[i] = 0;
   for (int i = tid; i < 2 * min(nblk, kBaseMax); i += kThreads) s_base[i] = blk[4 * (i >> 1) + (i & 1)];
   __syncthreads();
-  const int vb = br.j * kBasinBlock + tid;
+  const int vb = br.j * kBlock + tid;
   // rank of every element among the workgroup's elements of its level
   int cr[kPer];  // level code | rank << 16, -1: inactive
 #pragma unroll
@@ -681,13 +740,15 @@ __global__ __launch_bounds__(kThreads) void basin_resolve_kernel(BasinArgs a) {
       const int c = cr[r * kRound + t];
       if (c < 0) continue;
       const int lc = c & 0xffff;
-      list[s_cnt[lc] + (c >> 16)] = (uint16_t)basin(e[t], lc >= kBasinLevels ? 1 : 0, n[t]);
+      const uint16_t bn = (uint16_t)basin(e[t], lc >= kBasinLevels ? 1 : 0, n[t]);
+      list[s_cnt[lc] + (c >> 16)] = bn;
+      if (a.bas) a.bas[e0 + vb + (r * kRound + t) * kThreads] = bn;
     }
   }
   // the workgroup's saddle pairs, placed in level order by one reservation
   // per level and kThreads pairs (a returning atomic on the level's cursor per
   // pair took 5 ms of a 512-map launch whose pairs lie in few levels)
-  const int cap = S.basin.cand_blk;
+  const int cap = S.basin.cand_blk / Q;
   const int nev = blk[4 * br.j + 2];
   const uint64_t* cand = a.cand + (int64_t)br.lp * a.cand_total + S.basin.cand0 + (int64_t)br.j * cap;
   uint32_t* ev = a.ev + (int64_t)br.lp * a.ev_total + S.basin.ev0;
@@ -806,7 +867,10 @@ __device__ __forceinline__ void count_wave(int* size, int r) {
 // the level tables in registers, level l in lane l % 64.
 // P16: 16-bit parents and the values in global memory (the map's dead saddle
 // candidates), for images of more basins.
-template <int T, bool P16>
+// FULL: no values; every level's gain of every basin's component goes to the
+// image's table [level / 8][basin][level % 8], from which basin_sum_kernel sums
+// per element.
+template <int T, bool P16, bool FULL>
 __global__ __launch_bounds__(T) void basin_sweep_kernel(BasinArgs a, int nb_lo, int nb_hi) {
   extern __shared__ int s_dyn[];
   __shared__ float s_red[T / 64];
@@ -828,19 +892,22 @@ __global__ __launch_bounds__(T) void basin_sweep_kernel(BasinArgs a, int nb_lo, 
   Parents<P16> par{reinterpret_cast<typename Parents<P16>::type*>(s_dyn)};
   int* size = s_dyn + (P16 ? nb_hi / 2 : nb_hi);
   float* val = reinterpret_cast<float*>(size + nb_hi);
-  if constexpr (P16)
+  if constexpr (P16 && !FULL)
     val = reinterpret_cast<float*>(a.cand + (int64_t)lp * a.cand_total + S.basin.cand0) +
           (int64_t)g * S.basin.nblk * S.basin.cand_blk;
+  float* tab = FULL ? a.tab + ((int64_t)lp * a.n_signs + g) * a.tab_total + S.basin.tab0 : nullptr;
   auto val_get = [&](int c) -> float {
-    if constexpr (P16) return __hip_atomic_load(val + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if constexpr (FULL) return 0.0f;
+    else if constexpr (P16) return __hip_atomic_load(val + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else return val[c];
   };
   auto val_set = [&](int c, float v) {
-    if constexpr (P16) __hip_atomic_store(val + c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if constexpr (FULL) return;
+    else if constexpr (P16) __hip_atomic_store(val + c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else val[c] = v;
   };
   auto level_barrier = [&]() {
-    if constexpr (P16) __syncthreads();
+    if constexpr (P16 && !FULL) __syncthreads();
     else lds_barrier();
   };
   for (int c = tid; c < nb; c += T) {
@@ -853,7 +920,22 @@ __global__ __launch_bounds__(T) void basin_sweep_kernel(BasinArgs a, int nb_lo, 
   uint32_t* ev = a.ev + (int64_t)lp * a.ev_total + S.basin.ev0;
   // gains of level l for basins c0 + j T; a basin that is no root, or not yet
   // reached, has size 0
-  auto gain = [&](float HH) {
+  auto gain = [&](float HH, int l) {
+    if constexpr (FULL) {
+      float* out = tab + (int64_t)(l >> 3) * nb * 8 + (l & 7);
+      for (int c0 = tid; c0 < nb; c0 += kIlp * T) {
+        int r[kIlp], sz[kIlp];
+#pragma unroll
+        for (int j = 0; j < kIlp; ++j) r[j] = c0 + j * T < nb ? c0 + j * T : -1;
+        par.roots(r);
+#pragma unroll
+        for (int j = 0; j < kIlp; ++j) sz[j] = size[max(r[j], 0)];
+#pragma unroll
+        for (int j = 0; j < kIlp; ++j)
+          if (r[j] >= 0) out[(unsigned)(c0 + j * T) * 8u] = tfce_inc(sz[j], HH, S.E, S.sizepow);
+      }
+      return;
+    }
     if (nb <= T) {
       const int c = min(tid, nb - 1);
       const int sz = size[c];
@@ -896,7 +978,7 @@ __global__ __launch_bounds__(T) void basin_sweep_kernel(BasinArgs a, int nb_lo, 
     par.roots(r);
     if (sz) {  // 0: a basin reached at this level
       atomicAdd(&size[r[0]], sz);
-      atomicMax(reinterpret_cast<int*>(val) + r[0], __float_as_int(val_get(c)));
+      if constexpr (!FULL) atomicMax(reinterpret_cast<int*>(val) + r[0], __float_as_int(val_get(c)));
       size[c] = 0;
     }
   };
@@ -948,7 +1030,7 @@ __global__ __launch_bounds__(T) void basin_sweep_kernel(BasinArgs a, int nb_lo, 
           else ev[k] = (uint32_t)(hit + 1);
         }
       }
-      gain(HH);
+      if constexpr (!FULL) gain(HH, 0);
       if (moved) move_up();
       moved = pairs;
       HH = __int_as_float(__builtin_amdgcn_readlane(t_HH, l));
@@ -977,13 +1059,18 @@ __global__ __launch_bounds__(T) void basin_sweep_kernel(BasinArgs a, int nb_lo, 
           if (r[j] >= 0) count_wave(size, r[j]);
       }
       level_barrier();
+      if constexpr (FULL) {  // before the next level's unions
+        gain(HH, lb + l);
+        level_barrier();
+      }
       b0 = nb0;
       b1 = nb1;
       e0 = ne0;
       e1 = ne1;
     }
   }
-  if (L > 0) gain(HH);
+  if constexpr (FULL) return;
+  if (L > 0) gain(HH, 0);
   __syncthreads();
   float best = 0.0f;
   for (int c = tid; c < nb; c += T) best = fmaxf(best, val_get(c));
@@ -1001,57 +1088,221 @@ __global__ __launch_bounds__(T) void basin_sweep_kernel(BasinArgs a, int nb_lo, 
   }
 }
 
+// FULL mode, after the sweep: an element's TFCE is the sum of its basin's gains
+// from its own level on, in level order from the value it had (fast_tfce.hpp
+// accumulates per element in that order).  A wave walks the levels together,
+// eight at a time, four elements per thread, so that its loads fall into the few
+// lines of the basins around it and enough of them are in flight (512 images
+// of 38k elements: 152 us; 276 us with the gains as [level][basin], 318 us with
+// one element per thread).  Per workgroup: the largest sum and the largest weighted, rescaled
+// sum of each image.
+template <int Q>
+constexpr int kSumThreads = Q == 1 ? 256 : 1024;
+
+template <int Q>
+__global__ __launch_bounds__(kSumThreads<Q>) void basin_sum_kernel(BasinArgs a) {
+  constexpr int T = kSumThreads<Q>;
+  __shared__ float s_red[4][T / 64];
+  const int tid = threadIdx.x;
+  const BlockRef br = decode_block<Q>(a, a.s_first, a.n_surf);
+  const SurfDev S = a.surfs[br.s];
+  const int V = S.V;
+  const int32_t* unit = a.unit + unit_of(a, br.s, br.lp) * kBasinUnitWords;
+  const int64_t e0 = (int64_t)br.lp * a.elt_total + S.basin.elt0;
+  float* enhn = a.enhn ? a.enhn + (int64_t)(a.p0 + br.lp) * a.map_stride + S.offset : nullptr;
+  const float* vd = a.vdensity ? a.vdensity + S.offset : nullptr;
+  int L[2] = {0, 0}, nb[2] = {-1, -1};
+  float sc[2] = {0.0f, 0.0f};
+  const float* tab = a.tab + (int64_t)br.lp * a.n_signs * a.tab_total + S.basin.tab0;  // + g * tab_total
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    if (g >= a.n_signs) continue;
+    const int32_t* rec = a.prep + item_of(a, br.s, br.lp, g) * kPrepWords;
+    L[g] = max(rec[kPrepL], 0);
+    nb[g] = unit[kBasinCount + g];
+    const float own = __int_as_float(rec[kPrepOwn]);
+    sc[g] = __fdiv_rn((S.flags & kSurfZeroInScale) ? fmaxf(own, 0.0f) : own, 100.0f);
+  }
+  float best[2] = {0.0f, 0.0f}, mv[2] = {-INFINITY, -INFINITY};
+  // kEl elements per thread at once: their loads of eight levels are in flight
+  // together
+  constexpr int kEl = kBlockOf<Q> / T < 4 ? kBlockOf<Q> / T : 4;
+  for (int r = 0; r < kBlockOf<Q> / T; r += kEl) {
+    const int v0 = br.j * kBlockOf<Q> + r * T + tid;
+    if (v0 - tid >= V) break;
+    int c[kEl], g[kEl], lev[kEl], b[kEl];
+    unsigned n[kEl], nbg[kEl];
+    bool act[kEl];
+    float t[kEl];
+    int lo = kNever, hi = 0;
+#pragma unroll
+    for (int e = 0; e < kEl; ++e) {
+      const int v = v0 + e * T;
+      c[e] = v < V ? (int)a.code[e0 + v] : (int)kInactive;
+    }
+#pragma unroll
+    for (int e = 0; e < kEl; ++e) {
+      const int v = v0 + e * T;
+      g[e] = c[e] >= kBasinLevels ? 1 : 0;
+      lev[e] = c[e] - g[e] * kBasinLevels;
+      nbg[e] = (unsigned)max(g[e] ? nb[1] : nb[0], 0);
+      act[e] = c[e] != kInactive && nbg[e] > 0u;
+      n[e] = act[e] ? (unsigned)((g[e] ? L[1] : L[0]) - lev[e]) : 0u;
+      b[e] = act[e] ? (int)a.bas[e0 + v] : 0;
+      t[e] = act[e] && enhn ? enhn[v] : 0.0f;
+      if (act[e]) {
+        lo = min(lo, lev[e]);
+        hi = max(hi, lev[e] + (int)n[e]);
+      }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      lo = min(lo, __shfl_xor(lo, o, 64));
+      hi = max(hi, __shfl_xor(hi, o, 64));
+    }
+    lo = __builtin_amdgcn_readfirstlane(lo);
+    hi = __builtin_amdgcn_readfirstlane(hi);
+    for (int l = lo & ~7; l < hi; l += 8) {
+      float4 q[kEl][2];
+#pragma unroll
+      for (int e = 0; e < kEl; ++e) {
+        const float4* row = reinterpret_cast<const float4*>(tab + g[e] * a.tab_total);
+        const unsigned at = 2u * ((unsigned)(l >> 3) * nbg[e] + (unsigned)b[e]);
+        const bool mine = act[e] && l + 8 > lev[e] && l < lev[e] + (int)n[e];
+        q[e][0] = mine ? row[at] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        q[e][1] = mine ? row[at + 1] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      }
+#pragma unroll
+      for (int e = 0; e < kEl; ++e) {
+        const float w[8] = {q[e][0].x, q[e][0].y, q[e][0].z, q[e][0].w, q[e][1].x, q[e][1].y, q[e][1].z, q[e][1].w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) t[e] = (unsigned)(l + j - lev[e]) < n[e] ? t[e] + w[j] : t[e];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < kEl; ++e) {
+      const int v = v0 + e * T;
+      if (act[e] && enhn) enhn[v] = t[e];
+      if (v >= V) continue;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const float tq = (act[e] && g[e] == q) ? t[e] : 0.0f;
+        best[q] = fmaxf(best[q], tq);
+        if (vd) mv[q] = fmaxf(mv[q], __fmul_rn(__fmul_rn(tq, sc[q]), vd[v]));
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float m = wave_max(q < 2 ? best[q & 1] : mv[q & 1]);
+    if ((tid & 63) == 0) s_red[q][tid >> 6] = m;
+  }
+  __syncthreads();
+  if (tid < 4) {
+    float m = s_red[tid][0];
+    for (int i = 1; i < T / 64; ++i) m = fmaxf(m, s_red[tid][i]);
+    a.part2[(((int64_t)br.lp * a.blk_total + S.basin.blk0 - a.blk_first) * Q + br.j) * 4 + tid] = m;
+  }
+}
+
+// FULL mode: one wave per image of the chunk, over its workgroups' maxima.
+__global__ __launch_bounds__(64) void basin_final_kernel(BasinArgs a) {
+  const int s = a.s_first + blockIdx.x / (a.pc * a.n_signs);
+  const int lp = blockIdx.x / a.n_signs % a.pc, g = blockIdx.x % a.n_signs;
+  if (a.unit[unit_of(a, s, lp) * kBasinUnitWords + kBasinCount + g] < 0) return;  // the element-wise sweep's
+  const SurfDev S = a.surfs[s];
+  const float* part = a.part2 + ((int64_t)lp * a.blk_total + S.basin.blk0 - a.blk_first) * a.q * 4;
+  float best = 0.0f, mv = -INFINITY;
+  for (int b = threadIdx.x; b < S.basin.nblk * a.q; b += 64) {
+    best = fmaxf(best, part[4 * b + g]);
+    mv = fmaxf(mv, part[4 * b + 2 + g]);
+  }
+  best = wave_max(best);
+  mv = wave_max(mv);
+  if (threadIdx.x != 0) return;
+  const int64_t item = item_of(a, s, lp, g);
+  const int32_t* rec = a.prep + item * kPrepWords;
+  const float own = __int_as_float(rec[kPrepOwn]);
+  const float smax = (S.flags & kSurfZeroInScale) ? fmaxf(own, 0.0f) : own;
+  a.raw_max[item] = best;
+  if (a.scaled_max)
+    a.scaled_max[item * a.out_mul + a.out_add] = a.vdensity ? mv : __fmul_rn(best, __fdiv_rn(smax, 100.0f));
+  if (a.own_max) a.own_max[item] = own;
+  if (a.status) a.status[item] = rec[kPrepL];
+}
+
 __global__ void basin_clear_kernel(int32_t* rest, int32_t* queue) {
   rest[0] = 0;
   queue[0] = queue[1] = 0;
 }
 
 // Images of at most `hi` basins and more than *lo, which becomes hi.
-template <int T, bool P16>
+template <int T, bool P16, bool FULL>
 hipError_t launch_sweep(const BasinArgs& a, unsigned units, int* lo, int hi, hipStream_t stream) {
   hi = std::min(hi, (a.nb_max + 1) & ~1);
   if (hi <= *lo) return hipSuccess;
-  const size_t lds = (size_t)hi * (P16 ? 6 : 12);
+  const size_t lds = (size_t)hi * (P16 ? 6 : (FULL ? 8 : 12));
   if (lds > 65536) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(basin_sweep_kernel<T, P16>),
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(basin_sweep_kernel<T, P16, FULL>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((basin_sweep_kernel<T, P16>), dim3(units * a.n_signs), dim3(T), lds, stream, a, *lo, hi);
+  hipLaunchKernelGGL((basin_sweep_kernel<T, P16, FULL>), dim3(units * a.n_signs), dim3(T), lds, stream, a, *lo, hi);
   *lo = hi;
   return hipSuccess;
+}
+
+template <int W, int Q>
+void launch_assign(const BasinArgs& a, const BasinGroup& g, hipStream_t stream) {
+  const dim3 grid((unsigned)((int64_t)g.blocks * Q * a.pc));
+  if constexpr (W == 0)
+    hipLaunchKernelGGL(basin_assign_ring_kernel<Q>, grid, dim3(kThreads), 0, stream, a, g.s0, g.s1);
+  else
+    hipLaunchKernelGGL((basin_assign_table_kernel<W, Q>), grid, dim3(kThreads), 0, stream, a, g.s0, g.s1);
+}
+
+template <int Q>
+hipError_t launch_basin(const BasinArgs& a, const BasinGroup* groups, int n_groups, hipStream_t stream) {
+  const unsigned units = (unsigned)((a.n_surf - a.s_first) * a.pc);
+  const dim3 grid((unsigned)((int64_t)a.blk_total * Q * a.pc)), threads(kThreads);
+  hipLaunchKernelGGL(basin_clear_kernel, dim3(1), dim3(1), 0, stream, a.rest, a.queue);
+  if (a.part) hipLaunchKernelGGL(basin_max_kernel<Q>, grid, threads, 0, stream, a);
+  hipLaunchKernelGGL(basin_prepare_kernel, dim3(units), dim3(1024), 0, stream, a);
+  for (int i = 0; i < n_groups; ++i) {
+    switch (groups[i].width) {
+      case 0: launch_assign<0, Q>(a, groups[i], stream); break;
+      case 4: launch_assign<4, Q>(a, groups[i], stream); break;
+      case 8: launch_assign<8, Q>(a, groups[i], stream); break;
+      case 12: launch_assign<12, Q>(a, groups[i], stream); break;
+      case 16: launch_assign<16, Q>(a, groups[i], stream); break;
+      default: launch_assign<32, Q>(a, groups[i], stream); break;
+    }
+  }
+  hipLaunchKernelGGL(basin_scan_kernel, dim3(units), threads, 0, stream, a);
+  hipLaunchKernelGGL(basin_resolve_kernel<Q>, grid, threads, 0, stream, a);
+  int lo = -1;
+  hipError_t e = hipSuccess;
+  if (a.tab) {
+    e = launch_sweep<256, false, true>(a, units, &lo, kBasinTiny, stream);
+    if (e == hipSuccess) e = launch_sweep<512, false, true>(a, units, &lo, kBasinMid, stream);
+    if (e == hipSuccess) e = launch_sweep<1024, true, true>(a, units, &lo, kBasinMax, stream);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(basin_sum_kernel<Q>, grid, dim3(kSumThreads<Q>), 0, stream, a);
+    hipLaunchKernelGGL(basin_final_kernel, dim3(units * a.n_signs), dim3(64), 0, stream, a);
+    return hipGetLastError();
+  }
+  e = launch_sweep<256, false, false>(a, units, &lo, kBasinTiny, stream);
+  if (e == hipSuccess) e = launch_sweep<256, false, false>(a, units, &lo, kBasinSmall, stream);
+  if (e == hipSuccess) e = launch_sweep<512, false, false>(a, units, &lo, kBasinMid, stream);
+  if (e == hipSuccess) e = launch_sweep<1024, false, false>(a, units, &lo, kBasinMax12, stream);
+  if (e == hipSuccess) e = launch_sweep<1024, true, false>(a, units, &lo, kBasinMax, stream);
+  return e != hipSuccess ? e : hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t launch_basin_batch(const BasinArgs& a, const BasinGroup* groups, int n_groups, hipStream_t stream) {
-  const int n_bs = a.n_surf - a.s_first;
-  const unsigned units = (unsigned)(n_bs * a.pc);
-  hipLaunchKernelGGL(basin_clear_kernel, dim3(1), dim3(1), 0, stream, a.rest, a.queue);
-  hipLaunchKernelGGL(basin_prepare_kernel, dim3(units), dim3(1024), 0, stream, a);
-  const unsigned blocks = (unsigned)((int64_t)a.blk_total * a.pc);
-  for (int i = 0; i < n_groups; ++i) {
-    const BasinGroup& q = groups[i];
-    const dim3 grid((unsigned)((int64_t)q.blocks * a.pc));
-    switch (q.width) {
-      case 0: hipLaunchKernelGGL(basin_assign_ring_kernel, grid, dim3(kThreads), 0, stream, a, q.s0, q.s1); break;
-      case 4: hipLaunchKernelGGL(basin_assign_table_kernel<4>, grid, dim3(kThreads), 0, stream, a, q.s0, q.s1); break;
-      case 8: hipLaunchKernelGGL(basin_assign_table_kernel<8>, grid, dim3(kThreads), 0, stream, a, q.s0, q.s1); break;
-      case 12: hipLaunchKernelGGL(basin_assign_table_kernel<12>, grid, dim3(kThreads), 0, stream, a, q.s0, q.s1); break;
-      case 16: hipLaunchKernelGGL(basin_assign_table_kernel<16>, grid, dim3(kThreads), 0, stream, a, q.s0, q.s1); break;
-      default: hipLaunchKernelGGL(basin_assign_table_kernel<32>, grid, dim3(kThreads), 0, stream, a, q.s0, q.s1); break;
-    }
-  }
-  hipLaunchKernelGGL(basin_scan_kernel, dim3(units), dim3(kThreads), 0, stream, a);
-  hipLaunchKernelGGL(basin_resolve_kernel, dim3(blocks), dim3(kThreads), 0, stream, a);
-  int lo = -1;
-  hipError_t e = launch_sweep<256, false>(a, units, &lo, kBasinTiny, stream);
-  if (e == hipSuccess) e = launch_sweep<256, false>(a, units, &lo, kBasinSmall, stream);
-  if (e == hipSuccess) e = launch_sweep<512, false>(a, units, &lo, kBasinMid, stream);
-  if (e == hipSuccess) e = launch_sweep<1024, false>(a, units, &lo, kBasinMax12, stream);
-  if (e == hipSuccess) e = launch_sweep<1024, true>(a, units, &lo, kBasinMax, stream);
-  if (e != hipSuccess) return e;
-  return hipGetLastError();
+  return a.q == 1 ? launch_basin<1>(a, groups, n_groups, stream) : launch_basin<4>(a, groups, n_groups, stream);
 }
 
 }  // namespace tfcehip

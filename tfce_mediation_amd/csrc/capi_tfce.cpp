@@ -21,10 +21,11 @@ using namespace tfcehip;
 struct BasinSpan {
   int32_t first = 0, n = 0;
   int32_t blk_first = 0, blk_total = 0;
-  int64_t elt_total = 0, cand_total = 0, ev_total = 0;
+  int64_t elt_total = 0, cand_total = 0, ev_total = 0, tab_total = 0;
   int32_t nb_max = 0;  // most basins of one image
   bool all_ring = true;
   bool sure = true;  // no image of these surfaces can exceed the sweep's limits
+  bool sure_full = true;  // nor its table of gains
   std::vector<BasinGroup> groups;
 };
 
@@ -82,6 +83,11 @@ static bool g_pair_sweep = true;  // both signs of a map in one workgroup (ring-
 static int g_coop_mode = -1;
 static int g_coop_grid = 0;
 constexpr int32_t kCoopMinV = 32768;
+// Workgroups of the vertex passes per compute unit below which they take 1,024
+// elements instead of 4,096: 64 maps of 2,562 elements took 25 + 10 us in the
+// two passes with 64 large workgroups, 13 + 8 with 192 small ones; 512 maps of
+// 10,242 elements 65 + 29 with 1,536 large ones, 65 + 37 with 5,632 small ones.
+constexpr int64_t kBasinFill = 4;
 
 int current_device() {
   int d = 0;
@@ -258,8 +264,13 @@ static void span_add(BasinSpan& p, const tfce_adj* a, SurfDev& sd) {
   // rarely have a second arc (0.02 per voxel of smoothed 26-connected volumes,
   // 0.1 of white noise): room for two per element, and an image with more in
   // one workgroup's elements goes to the element-wise sweep
-  const int64_t all = std::min<int64_t>((int64_t)std::min(a->V, kBasinBlock) * a->pairs_max, a->earlier_max + 1);
-  b.cand_blk = (int32_t)((a->flags & kSurfRing) ? all : std::min<int64_t>(all, 2 * kBasinBlock));
+  const int64_t sub = std::min<int64_t>((int64_t)std::min(a->V, kBasinBlock / 4) * a->pairs_max, a->earlier_max + 1);
+  b.cand_blk = (int32_t)(4 * ((a->flags & kSurfRing) ? sub : std::min<int64_t>(sub, kBasinBlock / 2)));
+  const bool room = b.cand_blk == 4 * sub;
+  // gains of 16 (level, basin) pairs per element: 0.15 basins per element at
+  // 102 levels, white noise on a triangle mesh
+  b.tab0 = p.tab_total;
+  b.tab_cap = (std::max<int64_t>(16 * (int64_t)a->V, 64 * kBasinLevels) + 7) & ~(int64_t)7;
   b.ev_cap = (int32_t)std::min<int64_t>(a->earlier_max + 1, (int64_t)b.nblk * b.cand_blk);
   p.blk_total += b.nblk;
   p.elt_total += ((int64_t)a->V + 63) & ~(int64_t)63;
@@ -267,7 +278,9 @@ static void span_add(BasinSpan& p, const tfce_adj* a, SurfDev& sd) {
   p.ev_total += (b.ev_cap + 15) & ~15;
   p.nb_max = std::max(p.nb_max, a->basins_max);
   p.all_ring = p.all_ring && (a->flags & kSurfRing) != 0;
-  p.sure = p.sure && a->basins_max <= kBasinMax && b.cand_blk == all;
+  p.tab_total += b.tab_cap;
+  p.sure = p.sure && a->basins_max <= kBasinMax && room;
+  p.sure_full = p.sure_full && (int64_t)a->basins_max * kBasinLevels <= b.tab_cap;
   const int32_t at = p.first + p.n++;
   if (p.groups.empty() || p.groups.back().width != basin_width(a))
     p.groups.push_back(BasinGroup{basin_width(a), at, at, 0});
@@ -656,20 +669,30 @@ static bool lds_eligible(const tfce_adj* a) {
 // arrays.  The chunk is all P maps where that stays within a sixteenth of the
 // device's memory (18 GB of 288), a multiple of eight maps (one per XCD) below
 // that.  The list of leftover items comes last, so that everything before it
-// can serve as the element-wise sweep's slots, one at least.
+// can serve as the element-wise sweep's slots, `rest_bytes` at least.
 struct BasinLayout {
-  int32_t maps = 0;
-  size_t word = 0, code = 0, list = 0, cand = 0, ev = 0, blk = 0, unit = 0, rest = 0, bytes = 0;
+  int32_t maps = 0, q = 1;
+  bool split = false;  // maxima in a launch of their own
+  bool full = false;
+  size_t word = 0, code = 0, list = 0, cand = 0, ev = 0, blk = 0, unit = 0, part = 0, tab = 0, bas = 0, rest = 0,
+         bytes = 0;
 };
 
-static void basin_layout(const BasinSpan& s, int P, int n_signs, size_t slot_bytes, BasinLayout* out) {
+static void basin_layout(const BasinSpan& s, int P, int n_signs, bool full, size_t rest_bytes, BasinLayout* out) {
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-  const size_t per_map = (size_t)s.elt_total * 8 + (size_t)s.cand_total * 8 + (size_t)s.ev_total * 4 +
-                         (size_t)s.blk_total * 16 + (size_t)s.n * kBasinUnitWords * 4;
+  BasinLayout l;
+  l.full = full;
+  const int64_t cus = cu_count(current_device());
+  l.q = (int64_t)s.blk_total * P < kBasinFill * cus ? 4 : 1;
+  // (a map's maximum by one workgroup takes 0.4 us per 1,024 elements)
+  l.split = (int64_t)s.n * P < cus && s.blk_total > 4 * s.n;
+  const size_t nblk = (size_t)s.blk_total * l.q;
+  const size_t per_map = (size_t)s.elt_total * (full ? 10 : 8) + (size_t)s.cand_total * 8 + (size_t)s.ev_total * 4 +
+                         nblk * 32 + (size_t)s.n * kBasinUnitWords * 4 +
+                         (full ? (size_t)s.tab_total * 4 * n_signs : 0);
   int64_t maps = (int64_t)(device_memory(current_device()) / 16 / per_map);
   if (maps > 8) maps &= ~(int64_t)7;
   maps = std::max<int64_t>(1, std::min<int64_t>(maps, P));
-  BasinLayout l;
   l.maps = (int32_t)maps;
   const size_t m = (size_t)maps;
   l.cand = 0;
@@ -678,11 +701,42 @@ static void basin_layout(const BasinSpan& s, int P, int n_signs, size_t slot_byt
   l.code = l.ev + up(m * s.ev_total * 4);
   l.list = l.code + up(m * s.elt_total * 2);
   l.blk = l.list + up(m * s.elt_total * 2);
-  l.unit = l.blk + up(m * s.blk_total * 16);
-  l.rest = l.unit + up(m * s.n * kBasinUnitWords * 4);
-  if (!s.sure) l.rest = std::max(l.rest, up(slot_bytes));
+  l.part = l.blk + up(m * nblk * 16);
+  l.unit = l.part + up(m * nblk * 16);
+  l.tab = l.unit + up(m * s.n * kBasinUnitWords * 4);
+  l.bas = l.tab + (full ? up(m * n_signs * s.tab_total * 4) : 0);
+  l.rest = l.bas + (full ? up(m * s.elt_total * 2) : 0);
+  if (!s.sure || (full && !s.sure_full)) l.rest = std::max(l.rest, up(rest_bytes));
   l.bytes = l.rest + up((1 + m * s.n * n_signs) * 4);
   *out = l;
+}
+
+// Addresses of the layout at `base` in the kernel arguments.
+static void basin_place(const BasinLayout& l, char* base, BasinArgs* b) {
+  b->q = l.q;
+  b->word = reinterpret_cast<int32_t*>(base + l.word);
+  b->code = reinterpret_cast<uint16_t*>(base + l.code);
+  b->list = reinterpret_cast<uint16_t*>(base + l.list);
+  b->cand = reinterpret_cast<uint64_t*>(base + l.cand);
+  b->ev = reinterpret_cast<uint32_t*>(base + l.ev);
+  b->blk = reinterpret_cast<int32_t*>(base + l.blk);
+  b->unit = reinterpret_cast<int32_t*>(base + l.unit);
+  b->rest = reinterpret_cast<int32_t*>(base + l.rest);
+  b->part = l.split ? reinterpret_cast<float*>(base + l.part) : nullptr;
+  b->part2 = reinterpret_cast<float*>(base + l.part);  // read by the prepare kernel before it is written again
+  b->tab = l.full ? reinterpret_cast<float*>(base + l.tab) : nullptr;
+  b->bas = l.full ? reinterpret_cast<uint16_t*>(base + l.bas) : nullptr;
+}
+
+static void basin_span_args(const BasinSpan& s, BasinArgs* b) {
+  b->s_first = s.first;
+  b->nb_max = std::min(kBasinMax, s.nb_max);
+  b->blk_first = s.blk_first;
+  b->blk_total = s.blk_total;
+  b->elt_total = s.elt_total;
+  b->cand_total = s.cand_total;
+  b->ev_total = s.ev_total;
+  b->tab_total = s.tab_total;
 }
 
 static int run_batch(const SurfDev* d_surfs, int32_t n_surf, int32_t v_max, int32_t np_w, const float* d_maps,
@@ -697,8 +751,8 @@ static int run_batch(const SurfDev* d_surfs, int32_t n_surf, int32_t v_max, int3
   if (sign_mask < 1 || sign_mask > 3) return set_error(TFCE_EINVAL, "sign_mask must be 1, 2 or 3");
   const int n_signs = (sign_mask == 3) ? 2 : 1;
   const int64_t n_items = (int64_t)n_surf * P * n_signs;
-  // the basin sweep: MAX mode with the reference's step, on the stream's scratch
-  const bool basin = span && span->n > 0 && !full && !ext && dh == 0.0f && min_t == 0.0f;
+  // the basin sweep: the reference's step, on the stream's scratch
+  const bool basin = span && span->n > 0 && !ext && dh == 0.0f && min_t == 0.0f && labels_level < 0;
   const int32_t n_old_surf = basin ? span->first : n_surf;
   const int64_t n_old = (int64_t)n_old_surf * P * n_signs;
   const int64_t slot_words = tfce_slot_words(v_max, np_w);
@@ -736,7 +790,7 @@ static int run_batch(const SurfDev* d_surfs, int32_t n_surf, int32_t v_max, int3
     Workspace* ws = nullptr;
     size_t slots_bytes = n_old > 0 ? (size_t)grid * slot_bytes : 0;
     if (basin) {
-      basin_layout(*span, P, n_signs, slot_bytes, &bl);
+      basin_layout(*span, P, n_signs, full, slot_bytes, &bl);
       slots_bytes = std::max(slots_bytes, bl.bytes);
     }
     int rc = workspace_get(stream, slots_bytes + prep_bytes + raw_bytes + t0_bytes + 512, &ws);
@@ -808,7 +862,6 @@ static int run_batch(const SurfDev* d_surfs, int32_t n_surf, int32_t v_max, int3
   BasinArgs b{};
   b.surfs = d_surfs;
   b.n_surf = n_surf;
-  b.s_first = span->first;
   b.n_maps = P;
   b.n_signs = n_signs;
   b.sign0 = a.sign0;
@@ -816,23 +869,13 @@ static int run_batch(const SurfDev* d_surfs, int32_t n_surf, int32_t v_max, int3
   b.map_stride = map_stride;
   b.ext_T0 = a.ext_T0;
   b.prep = a.prep;
-  b.nb_max = std::min(kBasinMax, span->nb_max);
-  b.blk_first = span->blk_first;
-  b.blk_total = span->blk_total;
-  b.elt_total = span->elt_total;
-  b.cand_total = span->cand_total;
-  b.ev_total = span->ev_total;
-  b.word = reinterpret_cast<int32_t*>(slots + bl.word);
-  b.code = reinterpret_cast<uint16_t*>(slots + bl.code);
-  b.list = reinterpret_cast<uint16_t*>(slots + bl.list);
-  b.cand = reinterpret_cast<uint64_t*>(slots + bl.cand);
-  b.ev = reinterpret_cast<uint32_t*>(slots + bl.ev);
-  b.blk = reinterpret_cast<int32_t*>(slots + bl.blk);
-  b.unit = reinterpret_cast<int32_t*>(slots + bl.unit);
-  b.rest = reinterpret_cast<int32_t*>(slots + bl.rest);
+  basin_span_args(*span, &b);
+  basin_place(bl, slots, &b);
   b.queue = queue;
+  b.enhn = full ? d_enhn : nullptr;
+  b.vdensity = full ? d_vdensity : nullptr;
   b.raw_max = a.raw_max;
-  b.scaled_max = a.scaled_max;
+  b.scaled_max = d_scaled;
   b.out_mul = out_mul;
   b.out_add = out_add;
   b.own_max = d_own;
@@ -841,13 +884,14 @@ static int run_batch(const SurfDev* d_surfs, int32_t n_surf, int32_t v_max, int3
     b.pc = std::min(bl.maps, P - b.p0);
     e = launch_basin_batch(b, span->groups.data(), (int)span->groups.size(), stream);
     if (e != hipSuccess) return set_error(-(int)e, std::string("tfce basin launch: ") + hipGetErrorString(e));
-    if (span->sure) continue;
+    if (span->sure && (!full || span->sure_full)) continue;
     // the images with more basins than the LDS holds: element-wise, on slots
     // that reuse the chunk's scratch (its lists are dead by then)
     TfceBatchArgs r = a;
+    r.n_items = n_items;
     r.rest = b.rest;
     const int64_t most = std::min<int64_t>(tfce_grid((int64_t)span->n * b.pc * n_signs), (int64_t)(bl.rest / slot_bytes));
-    e = launch_tfce_rest(r, span->all_ring, (int)std::max<int64_t>(1, most), stream);
+    e = launch_tfce_rest(r, full, span->all_ring, (int)std::max<int64_t>(1, most), stream);
     if (e != hipSuccess) return set_error(-(int)e, std::string("tfce launch: ") + hipGetErrorString(e));
   }
   return 0;
@@ -893,7 +937,9 @@ static bool coop_supported() {
   return ok;
 }
 
-// One image over the whole GPU: its record, then the cooperative level sweep.
+// One image over the whole GPU: the basin sweep where the surface takes it,
+// with the cooperative level sweep behind it for an image of too many basins;
+// the cooperative sweep alone for the others.
 static int run_coop(tfce_adj_t* adj, const float* d_image, float* d_enhn, float min_t, float dh,
                     int32_t* d_status, hipStream_t stream) {
   const int64_t V = adj->V;
@@ -901,12 +947,43 @@ static int run_coop(tfce_adj_t* adj, const float* d_image, float* d_enhn, float 
   const size_t arr_bytes = ((size_t)V * sizeof(int32_t) + 255) / 256 * 256;
   const size_t ctl_bytes = (size_t)kCoopCtlWords * sizeof(int32_t);
   Workspace* ws = nullptr;
-  int rc = workspace_get(stream, rec_bytes + 256 + 8 * arr_bytes + ctl_bytes + 256, &ws);
+  const bool basin = adj->span.n > 0 && dh == 0.0f && min_t == 0.0f && g_coop_mode != 1;
+  size_t body = 8 * arr_bytes + ctl_bytes + 256;
+  BasinLayout bl;
+  if (basin) {
+    basin_layout(adj->span, 1, 1, true, body, &bl);
+    body = bl.bytes;
+  }
+  int rc = workspace_get(stream, rec_bytes + 256 + body, &ws);
   if (rc) return rc;
   char* base = reinterpret_cast<char*>(ws->ptr);
   int32_t* rec = reinterpret_cast<int32_t*>(base);
   float* raw = reinterpret_cast<float*>(base + rec_bytes);
   char* arr = base + rec_bytes + 256;
+  const int32_t* rest = nullptr;
+  hipError_t e;
+  if (basin) {
+    BasinArgs b{};
+    b.surfs = adj->d_surf;
+    b.n_surf = 1;
+    b.n_maps = 1;
+    b.pc = 1;
+    b.n_signs = 1;
+    b.sign0 = 1.0f;
+    b.maps = d_image;
+    b.map_stride = V;
+    b.prep = rec;
+    basin_span_args(adj->span, &b);
+    basin_place(bl, arr, &b);
+    b.queue = ws->queue;
+    b.enhn = d_enhn;
+    b.raw_max = raw;
+    b.status = d_status;
+    e = launch_basin_batch(b, adj->span.groups.data(), (int)adj->span.groups.size(), stream);
+    if (e != hipSuccess) return set_error(-(int)e, std::string("tfce basin launch: ") + hipGetErrorString(e));
+    if (adj->span.sure && adj->span.sure_full) return 0;
+    rest = b.rest;
+  }
   TfceBatchArgs a{};
   a.surfs = adj->d_surf;
   a.n_surf = 1;
@@ -922,9 +999,12 @@ static int run_coop(tfce_adj_t* adj, const float* d_image, float* d_enhn, float 
   a.n_items = 1;
   a.prep = rec;
   a.v_max = (int32_t)V;
-  hipError_t e = launch_tfce_batch(a, true, false, 1, 0, stream);
-  if (e != hipSuccess) return set_error(-(int)e, std::string("tfce record launch: ") + hipGetErrorString(e));
+  if (!basin) {
+    e = launch_tfce_batch(a, true, false, 1, 0, stream);
+    if (e != hipSuccess) return set_error(-(int)e, std::string("tfce record launch: ") + hipGetErrorString(e));
+  }
   TfceCoopArgs c{};
+  c.rest = rest;
   c.row_ptr = adj->d_row_ptr;
   c.col = adj->d_col;
   c.sizepow = adj->d_sizepow;
@@ -972,7 +1052,7 @@ int tfce_run_ex(tfce_adj_t* adj, const float* d_image, float* d_enhn, float min_
     return run_coop(adj, d_image, d_enhn, min_t, dh, d_status, stream);
   return run_batch(adj->d_surf, 1, adj->V, np_width(adj), d_image, adj->V, 1, 1, nullptr, nullptr, true, d_enhn, min_t,
                    dh, labels_level, d_labels, nullptr, nullptr, nullptr, d_status, stream, 1, 0, 0u, nullptr,
-                   (adj->flags & kSurfRing) != 0);
+                   (adj->flags & kSurfRing) != 0, 0, false, g_coop_mode == 0 ? nullptr : &adj->span);
 }
 
 int tfce_run(tfce_adj_t* adj, const float* d_image, float* d_enhn, float dh, int accumulate,

@@ -65,6 +65,7 @@ constexpr int kLdsMaxLevels = 128;
 struct BasinSurf {
   int32_t blk0, nblk, cand_blk, ev_cap;
   int64_t elt0, cand0, ev0;
+  int64_t tab0, tab_cap;  // FULL mode: first entry and number of entries of an image's gains
 };
 constexpr int kBasinBlock = 4096;
 // Levels per image the basin sweep takes.  A step of fl(T0 / 100) gives at
@@ -165,6 +166,7 @@ struct TfceCoopArgs {
   int32_t* ctl;            // [kCoopCtlWords], the barrier words zero at launch
   int32_t* status;         // [1] or null
   int32_t grid_limit;      // at most this many workgroups (0: one per compute unit)
+  const int32_t* rest;     // null, or a count: nothing is done where it is 0
 };
 // ctl layout: level starts [kMaxLevels + 1], cursors [kMaxLevels], root-list
 // lengths [3], failure flag [1], grid barrier counter and generation [2]
@@ -199,6 +201,7 @@ struct BasinArgs {
   const float* ext_T0;     // optional [n_items] first thresholds
   int32_t* prep;           // [n_items][kPrepWords]
   int32_t nb_max;          // most basins of an image taken here
+  int32_t q;               // workgroups of the vertex passes per kBasinBlock elements: 1 or 4
   int32_t blk_first, blk_total;  // workgroups of the vertex passes per map
   int64_t elt_total, cand_total, ev_total;
   // scratch of the chunk, [pc][...] each
@@ -207,10 +210,20 @@ struct BasinArgs {
   uint16_t* list;          // [elt_total] basins of the elements in level order
   uint64_t* cand;          // [cand_total] saddle pairs: level code | element << 16 | element << 40
   uint32_t* ev;            // [ev_total] saddle pairs in level order: basin | basin << 16
-  int32_t* blk;            // [blk_total][4] local maxima of each sign, saddle pairs
+  int32_t* blk;            // [blk_total * q][4] local maxima of each sign, saddle pairs
+  float* part;             // null, or [blk_total * q][4]: maxima of +map and -map per workgroup
   int32_t* unit;           // [surfaces][kBasinUnitWords]
   int32_t* rest;           // [1 + items] number and list of the items not taken
   int32_t* queue;          // work counter of the sweep of those
+  // FULL mode (tab not null): gains per level and basin [pc][n_signs][tab_total] (entries of an image:
+  // [level / 8][basin][level % 8]),
+  // the element's basins [elt_total], maxima per workgroup [blk_total * q][4]
+  float* tab;
+  int64_t tab_total;
+  uint16_t* bas;
+  float* part2;
+  float* enhn;             // accumulated image, or null
+  const float* vdensity;   // element weights of the rescaled maximum, or null
   // outputs, as TfceBatchArgs
   float* raw_max;
   float* scaled_max;
@@ -224,9 +237,9 @@ struct BasinGroup {
   int32_t width, s0, s1, blocks;
 };
 hipError_t launch_basin_batch(const BasinArgs& a, const BasinGroup* groups, int n_groups, hipStream_t stream);
-// The element-wise MAX sweep over a list of items whose records are written
+// The element-wise sweep over a list of items whose records are written
 // (a.rest; the work counter already zero).
-hipError_t launch_tfce_rest(const TfceBatchArgs& a, bool ring_only, int grid, hipStream_t stream);
+hipError_t launch_tfce_rest(const TfceBatchArgs& a, bool full, bool ring_only, int grid, hipStream_t stream);
 hipError_t launch_sizepow(double* out, int32_t n, float E, hipStream_t stream);
 hipError_t launch_shared_T0(const TfceBatchArgs& a, float* T0, int zero_in_image, hipStream_t stream);
 hipError_t launch_fill_f32(float* p, int64_t n, float v, hipStream_t stream);

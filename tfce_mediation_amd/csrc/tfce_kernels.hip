@@ -1919,6 +1919,7 @@ __global__ __launch_bounds__(kCoopThreads) void tfce_coop_kernel(TfceCoopArgs a)
   __shared__ float s_HH[kMaxLevels];
   __shared__ int s_start[kMaxLevels + 1];
   const int tid = threadIdx.x;
+  if (a.rest && a.rest[0] == 0) return;  // the same count for every workgroup
   const int status = a.rec[kPrepL];
   if (blockIdx.x == 0 && tid == 0 && a.status && status <= 0) a.status[0] = status;
   const int L = status > 0 ? status : 0;
@@ -2097,8 +2098,12 @@ hipError_t launch_tfce_batch(const TfceBatchArgs& a, bool full, bool ring_only, 
   return hipGetLastError();
 }
 
-hipError_t launch_tfce_rest(const TfceBatchArgs& a, bool ring_only, int grid, hipStream_t stream) {
-  if (ring_only)
+hipError_t launch_tfce_rest(const TfceBatchArgs& a, bool full, bool ring_only, int grid, hipStream_t stream) {
+  if (full && ring_only)
+    hipLaunchKernelGGL((tfce_batch_kernel<true, true>), dim3(grid), dim3(kTfceThreads), 0, stream, a);
+  else if (full)
+    hipLaunchKernelGGL((tfce_batch_kernel<true, false>), dim3(grid), dim3(kTfceThreads), 0, stream, a);
+  else if (ring_only)
     hipLaunchKernelGGL((tfce_batch_kernel<false, true>), dim3(grid), dim3(kTfceThreads), 0, stream, a);
   else
     hipLaunchKernelGGL((tfce_batch_kernel<false, false>), dim3(grid), dim3(kTfceThreads), 0, stream, a);
