@@ -426,7 +426,8 @@ static int perm_run(const tfce_ols_model_t* md, const int32_t* d_perm, int32_t P
   // whole permutations (the epilogue reads a permutation's rows from LDS, so
   // they need not align with the 32-row MFMA tiles)
   const int rpp = md->m > 0 ? md->m : 1;
-  const int tile = (d->precision == kPrecFP32 || n_blk > 0) ? 0 : g_gemm_tile;
+  const bool any_tile = d->precision != kPrecFP32 && ols_gemm_any_tile(md->f, md2 != nullptr, tss || n_blk > 0);
+  const int tile = any_tile ? g_gemm_tile : 0;
   const int tile_rows = d->precision == kPrecFP32 ? kGemmRows : gemm_tile_rows(tile);
   const int tile_cols = d->precision == kPrecFP32 ? kGemmCols : gemm_tile_cols(tile);
   const int per_tile = tile_rows / rpp;
@@ -566,6 +567,7 @@ static int perm_run(const tfce_ols_model_t* md, const int32_t* d_perm, int32_t P
     ga.alg = alg;
     ga.f2 = md2->f;
     ga.k2 = md2->k;
+    ga.inv_dof2 = 1.0 / (double)(d->n - md2->k);
     ga.con2 = md2->con[0];
     ga.con2_is_intercept = md2->con_is_intercept[0];
     ga.shared2 = md2->shared ? 1 : 0;
@@ -575,7 +577,12 @@ static int perm_run(const tfce_ols_model_t* md, const int32_t* d_perm, int32_t P
     ga.hF2 = md2->hF;
     ga.r02 = md2->r0;
   }
-  e = launch_ols_gemm(ga, d->precision, tile, stream);
+  switch (d->precision) {
+    case kPrecFP32: e = launch_ols_gemm_fp32(ga, stream); break;
+    case kPrecFP16x3: e = launch_ols_gemm_fp16x3(ga, tile, stream); break;
+    case kPrecBF16x3: e = launch_ols_gemm_bf16x3(ga, tile, stream); break;
+    default: e = launch_ols_gemm_bf16x6(ga, tile, stream); break;
+  }
   if (e != hipSuccess) return set_error(-(int)e, "ols gemm launch");
   return 0;
 }

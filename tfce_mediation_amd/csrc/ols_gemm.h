@@ -1,0 +1,611 @@
+// Permuted contraction and its epilogues (see ols_kernels.hip for what is
+// computed), instantiated per precision in ols_gemm_*.hip.
+#pragma once
+#include <type_traits>
+
+#include "ols_internal.h"
+#include "ols_math.h"
+
+namespace tfcehip {
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// What a kernel's epilogue computes: an instance each, so that none carries
+// another's registers (the t epilogues together took 240 registers instead of
+// 100, one workgroup per compute unit instead of two).
+enum EpiKind {
+  kEpiT1,    // t, at most one fixed column
+  kEpiT2,    // t, two fixed columns
+  kEpiT4,    // t, three or four
+  kEpiT7,    // t, five to seven
+  kEpiPair,  // z of a mediation's two models
+  kEpiF,     // sqrt(max(F, 0)) of the whole model
+  kEpiBlk,   // partial F of column blocks
+};
+
+// F epilogues for one (permutation, element): gz holds X_p'y for the permuted
+// columns (FP32 accumulators), everything else comes from per-element and
+// per-permutation tables.
+// UNIFORM: the caller guarantees p is the same in every lane of the wave, so
+// the permutation's factor is read with scalar loads.
+template <bool UNIFORM, bool BLK>
+__device__ __forceinline__ void f_epilogue(const OlsGemmArgs& a, int p, int64_t col, const float* gz, const float* gF,
+                                           const float* hF, double r0) {
+  const int f = a.f, m = a.m, k = f + m;
+  const int fi = a.shared_factor ? 0 : (UNIFORM ? __builtin_amdgcn_readfirstlane(p) : p);
+  const float* L = a.Linv + (int64_t)fi * 64;
+  float hz[kOlsMaxK];
+  double ssz = 0.0;
+#pragma unroll
+  for (int i = 0; i < kOlsMaxK; ++i) {
+    hz[i] = 0.0f;
+    if (i < m) {
+      const int row = f + i;
+      float s = 0.0f;
+#pragma unroll
+      for (int j = 0; j < kOlsMaxK; ++j)
+        if (j < f) s = fmaf(L[row * 8 + j], gF[j], s);
+#pragma unroll
+      for (int j = 0; j < kOlsMaxK; ++j)
+        if (j <= i) s = fmaf(L[row * 8 + f + j], gz[j], s);
+      hz[i] = s;
+      ssz += (double)s * (double)s;
+    }
+  }
+  double sse = r0 - ssz;
+  if (sse < 0.0) sse = 0.0;
+  if constexpr (BLK) {
+    // partial F of each column block: |Rb h|^2 / w over SSE / (n - k)
+    // (pyfunc.py:2340-2352 computes the same extra sum of squares as the
+    // difference of the reduced and the full model's residual sums)
+    const float* R = a.Rb + (int64_t)(a.blk_shared ? 0 : fi) * a.n_blk * 64;
+    const double s2 = sse / (double)(a.n - k);
+#pragma unroll 1
+    for (int b = 0; b < a.n_blk; ++b) {
+      double ex = 0.0;
+#pragma unroll 1
+      for (int r = 0; r < a.blk_w[b]; ++r) {
+        const float* Rr = R + b * 64 + r * 8;
+        float u = 0.0f;
+#pragma unroll
+        for (int j = 0; j < kOlsMaxK; ++j)
+          if (j < k) u = fmaf(Rr[j], (j < f) ? hF[j] : hz[(j - f) & (kOlsMaxK - 1)], u);
+        ex += (double)u * (double)u;
+      }
+      a.t[((int64_t)b * a.P + p) * a.ldt + col] = (float)(ex / (double)a.blk_w[b] / s2);
+    }
+    return;
+  }
+  // F of the whole model against the caller's total sum of squares
+  // (cynumstats.pyx:31-36), as sqrt(max(F, 0)) (voxel randomise :85-87)
+  const double F = ((a.tss[col] - sse) / (double)(k - 1)) / (sse / (double)(a.n - k));
+  a.t[(int64_t)p * a.ldt + col] = (float)(F < 0.0 ? 0.0 : sqrt(F));
+}
+
+// t of contrast column ci of a model with f fixed columns (FF > 0: a
+// compile-time f) and one permuted column whose X_p'y is gz0: the arithmetic
+// of epi_t for m = 1, operation for operation.
+template <int FF>
+__device__ __forceinline__ float single_t(int f_rt, int k, double inv_dof, const float* L, double dcv, int ci, int is_icpt,
+                                          int centered, const float* gF, const float* hF, double r0, double mu,
+                                          float gz0) {
+  const int f = FF > 0 ? FF : f_rt;
+  float s = 0.0f;
+#pragma unroll
+  for (int j = 0; j < kOlsMaxK; ++j)
+    if (j < f) s = fmaf(L[f * 8 + j], gF[j], s);
+  s = fmaf(L[f * 8 + f], gz0, s);
+  const double ssz = 0.0 + (double)s * (double)s;
+  double sse = r0 - ssz;
+  if (sse < 0.0) sse = 0.0;
+  float ac = 0.0f;
+#pragma unroll
+  for (int j = 0; j < kOlsMaxK; ++j) {
+    if (j >= ci && j < k) {
+      const float hj = (j < f) ? hF[j] : s;
+      ac = fmaf(L[j * 8 + ci], hj, ac);
+    }
+  }
+  const float se = sqrt_f32(sse * inv_dof * dcv);
+  if (centered && is_icpt) return (float)(((double)ac + mu) / (double)se);
+  return __fdiv_rn(ac, se);  // what the double quotient rounds to: its 53 bits hold a float quotient's tie
+}
+
+// Epilogue through LDS.  The accumulators of a wave cover, for tile (rt, ct),
+// rows row0 + 32 rt + 8 (i / 4) + 4 h + (i % 4) (i = accumulator index 0..15)
+// of column 32 ct + r.  The workgroup writes one 32-column slice of every
+// wave's tiles into an LDS block ep[256 rows][ldc], then each thread owns one
+// column of the block and walks permutations: it reads the permutation's
+// rpp rows (X_p'y for the permuted columns) and runs the per-element
+// epilogue.  Unrolled register code stays small (only the LDS write is
+// unrolled), so the accumulators never leave registers for scratch.
+template <int RT, int CT>
+__device__ __forceinline__ void epi_put(float* ep, int ldc, const f32x16 (&acc)[RT][CT], int sel, int row0,
+                                        int c0, int h, int r) {
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) {
+    if (ct != sel) continue;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        ep[(row0 + 32 * rt + 8 * (i >> 2) + 4 * h + (i & 3)) * ldc + c0 + r] = acc[rt][ct][i];
+  }
+}
+
+// Thread (cl, slot): column cl of the block (global element `col`),
+// permutations slot, slot + step, ... of the workgroup's row tile.
+template <int LDC, bool BLK>
+__device__ __forceinline__ void epi_loop_f(const OlsGemmArgs& a, const float* ep, int cl, int64_t col, int p0, int ppt,
+                                         int slot, int step, const float* gF, const float* hF, double r0, double mu,
+                                         float yinv) {
+  const int m = a.m, rpp = a.rpp;
+  for (int pp = slot; pp < ppt; pp += step) {
+    const int p = p0 + pp;
+    if (p >= a.P) break;
+    float gz[kOlsMaxK];
+#pragma unroll
+    for (int q = 0; q < kOlsMaxK; ++q) {
+      gz[q] = q < m ? ep[(pp * rpp + q) * LDC + cl] : 0.0f;
+      if (a.yinv) gz[q] = gz[q] * a.zinv[q] * yinv;  // powers of two: exact
+      if (!a.centered && q < m) gz[q] += (float)(a.colsumZ[q] * mu);
+    }
+    // with 64 columns per block a wave's lanes share one permutation
+    f_epilogue<LDC == 64, BLK>(a, p, col, gz, gF, hF, r0);
+  }
+}
+
+// t-values of the contrasts: epi_loop_f's walk with the column counts as
+// compile-time constants, M permuted columns and FC >= f fixed ones (gF and hF
+// hold zeros beyond f, which add nothing).  Bound by
+// instructions: at 84M values (256 permutations of 327,684 elements, five
+// permuted columns) the epilogue was 0.65 of the contraction's 2.1 ms with the
+// library's FP64 square root and two FP64 divisions per value; the square root
+// is sqrt_f32, the division by n - k a multiplication, and a / se the float
+// quotient.  Two permutations per iteration, so that their chains overlap (two
+// waves per SIMD).
+// kUniform: L and dc are read through the constant address space, so that a
+// wave-uniform address gives scalar loads also after the kernel's own stores
+// (vector loads of the factor took the registers from 100 to 240).
+template <bool U>
+struct FactorPtr {
+  typedef const float* F;
+  typedef const double* D;
+};
+template <>
+struct FactorPtr<true> {
+  typedef const __attribute__((address_space(4))) float* F;
+  typedef const __attribute__((address_space(4))) double* D;
+};
+
+template <int LDC, int FC, int M>
+__device__ __forceinline__ void epi_t(const OlsGemmArgs& a, const float* ep, int cl, int64_t col, int p0, int ppt,
+                                      int slot, int step, const float* gF, const float* hF, double r0, double mu,
+                                      float yinv) {
+  constexpr int U = LDC >= 64 ? 2 : 1;
+  constexpr bool kUniform = LDC >= 64;  // a wave's lanes share one permutation
+  const int f = a.f;
+  ppt = min(ppt, a.P - p0);
+  for (int i0 = slot; i0 < ppt; i0 += U * step) {
+    float hz[U][M];
+    double x[U];
+    typename FactorPtr<kUniform>::F L[U];
+    int fi[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = min(i0 + u * step, ppt - 1);
+      fi[u] = a.shared_factor ? 0 : (kUniform ? __builtin_amdgcn_readfirstlane(p0 + i) : p0 + i);
+      L[u] = (typename FactorPtr<kUniform>::F)(a.Linv + (int64_t)fi[u] * 64);
+      float gz[M];
+#pragma unroll
+      for (int q = 0; q < M; ++q) {
+        gz[q] = ep[(i * M + q) * LDC + cl];
+        if (a.yinv) gz[q] = gz[q] * a.zinv[q] * yinv;  // powers of two: exact
+        if (!a.centered) gz[q] += (float)(a.colsumZ[q] * mu);
+      }
+      double ssz = 0.0;
+#pragma unroll
+      for (int r = 0; r < M; ++r) {
+        const auto row = L[u] + (f + r) * 8;
+        float s = 0.0f;
+#pragma unroll
+        for (int j = 0; j < FC; ++j) s = fmaf(row[j], gF[j], s);
+#pragma unroll
+        for (int j = 0; j <= r; ++j) s = fmaf(row[f + j], gz[j], s);
+        hz[u][r] = s;
+        ssz = fma((double)s, (double)s, ssz);  // the product is exact
+      }
+      const double sse = r0 - ssz;
+      x[u] = (sse < 0.0 ? 0.0 : sse) * a.inv_dof;
+    }
+    for (int c = 0; c < a.n_con; ++c) {
+      const int ci = a.con[c];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        float ac = 0.0f;
+        if (ci < f) {
+#pragma unroll
+          for (int j = 0; j < FC; ++j) ac = fmaf(L[u][j * 8 + ci], hF[j], ac);
+        }
+#pragma unroll
+        for (int r = 0; r < M; ++r) ac = fmaf(L[u][(f + r) * 8 + ci], hz[u][r], ac);
+        const auto dc = (typename FactorPtr<kUniform>::D)(a.dc + (int64_t)fi[u] * kOlsMaxContrasts);
+        const float se = sqrt_f32(x[u] * dc[c]);
+        // a / se is what the double quotient rounds to (53 bits hold a float
+        // quotient's tie)
+        const float t = (a.centered && a.con_is_intercept[c]) ? (float)(((double)ac + mu) / (double)se)
+                                                              : __fdiv_rn(ac, se);
+        if (i0 + u * step < ppt) a.t[((int64_t)c * a.P + p0 + i0 + u * step) * a.ldt + col] = t;
+      }
+    }
+  }
+}
+
+// epi_t for the model's column counts.
+template <int LDC, int FC>
+__device__ __forceinline__ void epi_t_cols(const OlsGemmArgs& a, const float* ep, int cl, int64_t col, int p0, int ppt,
+                                           int slot, int step, const float* gF, const float* hF, double r0, double mu,
+                                           float yinv) {
+  // (f + m <= 8)
+  switch (a.m) {
+    case 1: epi_t<LDC, FC, 1>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
+    case 2: epi_t<LDC, FC, 2>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
+    case 3: epi_t<LDC, FC, 3>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
+  }
+  if constexpr (FC <= 4) {
+    switch (a.m) {
+      case 4: epi_t<LDC, FC, 4>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
+      case 5: epi_t<LDC, FC, 5>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
+    }
+  }
+  if constexpr (FC <= 2) {
+    switch (a.m) {
+      case 6: epi_t<LDC, FC, 6>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
+      case 7: epi_t<LDC, FC, 7>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
+      case 8: epi_t<LDC, FC, 8>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
+    }
+  }
+}
+
+// The paired mediation epilogue: thread (cl, slot) walks its permutations,
+// computes t of both models from the one permuted column's X_p'y, and writes z.
+template <int LDC, int F1, int F2>
+__device__ __forceinline__ void epi_loop_pair(const OlsGemmArgs& a, const float* ep, int cl, int64_t col, int p0,
+                                              int ppt, int slot, int step, double mu, float yinv) {
+  float gF1[kOlsMaxK], hF1[kOlsMaxK], gF2[kOlsMaxK], hF2[kOlsMaxK];
+#pragma unroll
+  for (int q = 0; q < kOlsMaxK; ++q) {
+    gF1[q] = q < a.f ? a.gF[(int64_t)q * a.V + col] : 0.0f;
+    hF1[q] = q < a.f ? a.hF[(int64_t)q * a.V + col] : 0.0f;
+    gF2[q] = q < a.f2 ? a.gF2[(int64_t)q * a.V + col] : 0.0f;
+    hF2[q] = q < a.f2 ? a.hF2[(int64_t)q * a.V + col] : 0.0f;
+  }
+  const double r01 = a.r0[col], r02 = a.r02[col];
+  for (int pp = slot; pp < ppt; pp += step) {
+    const int p = p0 + pp;
+    if (p >= a.P) break;
+    float gz0 = ep[pp * LDC + cl];
+    if (a.yinv) gz0 = gz0 * a.zinv[0] * yinv;  // powers of two: exact
+    if (!a.centered) gz0 += (float)(a.colsumZ[0] * mu);
+    const int fi1 = a.shared_factor ? 0 : p, fi2 = a.shared2 ? 0 : p;
+    const float ta = single_t<F1>(a.f, a.k, a.inv_dof, a.Linv + (int64_t)fi1 * 64, a.dc[(int64_t)fi1 * kOlsMaxContrasts],
+                                  a.con[0], a.con_is_intercept[0], a.centered, gF1, hF1, r01, mu, gz0);
+    const float tb = single_t<F2>(a.f2, a.k2, a.inv_dof2, a.Linv2 + (int64_t)fi2 * 64,
+                                  a.dc2[(int64_t)fi2 * kOlsMaxContrasts], a.con2, a.con2_is_intercept, a.centered,
+                                  gF2, hF2, r02, mu, gz0);
+    a.t[(int64_t)p * a.ldt + col] = sobel_z((double)ta, (double)tb, a.alg);
+  }
+}
+
+template <int LDC, EpiKind EPI>
+__device__ __forceinline__ void epi_run(const OlsGemmArgs& a, const float* ep, int cl, int64_t col, int64_t mrow0,
+                                        int rows, int slot, int step) {
+  const bool cvalid = col < a.V;
+  if (!cvalid) return;
+  const double mu = a.mu[col];
+  const float yinv = a.yinv ? a.yinv[col] : 1.0f;
+  const int ppt = rows / a.rpp;
+  const int p0 = (int)(mrow0 / rows) * ppt;
+  if constexpr (EPI == kEpiPair) {
+    // mediation types M and I: path A [1, x], path B [1, y, x]
+    if (a.f == 1 && a.f2 == 2) epi_loop_pair<LDC, 1, 2>(a, ep, cl, col, p0, ppt, slot, step, mu, yinv);
+    else epi_loop_pair<LDC, 0, 0>(a, ep, cl, col, p0, ppt, slot, step, mu, yinv);
+    return;
+  }
+  float gF[kOlsMaxK], hF[kOlsMaxK];
+#pragma unroll
+  for (int q = 0; q < kOlsMaxK; ++q) {
+    gF[q] = q < a.f ? a.gF[(int64_t)q * a.V + col] : 0.0f;
+    hF[q] = q < a.f ? a.hF[(int64_t)q * a.V + col] : 0.0f;
+  }
+  const double r0 = a.r0[col];
+  if constexpr (EPI == kEpiT1) epi_t_cols<LDC, 1>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv);
+  if constexpr (EPI == kEpiT2) epi_t_cols<LDC, 2>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv);
+  if constexpr (EPI == kEpiT4) epi_t_cols<LDC, 4>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv);
+  if constexpr (EPI == kEpiT7) epi_t_cols<LDC, 7>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv);
+  if constexpr (EPI == kEpiF) epi_loop_f<LDC, false>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv);
+  if constexpr (EPI == kEpiBlk) epi_loop_f<LDC, true>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv);
+}
+
+// Block -> tile mapping shared by both contraction kernels: the n_mtiles row
+// tiles of one column tile are consecutive blocks of one XCD (blockIdx mod 8),
+// so that XCD's L2 holds the column tile of Y while all of them read it.
+__device__ __forceinline__ bool gemm_tile(const OlsGemmArgs& a, int& mt, int& nt) {
+  const int b = blockIdx.x, xcd = b & 7, jb = b >> 3;
+  mt = jb % a.n_mtiles;
+  nt = (jb / a.n_mtiles) * 8 + xcd;
+  return nt < a.n_ntiles;
+}
+
+// Plain FP32 contraction (v_mfma_f32_32x32x2f32): each wave holds 64 rows x
+// 128 columns and reads its fragments straight from global memory.
+template <EpiKind EPI>
+__global__ __launch_bounds__(256) void ols_gemm_fp32_kernel(OlsGemmArgs a) {
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, h = l >> 5, r = l & 31;
+  int mt, nt;
+  if (!gemm_tile(a, mt, nt)) return;
+  const int64_t m0 = (int64_t)mt * kGemmRows + w * 64;
+  const int64_t n0 = (int64_t)nt * kGemmCols;
+  f32x16 acc[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
+  const int nkg = a.Kp / 8;
+  for (int kg0 = 0; kg0 < nkg; kg0 += 2) {
+    const int kg = kg0 + h;
+    float A[2][8], B[4][8];
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      const float4* s = reinterpret_cast<const float4*>(a.a32 + ((int64_t)kg * a.Mpad + m0 + 32 * rt + r) * 8);
+      float4 x0 = s[0], x1 = s[1];
+      A[rt][0] = x0.x; A[rt][1] = x0.y; A[rt][2] = x0.z; A[rt][3] = x0.w;
+      A[rt][4] = x1.x; A[rt][5] = x1.y; A[rt][6] = x1.z; A[rt][7] = x1.w;
+    }
+#pragma unroll
+    for (int ct = 0; ct < 4; ++ct) {
+      const float4* s = reinterpret_cast<const float4*>(a.b32 + ((int64_t)kg * a.Npad + n0 + 32 * ct + r) * 8);
+      float4 x0 = s[0], x1 = s[1];
+      B[ct][0] = x0.x; B[ct][1] = x0.y; B[ct][2] = x0.z; B[ct][3] = x0.w;
+      B[ct][4] = x1.x; B[ct][5] = x1.y; B[ct][6] = x1.z; B[ct][7] = x1.w;
+    }
+#pragma unroll
+    for (int jj = 0; jj < 8; ++jj)
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < 4; ++ct)
+          acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x2f32(A[rt][jj], B[ct][jj], acc[rt][ct], 0, 0, 0);
+  }
+  // epilogue: four passes of 32 columns through a [256][32] LDS block
+  __shared__ float ep[kGemmRows * 32];
+#pragma unroll
+  for (int pass = 0; pass < 4; ++pass) {
+    __syncthreads();
+    epi_put<2, 4>(ep, 32, acc, pass, w * 64, 0, h, r);
+    __syncthreads();
+    epi_run<32, EPI>(a, ep, tid & 31, n0 + 32 * pass + (tid & 31), (int64_t)mt * kGemmRows, kGemmRows, tid >> 5, 8);
+  }
+}
+
+// Split-bf16 / split-fp16 contraction staged through LDS.  The waves of a
+// workgroup form a WR x WC grid of 128 x 64 wave tiles (4 x 2 MFMA 32x32x16
+// tiles each), so the workgroup tile is (128 WR) rows x (64 WC) columns; the
+// shape is a launch-time choice (the autotuner's).  One k step is a pair of
+// k-groups (16 k); its A fragments ([2][rows][8] per plane) and B fragments
+// ([2][columns][8]) are copied global -> LDS by the LDS DMA
+// (global_load_lds_dwordx4: each wave instruction moves 64 consecutive
+// 16-byte fragments, landing at consecutive LDS addresses), so every A and B
+// element crosses from L2 once per workgroup instead of once per wave.  Two
+// LDS stages: step s issues the DMA of step s+1 into the other stage, then
+// reads its own fragments into registers and runs its MFMAs (each group of
+// products waits only for the fragments it uses) while that DMA is in
+// flight; one barrier per step separates the DMA of a stage from the reads
+// of the step before.
+template <int NP, int WR, int WC>
+struct GemmStage {
+  static constexpr int kRows = 128 * WR, kCols = 64 * WC, kThreads = 64 * WR * WC;
+  static constexpr int kA = 2 * kRows * 16;   // bytes of A per plane
+  static constexpr int kB = 2 * kCols * 16;   // bytes of B per plane
+  static constexpr int kPlane = kA + kB;
+  static constexpr int kBytes = NP * kPlane;
+  static constexpr int kEpi = kRows * 32 * WC * 4;  // epilogue block: rows x (32 WC) floats
+  // LDS stages: the loop is written for 2 or 3 (two copies in flight behind
+  // the one being read); 3 measured slower on MI355X at C3 (less occupancy,
+  // no gain in overlap), so 2.
+  static constexpr int kStages = 2;
+  static constexpr int kSmem = kStages * kBytes > kEpi ? kStages * kBytes : kEpi;
+  // fewest copies any wave issues per stage (the round-robin leaves the last
+  // waves one short when a chunk count is not a multiple of the wave count)
+  static constexpr int kMinCopies = NP * ((2 * kRows / 64) / (WR * WC) + (2 * kCols / 64) / (WR * WC));
+};
+
+// s_waitcnt immediate for vmcnt(n) with lgkmcnt and expcnt left free (gfx9
+// encoding: vmcnt[3:0] and [15:14], expcnt [6:4], lgkmcnt [11:8]).
+template <int N>
+struct VmCnt {
+  static_assert(N >= 0 && N < 64, "vmcnt range");
+  static constexpr int kImm = (N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8);
+};
+
+// The 1 KiB copies of one stage (64 rows or columns of one k-group of one
+// plane each) go round-robin over the waves.
+template <int NP, int WR, int WC>
+__device__ __forceinline__ void gemm_stage_copy(const OlsGemmArgs& a, uint8_t* stage, int kg0, int64_t mrow0,
+                                                int64_t ncol0, int w) {
+  using S = GemmStage<NP, WR, WC>;
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  constexpr int W = WR * WC, nA = 2 * S::kRows / 64, nB = 2 * S::kCols / 64;
+  const int l = threadIdx.x & 63;
+#pragma unroll
+  for (int q = 0; q < NP; ++q) {
+#pragma unroll
+    for (int c0 = 0; c0 < nA; c0 += W) {
+      const int c = c0 + w;
+      if (c < nA) {
+        const int j = c / (S::kRows / 64), rc = (c % (S::kRows / 64)) * 64;
+        const uint16_t* src = a.abf[q] + ((int64_t)(kg0 + j) * a.Mpad + mrow0 + rc + l) * 8;
+        __builtin_amdgcn_global_load_lds((const void*)src,
+                                         (lds_ptr)(stage + q * S::kPlane + (j * S::kRows + rc) * 16), 16, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int c0 = 0; c0 < nB; c0 += W) {
+      const int c = c0 + w;
+      if (c < nB) {
+        const int j = c / (S::kCols / 64), nc = (c % (S::kCols / 64)) * 64;
+        const uint16_t* src = a.bbf[q] + ((int64_t)(kg0 + j) * a.Npad + ncol0 + nc + l) * 8;
+        __builtin_amdgcn_global_load_lds((const void*)src,
+                                         (lds_ptr)(stage + q * S::kPlane + S::kA + (j * S::kCols + nc) * 16), 16,
+                                         0, 0);
+      }
+    }
+  }
+}
+
+template <int NP, bool F16, int WR, int WC, EpiKind EPI>
+__global__ __launch_bounds__(64 * WR * WC) void ols_gemm_split_kernel(OlsGemmArgs a) {
+  using S = GemmStage<NP, WR, WC>;
+  __shared__ __attribute__((aligned(16))) uint8_t smem[S::kSmem];
+  const int tid = threadIdx.x, l = tid & 63, h = l >> 5, r = l & 31;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = w / WC, wc = w % WC;
+  int mt, nt;
+  if (!gemm_tile(a, mt, nt)) return;
+  const int64_t mrow0 = (int64_t)mt * S::kRows, ncol0 = (int64_t)nt * S::kCols;
+  f32x16 acc[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.0f;
+
+  const int nsteps = a.Kp / 16;  // k steps of two k-groups
+  constexpr int D = S::kStages;
+#pragma unroll
+  for (int s = 0; s < D - 1; ++s)
+    if (s < nsteps) gemm_stage_copy<NP, WR, WC>(a, smem + s * S::kBytes, 2 * s, mrow0, ncol0, w);
+  for (int step = 0; step < nsteps; ++step) {
+    // stage `step` has landed once at most the copies of the stages issued
+    // after it are outstanding (counted with the fewest copies per wave, so
+    // a wave with more copies waits a little longer than it must)
+    if (D == 3 && step + 1 < nsteps)
+      __builtin_amdgcn_s_waitcnt(VmCnt<S::kMinCopies>::kImm);
+    else
+      __builtin_amdgcn_s_waitcnt(VmCnt<0>::kImm);
+    // Every wave's copies of this stage have landed (each wave waited for its
+    // own above), and every wave has finished reading the stage the next copy
+    // reuses.  A bare s_barrier: __syncthreads' release fence would also wait
+    // for the copies still in flight.  The empty asm keeps the compiler from
+    // moving LDS reads across it.
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    // the copy of a later stage goes first, into the buffer every wave
+    // finished reading before the barrier, so that the fragment reads below
+    // are the last LDS operations before the products and can be waited for
+    // in part
+    if (step + D - 1 < nsteps)
+      gemm_stage_copy<NP, WR, WC>(a, smem + ((step + D - 1) % D) * S::kBytes, 2 * (step + D - 1), mrow0, ncol0, w);
+    const uint8_t* cur = smem + (step % D) * S::kBytes;
+    typedef typename std::conditional<F16, f16x8, bf16x8>::type op8;
+    op8 A[NP][4], B[NP][2];
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt)
+        A[q][rt] = *reinterpret_cast<const op8*>(cur + q * S::kPlane +
+                                                  (h * S::kRows + wr * 128 + 32 * rt + r) * 16);
+#pragma unroll
+      for (int ct = 0; ct < 2; ++ct)
+        B[q][ct] = *reinterpret_cast<const op8*>(cur + q * S::kPlane + S::kA +
+                                                  (h * S::kCols + wc * 64 + 32 * ct + r) * 16);
+    }
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+      for (int ct = 0; ct < 2; ++ct) {
+        f32x16 c = acc[rt][ct];
+        if constexpr (F16) {
+          c = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[1][rt], B[0][ct], c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[0][rt], B[1][ct], c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[0][rt], B[0][ct], c, 0, 0, 0);
+        } else {
+          if constexpr (NP == 3) {
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[2][rt], B[0][ct], c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[1][rt], B[1][ct], c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[0][rt], B[2][ct], c, 0, 0, 0);
+          }
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[1][rt], B[0][ct], c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[0][rt], B[1][ct], c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[0][rt], B[0][ct], c, 0, 0, 0);
+        }
+        acc[rt][ct] = c;
+      }
+  }
+  // epilogue: two passes (column tile ct of every wave) through an LDS block
+  // [rows][32 WC] that reuses the staging buffer
+  float* ep = reinterpret_cast<float*>(smem);
+  constexpr int ldc = 32 * WC;
+#pragma unroll
+  for (int pass = 0; pass < 2; ++pass) {
+    __syncthreads();
+    epi_put<4, 2>(ep, ldc, acc, pass, wr * 128, wc * 32, h, r);
+    __syncthreads();
+    const int cl = tid % ldc;
+    epi_run<ldc, EPI>(a, ep, cl, ncol0 + (cl >> 5) * 64 + 32 * pass + (cl & 31), mrow0, S::kRows, tid / ldc,
+                 S::kThreads / ldc);
+  }
+}
+
+inline EpiKind epi_kind(const OlsGemmArgs& a) {
+  if (a.n_blk > 0) return kEpiBlk;
+  if (a.pair) return kEpiPair;
+  if (a.tss) return kEpiF;
+  return a.f <= 1 ? kEpiT1 : (a.f == 2 ? kEpiT2 : (a.f <= 4 ? kEpiT4 : kEpiT7));
+}
+
+inline unsigned gemm_blocks(const OlsGemmArgs& a) {
+  return (unsigned)((int64_t)(a.n_ntiles + 7) / 8 * 8 * a.n_mtiles);
+}
+
+template <int NP, bool F16, int WR, int WC, EpiKind EPI>
+void launch_one(const OlsGemmArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL((ols_gemm_split_kernel<NP, F16, WR, WC, EPI>), dim3(gemm_blocks(a)), dim3(64 * WR * WC), 0, s, a);
+}
+
+// The tiles other than 256 x 128 are compiled for the epilogues that
+// ols_gemm_any_tile names (the caller sizes the rows for tile 0 otherwise).
+template <int NP, bool F16, int WR, int WC>
+void launch_tile(const OlsGemmArgs& a, hipStream_t s) {
+  const EpiKind e = epi_kind(a);
+  if (e == kEpiPair) return launch_one<NP, F16, WR, WC, kEpiPair>(a, s);
+  if (e == kEpiT2) return launch_one<NP, F16, WR, WC, kEpiT2>(a, s);
+  if constexpr (WR == 2 && WC == 2) {
+    if (e == kEpiT4) return launch_one<NP, F16, WR, WC, kEpiT4>(a, s);
+    if (e == kEpiT7) return launch_one<NP, F16, WR, WC, kEpiT7>(a, s);
+    if (e == kEpiF) return launch_one<NP, F16, WR, WC, kEpiF>(a, s);
+    if (e == kEpiBlk) return launch_one<NP, F16, WR, WC, kEpiBlk>(a, s);
+  }
+  launch_one<NP, F16, WR, WC, kEpiT1>(a, s);
+}
+
+template <int NP, bool F16>
+hipError_t launch_split(const OlsGemmArgs& a, int tile, hipStream_t s) {
+  if (tile == 1) launch_tile<NP, F16, 4, 1>(a, s);
+  else if (tile == 2) launch_tile<NP, F16, 4, 2>(a, s);
+  else if (tile == 3) launch_tile<NP, F16, 2, 4>(a, s);
+  else launch_tile<NP, F16, 2, 2>(a, s);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+}  // namespace tfcehip

@@ -116,6 +116,7 @@ struct OlsGemmArgs {
   // contrast 0 of each model combine into the Sobel-type z of alg (0 aroian,
   // 1 sobel, 2 goodman), written to t[p][col].
   int32_t pair, alg;
+  double inv_dof2;       // 1 / (n - k2)
   int32_t f2, k2, con2, con2_is_intercept, shared2;
   const float* Linv2;    // [P or 1][8][8]
   const double* dc2;     // [P or 1][kOlsMaxContrasts]
@@ -193,6 +194,12 @@ hipError_t launch_ols_build_a(const OlsBuildAArgs& a, hipStream_t s);
 constexpr int kGemmTiles = 4;
 inline int gemm_tile_rows(int tile) { return (tile == 0 || tile == 3) ? 256 : 512; }
 inline int gemm_tile_cols(int tile) { return tile == 1 ? 64 : (tile == 3 ? 256 : 128); }
-hipError_t launch_ols_gemm(const OlsGemmArgs& a, int precision, int tile, hipStream_t s);
+// Whether every tile is compiled for a design's epilogue: t with at most two
+// fixed columns, and the mediation z.  The others take tile 0.
+inline bool ols_gemm_any_tile(int fixed, bool pair, bool f_statistic) { return pair || (!f_statistic && fixed <= 2); }
+hipError_t launch_ols_gemm_fp32(const OlsGemmArgs& a, hipStream_t s);
+hipError_t launch_ols_gemm_fp16x3(const OlsGemmArgs& a, int tile, hipStream_t s);
+hipError_t launch_ols_gemm_bf16x3(const OlsGemmArgs& a, int tile, hipStream_t s);
+hipError_t launch_ols_gemm_bf16x6(const OlsGemmArgs& a, int tile, hipStream_t s);
 
 }  // namespace tfcehip

@@ -1,0 +1,48 @@
+// FP64 square roots of the t and z epilogues.
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace tfcehip {
+
+// Square root of a positive, finite double: the hardware's reciprocal square
+// root (24 bits and more) and two residual corrections, each squaring its
+// error; within 1 ulp of the rounded root (the library's sqrt, with its scaling
+// for subnormal arguments, is three times as many instructions).
+__device__ __forceinline__ double sqrt_pos(double x) {
+  const double r = __builtin_amdgcn_rsq(x), h = 0.5 * r;
+  double s = x * r;
+  s = fma(fma(-s, s, x), h, s);
+  return fma(fma(-s, s, x), h, s);
+}
+
+// fl32(sqrt(x)), x >= 0 or NaN
+__device__ __forceinline__ float sqrt_f32(double x) {
+  return (x > 0.0 && x < (double)INFINITY) ? (float)sqrt_pos(x) : (float)x;
+}
+
+// Sobel-type z of the indirect effect from the two path t-values
+// (pyfunc.py:150-161, calc_indirect :2678-2709): 0 aroian, 1 sobel, 2 goodman.
+// 1 / sqrt(1/b^2 + 1/a^2 [+ or - 1/(a^2 b^2)]) = sqrt(a^2 b^2 / (a^2 + b^2 [+ or
+// - 1])), one root in place of three divisions, a root and a division; written
+// out as the reference writes it where a t is zero, infinite or NaN.
+__device__ __forceinline__ float sobel_z(double a, double b, int alg) {
+  const double A = a * a, B = b * b;  // exact
+  const double N = A * B, D = A + B + (alg == 0 ? 1.0 : (alg == 1 ? 0.0 : -1.0));
+  const double nd = N * D;
+  if (nd > 0.0 && nd < (double)INFINITY) {
+    const double r = __builtin_amdgcn_rsq(nd), h = 0.5 * r;
+    double s = nd * r;  // sqrt(N D), z = N / sqrt(N D)
+    s = fma(fma(-s, s, nd), h, s);
+    double q = fma(fma(-s, r, 1.0), r, r);  // its reciprocal, corrected twice
+    q = fma(fma(-s, q, 1.0), q, q);
+    return (float)(N * q);
+  }
+  const double ia = 1.0 / A, ib = 1.0 / B, iab = 1.0 / (A * b * b);
+  double d;
+  if (alg == 0) d = ib + ia + iab;
+  else if (alg == 1) d = ib + ia;
+  else d = ib + ia - iab;
+  return (float)(1.0 / sqrt(d));
+}
+
+}  // namespace tfcehip
