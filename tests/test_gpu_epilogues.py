@@ -1,0 +1,89 @@
+"""Every column shape of the contraction epilogues (fixed x permuted design
+columns, contrasts on permuted, fixed and constant columns, data with and
+without an intercept) against FP64 least squares, and the Sobel-type z at the
+values where its fast form gives way to the written-out one.
+
+Bars: the norm-wise 1e-5 of the split contraction (as tests/test_gpu_ols.py) for
+t; for z one rounding of the float result, 2^-23 relative.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def t64(X, Y, perm, cols, con):
+    Xp = X.copy()
+    Xp[:, cols] = X[perm][:, cols]
+    n, k = Xp.shape
+    inv = np.linalg.inv(Xp.T @ Xp)
+    a = inv @ Xp.T @ Y
+    s2 = ((Y - Xp @ a) ** 2).sum(0) / (n - k)
+    return np.stack([a[c] / np.sqrt(s2 * inv[c, c]) for c in con])
+
+
+@pytest.mark.parametrize("precision", ["fp16x3", "fp32"])
+@pytest.mark.parametrize("fixed", range(0, 7))
+def test_t_of_every_column_shape(fixed, precision):
+    import torch
+    from tfce_mediation_amd.ols import PermutedOLS
+    rng = np.random.default_rng(fixed)
+    n, V, P = 41, 197, 21
+    Y = (rng.standard_normal((n, V)) + 0.7).astype(np.float32)
+    perms = np.stack([rng.permutation(n) for _ in range(P)]).astype(np.int32)
+    for m in range(1, 8 - fixed):
+        k = 1 + fixed + m
+        X = np.column_stack([np.ones(n), rng.standard_normal((n, k - 1))]).astype(np.float32).astype(np.float64)
+        moved = list(range(1 + fixed, k))
+        con = [k - 1] if m % 2 else [k - 1, 1 + fixed] + ([1] if fixed else []) + [0]
+        model = PermutedOLS(torch.from_numpy(Y).cuda(), X, contrasts=con, perm_columns=moved, precision=precision)
+        t = model.t(torch.from_numpy(perms).cuda()).cpu().numpy().astype(np.float64)
+        ref = np.stack([t64(X, Y.astype(np.float64), p, moved, con) for p in perms], 1)
+        for c in range(len(con)):
+            assert np.linalg.norm(t[c] - ref[c]) <= 1e-5 * np.linalg.norm(ref[c]), (fixed, m, con[c])
+
+
+@pytest.mark.parametrize("k", [1, 3, 8])
+def test_t_without_intercept(k):
+    import torch
+    from tfce_mediation_amd.ols import PermutedOLS
+    rng = np.random.default_rng(k)
+    n, V, P = 36, 130, 9
+    X = rng.standard_normal((n, k)).astype(np.float32).astype(np.float64)
+    Y = rng.standard_normal((n, V)).astype(np.float32)
+    perms = np.stack([rng.permutation(n) for _ in range(P)]).astype(np.int32)
+    model = PermutedOLS(torch.from_numpy(Y).cuda(), X, contrasts=[0, k - 1], precision="fp32")
+    t = model.t(torch.from_numpy(perms).cuda()).cpu().numpy().astype(np.float64)
+    ref = np.stack([t64(X, Y.astype(np.float64), p, list(range(k)), [0, k - 1]) for p in perms], 1)
+    assert np.linalg.norm(t - ref) <= 1e-5 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("alg", [0, 1, 2])
+def test_sobel_z_special_values(alg):
+    import torch
+    from tfce_mediation_amd import _lib
+    v = np.array([0.0, -0.0, 1e-30, -3e-8, 0.5, -0.7, 1.0, 2.5, -40.0, 1e20, 3e38, np.inf, -np.inf, np.nan], np.float32)
+    a, b = (x.ravel() for x in np.meshgrid(v, v))
+    rng = np.random.default_rng(2)
+    a = np.concatenate([a, rng.standard_normal(5000).astype(np.float32) * 3])
+    b = np.concatenate([b, rng.standard_normal(5000).astype(np.float32) * 3])
+    z = torch.empty(a.size, dtype=torch.float32, device="cuda")
+    da, db = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    _lib.check(_lib.lib().tfce_sobel_z(_lib.ptr(da), _lib.ptr(db), a.size, alg, 0.0, _lib.ptr(z), _lib.stream_ptr()))
+    with np.errstate(all="ignore"):
+        A, B = a.astype(np.float64), b.astype(np.float64)
+        ia, ib, iab = 1 / (A * A), 1 / (B * B), 1 / (A * A * B * B)
+        ref = (1 / np.sqrt([ib + ia + iab, ib + ia, ib + ia - iab][alg]))
+    got = z.cpu().numpy()
+    # Goodman's difference cancels in the written-out form: only where its
+    # terms differ by more than its rounding does it say what z is
+    if alg == 2:
+        with np.errstate(all="ignore"):
+            clear = ~np.isfinite(ref) | (np.abs(ib + ia - iab) > 1e-6 * iab)
+        clear &= ~((A * A + B * B <= 1.0 + 1e-6) & np.isfinite(ref))
+        got, ref = got[clear], ref[clear]
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    with np.errstate(over="ignore"):
+        r32 = ref.astype(np.float32)
+    m = ~np.isnan(ref)
+    np.testing.assert_allclose(got[m], r32[m], rtol=2.0 ** -23, atol=0)

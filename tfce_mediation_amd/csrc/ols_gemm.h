@@ -86,35 +86,6 @@ __device__ __forceinline__ void f_epilogue(const OlsGemmArgs& a, int p, int64_t 
   a.t[(int64_t)p * a.ldt + col] = (float)(F < 0.0 ? 0.0 : sqrt(F));
 }
 
-// t of contrast column ci of a model with f fixed columns (FF > 0: a
-// compile-time f) and one permuted column whose X_p'y is gz0: the arithmetic
-// of epi_t for m = 1, operation for operation.
-template <int FF>
-__device__ __forceinline__ float single_t(int f_rt, int k, double inv_dof, const float* L, double dcv, int ci, int is_icpt,
-                                          int centered, const float* gF, const float* hF, double r0, double mu,
-                                          float gz0) {
-  const int f = FF > 0 ? FF : f_rt;
-  float s = 0.0f;
-#pragma unroll
-  for (int j = 0; j < kOlsMaxK; ++j)
-    if (j < f) s = fmaf(L[f * 8 + j], gF[j], s);
-  s = fmaf(L[f * 8 + f], gz0, s);
-  const double ssz = 0.0 + (double)s * (double)s;
-  double sse = r0 - ssz;
-  if (sse < 0.0) sse = 0.0;
-  float ac = 0.0f;
-#pragma unroll
-  for (int j = 0; j < kOlsMaxK; ++j) {
-    if (j >= ci && j < k) {
-      const float hj = (j < f) ? hF[j] : s;
-      ac = fmaf(L[j * 8 + ci], hj, ac);
-    }
-  }
-  const float se = sqrt_f32(sse * inv_dof * dcv);
-  if (centered && is_icpt) return (float)(((double)ac + mu) / (double)se);
-  return __fdiv_rn(ac, se);  // what the double quotient rounds to: its 53 bits hold a float quotient's tie
-}
-
 // Epilogue through LDS.  The accumulators of a wave cover, for tile (rt, ct),
 // rows row0 + 32 rt + 8 (i / 4) + 4 h + (i % 4) (i = accumulator index 0..15)
 // of column 32 ct + r.  The workgroup writes one 32-column slice of every
@@ -166,8 +137,8 @@ __device__ __forceinline__ void epi_loop_f(const OlsGemmArgs& a, const float* ep
 // permuted columns) the epilogue was 0.65 of the contraction's 2.1 ms with the
 // library's FP64 square root and two FP64 divisions per value; the square root
 // is sqrt_f32, the division by n - k a multiplication, and a / se the float
-// quotient.  Two permutations per iteration, so that their chains overlap (two
-// waves per SIMD).
+// quotient; several permutations per iteration, so that their chains overlap
+// (two waves per SIMD).  The contraction went from 2.09 to 1.70 ms.
 // kUniform: L and dc are read through the constant address space, so that a
 // wave-uniform address gives scalar loads also after the kernel's own stores
 // (vector loads of the factor took the registers from 100 to 240).
@@ -182,13 +153,19 @@ struct FactorPtr<true> {
   typedef const __attribute__((address_space(4))) double* D;
 };
 
-template <int LDC, int FC, int M>
+// PLAIN: centred data and contrasts on permuted columns only (every driver's
+// case), without a branch between the permutations of an iteration, which would
+// keep their chains apart.
+template <int LDC, int FC, int M, bool PLAIN>
 __device__ __forceinline__ void epi_t(const OlsGemmArgs& a, const float* ep, int cl, int64_t col, int p0, int ppt,
                                       int slot, int step, const float* gF, const float* hF, double r0, double mu,
                                       float yinv) {
-  constexpr int U = LDC >= 64 ? 2 : 1;
   constexpr bool kUniform = LDC >= 64;  // a wave's lanes share one permutation
+  constexpr int U = PLAIN && kUniform ? (M <= 2 ? 4 : 2) : 1;
   const int f = a.f;
+  float zi[M];  // powers of two: exact
+#pragma unroll
+  for (int q = 0; q < M; ++q) zi[q] = a.yinv ? a.zinv[q] : 1.0f;
   ppt = min(ppt, a.P - p0);
   for (int i0 = slot; i0 < ppt; i0 += U * step) {
     float hz[U][M];
@@ -198,14 +175,14 @@ __device__ __forceinline__ void epi_t(const OlsGemmArgs& a, const float* ep, int
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int i = min(i0 + u * step, ppt - 1);
-      fi[u] = a.shared_factor ? 0 : (kUniform ? __builtin_amdgcn_readfirstlane(p0 + i) : p0 + i);
+      const int p = kUniform ? __builtin_amdgcn_readfirstlane(p0 + i) : p0 + i;
+      fi[u] = a.shared_factor ? 0 : p;
       L[u] = (typename FactorPtr<kUniform>::F)(a.Linv + (int64_t)fi[u] * 64);
       float gz[M];
 #pragma unroll
       for (int q = 0; q < M; ++q) {
-        gz[q] = ep[(i * M + q) * LDC + cl];
-        if (a.yinv) gz[q] = gz[q] * a.zinv[q] * yinv;  // powers of two: exact
-        if (!a.centered) gz[q] += (float)(a.colsumZ[q] * mu);
+        gz[q] = ep[(i * M + q) * LDC + cl] * zi[q] * yinv;
+        if (!PLAIN && !a.centered) gz[q] += (float)(a.colsumZ[q] * mu);
       }
       double ssz = 0.0;
 #pragma unroll
@@ -219,15 +196,15 @@ __device__ __forceinline__ void epi_t(const OlsGemmArgs& a, const float* ep, int
         hz[u][r] = s;
         ssz = fma((double)s, (double)s, ssz);  // the product is exact
       }
-      const double sse = r0 - ssz;
-      x[u] = (sse < 0.0 ? 0.0 : sse) * a.inv_dof;
+      x[u] = (r0 - ssz) * a.inv_dof;  // below zero (rounding): sqrt_f32 takes it as zero
     }
     for (int c = 0; c < a.n_con; ++c) {
       const int ci = a.con[c];
+      float t[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         float ac = 0.0f;
-        if (ci < f) {
+        if (!PLAIN && ci < f) {
 #pragma unroll
           for (int j = 0; j < FC; ++j) ac = fmaf(L[u][j * 8 + ci], hF[j], ac);
         }
@@ -237,67 +214,130 @@ __device__ __forceinline__ void epi_t(const OlsGemmArgs& a, const float* ep, int
         const float se = sqrt_f32(x[u] * dc[c]);
         // a / se is what the double quotient rounds to (53 bits hold a float
         // quotient's tie)
-        const float t = (a.centered && a.con_is_intercept[c]) ? (float)(((double)ac + mu) / (double)se)
-                                                              : __fdiv_rn(ac, se);
-        if (i0 + u * step < ppt) a.t[((int64_t)c * a.P + p0 + i0 + u * step) * a.ldt + col] = t;
+        if (!PLAIN && a.centered && a.con_is_intercept[c]) t[u] = (float)(((double)ac + mu) / (double)se);
+        else t[u] = __fdiv_rn(ac, se);
       }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (i0 + u * step < ppt) a.t[((int64_t)c * a.P + p0 + i0 + u * step) * a.ldt + col] = t[u];
     }
   }
 }
 
-// epi_t for the model's column counts.
-template <int LDC, int FC>
+// epi_t for the model's column counts (f + m <= 8).
+template <int LDC, int FC, bool PLAIN>
 __device__ __forceinline__ void epi_t_cols(const OlsGemmArgs& a, const float* ep, int cl, int64_t col, int p0, int ppt,
                                            int slot, int step, const float* gF, const float* hF, double r0, double mu,
                                            float yinv) {
-  // (f + m <= 8)
+#define EPI_T(M) \
+  case M: epi_t<LDC, FC, M, PLAIN>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return
   switch (a.m) {
-    case 1: epi_t<LDC, FC, 1>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
-    case 2: epi_t<LDC, FC, 2>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
-    case 3: epi_t<LDC, FC, 3>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
+    EPI_T(1);
+    EPI_T(2);
+    EPI_T(3);
   }
   if constexpr (FC <= 4) {
     switch (a.m) {
-      case 4: epi_t<LDC, FC, 4>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
-      case 5: epi_t<LDC, FC, 5>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
+      EPI_T(4);
+      EPI_T(5);
     }
   }
   if constexpr (FC <= 2) {
     switch (a.m) {
-      case 6: epi_t<LDC, FC, 6>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
-      case 7: epi_t<LDC, FC, 7>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
-      case 8: epi_t<LDC, FC, 8>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv); return;
+      EPI_T(6);
+      EPI_T(7);
+      EPI_T(8);
     }
   }
+#undef EPI_T
 }
 
+// One model of a mediation: f fixed columns (at most FC; gF and hF hold zeros
+// beyond f), one permuted column, contrast column ci.
+template <int FC>
+struct MedModel {
+  float gF[FC], hF[FC];
+  double r0, mu, inv_dof;
+  int f, ci;
+  bool icpt;  // the contrast is the intercept of centred data: the mean comes back
+  __device__ __forceinline__ void load(const float* gFs, const float* hFs, const double* r0s, int64_t V, int64_t col) {
+#pragma unroll
+    for (int q = 0; q < FC; ++q) {
+      gF[q] = q < f ? gFs[(int64_t)q * V + col] : 0.0f;
+      hF[q] = q < f ? hFs[(int64_t)q * V + col] : 0.0f;
+    }
+    r0 = r0s[col];
+  }
+  // the arithmetic of epi_t for one permuted column
+  template <bool PLAIN, class F>
+  __device__ __forceinline__ float t(F L, double dcv, float gz) const {
+    const F row = L + f * 8;
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < FC; ++j) s = fmaf(row[j], gF[j], s);
+    s = fmaf(row[f], gz, s);
+    const double sse = fma(-(double)s, (double)s, r0);  // the product is exact
+    float ac = 0.0f;
+#pragma unroll
+    for (int j = 0; j < FC; ++j) ac = fmaf(L[j * 8 + ci], hF[j], ac);
+    ac = fmaf(row[ci], s, ac);
+    const float se = sqrt_f32(sse * inv_dof * dcv);
+    return !PLAIN && icpt ? (float)(((double)ac + mu) / (double)se) : __fdiv_rn(ac, se);
+  }
+};
+
 // The paired mediation epilogue: thread (cl, slot) walks its permutations,
-// computes t of both models from the one permuted column's X_p'y, and writes z.
-template <int LDC, int F1, int F2>
+// computes t of both models from the one permuted column's X_p'y, and writes z
+// (several permutations per iteration and PLAIN as in epi_t).
+template <int LDC, int F1, int F2, bool PLAIN>
 __device__ __forceinline__ void epi_loop_pair(const OlsGemmArgs& a, const float* ep, int cl, int64_t col, int p0,
                                               int ppt, int slot, int step, double mu, float yinv) {
-  float gF1[kOlsMaxK], hF1[kOlsMaxK], gF2[kOlsMaxK], hF2[kOlsMaxK];
+  constexpr bool kUniform = LDC >= 64;
+  constexpr int U = PLAIN && kUniform ? 4 : 1;
+  typedef typename FactorPtr<kUniform>::F FP;
+  typedef typename FactorPtr<kUniform>::D DP;
+  MedModel<F1> A;
+  MedModel<F2> B;
+  A.f = a.f;
+  A.ci = a.con[0];
+  A.icpt = a.centered && a.con_is_intercept[0];
+  A.mu = mu;
+  A.inv_dof = a.inv_dof;
+  A.load(a.gF, a.hF, a.r0, a.V, col);
+  B.f = a.f2;
+  B.ci = a.con2;
+  B.icpt = a.centered && a.con2_is_intercept;
+  B.mu = mu;
+  B.inv_dof = a.inv_dof2;
+  B.load(a.gF2, a.hF2, a.r02, a.V, col);
+  const float add = a.centered ? 0.0f : (float)(a.colsumZ[0] * mu), zi = a.yinv ? a.zinv[0] : 1.0f;
+  const double one = sobel_one(a.alg);
+  ppt = min(ppt, a.P - p0);
+  for (int i0 = slot; i0 < ppt; i0 += U * step) {
+    float ta[U], tb[U], z[U];
+    bool ok = true, fine[U];
 #pragma unroll
-  for (int q = 0; q < kOlsMaxK; ++q) {
-    gF1[q] = q < a.f ? a.gF[(int64_t)q * a.V + col] : 0.0f;
-    hF1[q] = q < a.f ? a.hF[(int64_t)q * a.V + col] : 0.0f;
-    gF2[q] = q < a.f2 ? a.gF2[(int64_t)q * a.V + col] : 0.0f;
-    hF2[q] = q < a.f2 ? a.hF2[(int64_t)q * a.V + col] : 0.0f;
-  }
-  const double r01 = a.r0[col], r02 = a.r02[col];
-  for (int pp = slot; pp < ppt; pp += step) {
-    const int p = p0 + pp;
-    if (p >= a.P) break;
-    float gz0 = ep[pp * LDC + cl];
-    if (a.yinv) gz0 = gz0 * a.zinv[0] * yinv;  // powers of two: exact
-    if (!a.centered) gz0 += (float)(a.colsumZ[0] * mu);
-    const int fi1 = a.shared_factor ? 0 : p, fi2 = a.shared2 ? 0 : p;
-    const float ta = single_t<F1>(a.f, a.k, a.inv_dof, a.Linv + (int64_t)fi1 * 64, a.dc[(int64_t)fi1 * kOlsMaxContrasts],
-                                  a.con[0], a.con_is_intercept[0], a.centered, gF1, hF1, r01, mu, gz0);
-    const float tb = single_t<F2>(a.f2, a.k2, a.inv_dof2, a.Linv2 + (int64_t)fi2 * 64,
-                                  a.dc2[(int64_t)fi2 * kOlsMaxContrasts], a.con2, a.con2_is_intercept, a.centered,
-                                  gF2, hF2, r02, mu, gz0);
-    a.t[(int64_t)p * a.ldt + col] = sobel_z((double)ta, (double)tb, a.alg);
+    for (int u = 0; u < U; ++u) {
+      const int i = min(i0 + u * step, ppt - 1);
+      const int p = kUniform ? __builtin_amdgcn_readfirstlane(p0 + i) : p0 + i;
+      float gz = ep[i * LDC + cl] * zi * yinv;  // powers of two: exact
+      if (!PLAIN && !a.centered) gz += add;
+      const int fi1 = a.shared_factor ? 0 : p, fi2 = a.shared2 ? 0 : p;
+      ta[u] = A.template t<PLAIN>((FP)(a.Linv + (int64_t)fi1 * 64),
+                                  ((DP)(a.dc + (int64_t)fi1 * kOlsMaxContrasts))[0], gz);
+      tb[u] = B.template t<PLAIN>((FP)(a.Linv2 + (int64_t)fi2 * 64),
+                                  ((DP)(a.dc2 + (int64_t)fi2 * kOlsMaxContrasts))[0], gz);
+      fine[u] = sobel_z_fast((double)ta[u], (double)tb[u], one, z[u]);
+      ok = ok && fine[u];
+    }
+    if (!ok) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (!fine[u]) z[u] = sobel_z_general((double)ta[u], (double)tb[u], a.alg);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i0 + u * step < ppt) a.t[(int64_t)(p0 + i0 + u * step) * a.ldt + col] = z[u];
   }
 }
 
@@ -312,8 +352,11 @@ __device__ __forceinline__ void epi_run(const OlsGemmArgs& a, const float* ep, i
   const int p0 = (int)(mrow0 / rows) * ppt;
   if constexpr (EPI == kEpiPair) {
     // mediation types M and I: path A [1, x], path B [1, y, x]
-    if (a.f == 1 && a.f2 == 2) epi_loop_pair<LDC, 1, 2>(a, ep, cl, col, p0, ppt, slot, step, mu, yinv);
-    else epi_loop_pair<LDC, 0, 0>(a, ep, cl, col, p0, ppt, slot, step, mu, yinv);
+    const bool plain = a.centered && !a.con_is_intercept[0] && !a.con2_is_intercept;
+    if (plain && a.f <= 1 && a.f2 <= 2)
+      epi_loop_pair<LDC, 1, 2, true>(a, ep, cl, col, p0, ppt, slot, step, mu, yinv);
+    else
+      epi_loop_pair<LDC, 7, 7, false>(a, ep, cl, col, p0, ppt, slot, step, mu, yinv);
     return;
   }
   float gF[kOlsMaxK], hF[kOlsMaxK];
@@ -323,10 +366,13 @@ __device__ __forceinline__ void epi_run(const OlsGemmArgs& a, const float* ep, i
     hF[q] = q < a.f ? a.hF[(int64_t)q * a.V + col] : 0.0f;
   }
   const double r0 = a.r0[col];
-  if constexpr (EPI == kEpiT1) epi_t_cols<LDC, 1>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv);
-  if constexpr (EPI == kEpiT2) epi_t_cols<LDC, 2>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv);
-  if constexpr (EPI == kEpiT4) epi_t_cols<LDC, 4>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv);
-  if constexpr (EPI == kEpiT7) epi_t_cols<LDC, 7>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv);
+  if constexpr (EPI <= kEpiT7) {
+    constexpr int FC = EPI == kEpiT1 ? 1 : (EPI == kEpiT2 ? 2 : (EPI == kEpiT4 ? 4 : 7));
+    bool plain = a.centered;
+    for (int c = 0; c < a.n_con; ++c) plain = plain && a.con[c] >= a.f && !a.con_is_intercept[c];
+    if (plain) epi_t_cols<LDC, FC, true>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv);
+    else epi_t_cols<LDC, FC, false>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv);
+  }
   if constexpr (EPI == kEpiF) epi_loop_f<LDC, false>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv);
   if constexpr (EPI == kEpiBlk) epi_loop_f<LDC, true>(a, ep, cl, col, p0, ppt, slot, step, gF, hF, r0, mu, yinv);
 }
@@ -345,7 +391,8 @@ __device__ __forceinline__ bool gemm_tile(const OlsGemmArgs& a, int& mt, int& nt
 // 128 columns and reads its fragments straight from global memory.
 template <EpiKind EPI>
 __global__ __launch_bounds__(256) void ols_gemm_fp32_kernel(OlsGemmArgs a) {
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, h = l >> 5, r = l & 31;
+  const int tid = threadIdx.x, l = tid & 63, h = l >> 5, r = l & 31;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   int mt, nt;
   if (!gemm_tile(a, mt, nt)) return;
   const int64_t m0 = (int64_t)mt * kGemmRows + w * 64;
@@ -383,14 +430,15 @@ __global__ __launch_bounds__(256) void ols_gemm_fp32_kernel(OlsGemmArgs a) {
         for (int ct = 0; ct < 4; ++ct)
           acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x2f32(A[rt][jj], B[ct][jj], acc[rt][ct], 0, 0, 0);
   }
-  // epilogue: four passes of 32 columns through a [256][32] LDS block
-  __shared__ float ep[kGemmRows * 32];
+  // epilogue: two passes of 64 columns through a [256][64] LDS block
+  __shared__ float ep[kGemmRows * 64];
 #pragma unroll
-  for (int pass = 0; pass < 4; ++pass) {
+  for (int pass = 0; pass < 2; ++pass) {
     __syncthreads();
-    epi_put<2, 4>(ep, 32, acc, pass, w * 64, 0, h, r);
+    epi_put<2, 4>(ep, 64, acc, 2 * pass, w * 64, 0, h, r);
+    epi_put<2, 4>(ep, 64, acc, 2 * pass + 1, w * 64, 32, h, r);
     __syncthreads();
-    epi_run<32, EPI>(a, ep, tid & 31, n0 + 32 * pass + (tid & 31), (int64_t)mt * kGemmRows, kGemmRows, tid >> 5, 8);
+    epi_run<64, EPI>(a, ep, l, n0 + 64 * pass + l, (int64_t)mt * kGemmRows, kGemmRows, w, 4);
   }
 }
 
