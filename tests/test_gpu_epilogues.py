@@ -87,3 +87,23 @@ def test_sobel_z_special_values(alg):
         r32 = ref.astype(np.float32)
     m = ~np.isnan(ref)
     np.testing.assert_allclose(got[m], r32[m], rtol=2.0 ** -23, atol=0)
+
+
+@pytest.mark.parametrize("n,k,V", [(3, 2, 1), (15, 3, 64), (16, 1, 65), (17, 4, 63), (32, 5, 200), (33, 6, 129),
+                                   (100, 7, 1), (2047, 8, 70), (2048, 2, 128)])
+def test_single_design_in_fp64(n, k, V):
+    """Every column count; row counts around the 16 rows in flight.  Bars: 1e-10
+    norm-wise for FP64 sums of up to 2048 terms under a conditioning below 1e4."""
+    from oracle import ols
+    from tfce_mediation_amd.cynumstats import _direct
+    rng = np.random.default_rng(n)
+    X = np.column_stack([np.ones(n), np.linspace(-1, 1, n)[:, None] ** np.arange(1, 2) if k > 1 else np.empty((n, 0)),
+                         rng.standard_normal((n, max(k - 2, 0)))])
+    Y = rng.standard_normal((n, V)).astype(np.float32)
+    got = _direct(X, Y, coef=True, resid=True, sse=True, sums=True)
+    y = Y.astype(np.float64)
+    coef = ols.cy_lin_lstsqr_mat(X, y)
+    res = y - X @ coef
+    for name, ref in (("coef", coef), ("resid", res), ("sse", (res ** 2).sum(0)), ("sumyy", (y ** 2).sum(0))):
+        assert np.linalg.norm(got[name] - ref) <= 1e-10 * np.linalg.norm(ref), name
+    assert np.abs(got["sumy"] - y.sum(0)).max() <= 1e-10 * np.abs(y).sum(0).max()

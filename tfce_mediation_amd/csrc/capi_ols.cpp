@@ -655,13 +655,15 @@ int tfce_ols_direct(const float* d_Y, int32_t n, int64_t V, int64_t ldy, const d
       for (int q = std::max(a, b); q < k; ++q) s += Li[q * k + a] * Li[q * k + b];
       Ainv[a * k + b] = s;
     }
-  double *dX = nullptr, *dA = nullptr, *dS = nullptr;
-  int rc = 0;
-  if ((rc = dalloc(&dX, (size_t)n * k, "X")) || (rc = dalloc(&dA, (size_t)k * k, "Ainv")) ||
-      (rc = dalloc(&dS, (size_t)k * k, "Sinv")) || (rc = upload(dX, X, (size_t)n * k, "X")) ||
-      (rc = upload(dA, Ainv.data(), (size_t)k * k, "Ainv")) ||
-      (rc = upload(dS, invXX_se ? invXX_se : Ainv.data(), (size_t)k * k, "Sinv"))) {
-    for (void* p : {(void*)dX, (void*)dA, (void*)dS}) if (p) (void)hipFree(p);
+  // design, both inverses: one allocation and one copy
+  std::vector<double> host(X, X + (size_t)n * k);
+  host.insert(host.end(), Ainv.begin(), Ainv.end());
+  host.insert(host.end(), invXX_se ? invXX_se : Ainv.data(), (invXX_se ? invXX_se : Ainv.data()) + k * k);
+  double* dX = nullptr;
+  int rc = dalloc(&dX, host.size(), "X, Ainv, Sinv");
+  if (!rc) rc = upload(dX, host.data(), host.size(), "X, Ainv, Sinv");
+  if (rc) {
+    if (dX) (void)hipFree(dX);
     return rc;
   }
   OlsDirectArgs a{};
@@ -671,8 +673,8 @@ int tfce_ols_direct(const float* d_Y, int32_t n, int64_t V, int64_t ldy, const d
   a.V = V;
   a.ldy = ldy;
   a.X = dX;
-  a.Ainv = dA;
-  a.Sinv = dS;
+  a.Ainv = dX + (size_t)n * k;
+  a.Sinv = a.Ainv + k * k;
   a.coef = d_coef;
   a.se = d_se;
   a.t = d_t;
@@ -682,7 +684,7 @@ int tfce_ols_direct(const float* d_Y, int32_t n, int64_t V, int64_t ldy, const d
   a.sumyy = d_sumyy;
   hipError_t e = launch_ols_direct(a, stream);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
-  for (void* p : {(void*)dX, (void*)dA, (void*)dS}) (void)hipFree(p);
+  (void)hipFree(dX);
   if (e != hipSuccess) return set_error(-(int)e, "ols direct kernel");
   return 0;
 }
