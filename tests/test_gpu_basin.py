@@ -239,3 +239,33 @@ def test_weighted_maxima(gname):
             if x.max() > 0:
                 enh, _, _ = otfce.tfce(rp, col, x, 2.0, 1.0, exact_pow=True)
             assert out[p, k] == ((enh * np.float32(x.max() / np.float32(100))) * vd).max()
+
+
+def band(n, offsets):
+    """Elements v and v +- o joined for every offset o (no wrap-around)."""
+    i = np.arange(n)
+    nb = np.concatenate([i[:, None] + np.array([*offsets, *(-np.array(offsets))]), np.full((n, 1), -1)], 1)
+    ok = (nb >= 0) & (nb < n)
+    return (np.concatenate([[0], np.cumsum(ok.sum(1))]).astype(np.int32), nb[ok].astype(np.int32))
+
+
+# wide lists in tiles: every number of entries (18, 26, 32), neighbours as 16-bit
+# differences and as indices, values from LDS (up to 15,000 elements off in
+# launches of large workgroups) and from memory
+@pytest.mark.parametrize("P", [2, 150])
+@pytest.mark.parametrize("near,far", [(8, 40), (8, 15000), (9, 5000), (12, 15001), (12, 32767), (12, 15000), (15, 300),
+                                      (15, 32768), (8, 33000)])
+def test_wide_lists(near, far, P):
+    import torch
+    from tfce_mediation_amd.tfce import Adjacency, SurfaceSet
+    csr = band(far + 2500, [*range(1, near + 1), far])
+    V = len(csr[0]) - 1
+    say(f"[gpu] basin sweep, wide lists {2 * near + 2} entries, {far} off, V={V} P={P}")
+    maps = np.random.default_rng(near + far).standard_normal((P, V)).astype(np.float32)
+    maps[1] = np.round(2 * maps[1]) / 2
+    out = SurfaceSet([Adjacency(csr, 2.0, 1.0)], [0]).batch(torch.from_numpy(maps).cuda(), 3).cpu().numpy()[0]
+    for p in (0, 1, P - 1):
+        for k, sgn in enumerate((1, -1)):
+            x = (np.float32(sgn) * maps[p]).astype(np.float32)
+            enh, _, _ = otfce.tfce(*csr, x, 2.0, 1.0, exact_pow=True)
+            assert out[p, k] == np.float32(enh.max() * np.float32(x.max() / np.float32(100))), (p, k)

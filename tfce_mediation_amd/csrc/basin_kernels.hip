@@ -58,6 +58,10 @@ constexpr uint16_t kInactive = 0xffff;
 // with four of 512.
 constexpr int kBasinTiny = 1696, kBasinSmall = 3400, kBasinMid = 6800, kBasinMax12 = 13600;
 
+// A pointer read from a descriptor, known to be global memory.
+template <class T>
+using Global = const __attribute__((address_space(1))) T*;
+
 // Local unit of a workgroup of the vertex passes.  Consecutive workgroups go
 // round the eight XCDs; the workgroups of one map stay on one XCD, so its L2
 // holds the map and its pointers while they are gathered from.
@@ -66,23 +70,25 @@ struct BlockRef {
 };
 template <int Q>
 __device__ __forceinline__ BlockRef decode_block(const BasinArgs& a, int s0, int s1) {
-  const int64_t first = (int64_t)a.surfs[s0].basin.blk0 * Q;
-  int64_t b = (int64_t)blockIdx.x + first * a.pc;
+  // (a grid is below 2^31 workgroups, so 32 bits hold all of this)
+  const unsigned first = (unsigned)a.surfs[s0].basin.blk0, pc = (unsigned)a.pc;
+  unsigned b = blockIdx.x;
   int s = s0;
-  while (s + 1 < s1 && b >= (int64_t)a.surfs[s + 1].basin.blk0 * Q * a.pc) ++s;
-  b -= (int64_t)a.surfs[s].basin.blk0 * Q * a.pc;
-  const int nb = a.surfs[s].basin.nblk * Q;
-  const int64_t whole = (int64_t)(a.pc / 8) * 8 * nb;
+  while (s + 1 < s1 && b >= ((unsigned)a.surfs[s + 1].basin.blk0 - first) * Q * pc) ++s;
+  b -= ((unsigned)a.surfs[s].basin.blk0 - first) * Q * pc;
+  const unsigned nb = (unsigned)a.surfs[s].basin.nblk * Q;
+  const unsigned whole = pc / 8 * 8 * nb;
   BlockRef r;
   r.s = s;
   if (b < whole) {
-    r.lp = (int)(b / (8 * nb)) * 8 + (int)(b & 7);
-    r.j = (int)((b % (8 * nb)) >> 3);
+    const unsigned eight = b / (8 * nb);
+    r.lp = (int)(eight * 8 + (b & 7));
+    r.j = (int)((b - eight * 8 * nb) >> 3);
   } else {
-    const int rest = a.pc & 7;
+    const unsigned rest = pc & 7;
     b -= whole;
-    r.lp = (a.pc & ~7) + (int)(b % rest);
     r.j = (int)(b / rest);
+    r.lp = (int)((pc & ~7u) + (b - (unsigned)r.j * rest));
   }
   return r;
 }
@@ -255,7 +261,7 @@ __device__ __forceinline__ int32_t* block_counts(const BasinArgs& a, const SurfD
   return a.blk + (((int64_t)lp * a.blk_total + S.basin.blk0 - a.blk_first) * Q + j) * 4;
 }
 
-template <int Q>
+template <int Q, int T = kThreads>
 __device__ __forceinline__ void assign_begin(const BasinArgs& a, const SurfDev& S, const BlockRef& br, Assign& w,
                                              AssignShared<Q>& sh) {
   const int tid = threadIdx.x;
@@ -277,10 +283,10 @@ __device__ __forceinline__ void assign_begin(const BasinArgs& a, const SurfDev& 
     w.L[g] = (l > 0 && l <= kBasinLevels) ? l : 0;
     w.T0[g] = __int_as_float(rec[kPrepT0]);
     w.inv[g] = 1.0f / __int_as_float(rec[kPrepDT]);
-    for (int i = tid; i < w.L[g]; i += kThreads) sh.T[g][i] = __int_as_float(rec[kPrepT + i]);
+    for (int i = tid; i < w.L[g]; i += T) sh.T[g][i] = __int_as_float(rec[kPrepT + i]);
     if (w.L[g] > 0) w.last[g] = __int_as_float(rec[kPrepT + w.L[g] - 1]);
   }
-  for (int i = tid; i < 2 * kBasinLevels; i += kThreads) sh.hist[i] = sh.pairs[i] = 0;
+  for (int i = tid; i < 2 * kBasinLevels; i += T) sh.hist[i] = sh.pairs[i] = 0;
   if (tid < 2) sh.nmax[tid] = 0;
   if (tid == 2) sh.npairs = 0;
   const int64_t e0 = (int64_t)br.lp * a.elt_total + S.basin.elt0;
@@ -325,24 +331,49 @@ __device__ __forceinline__ void put_pair(const Assign& w, int at, int lev, int u
 // Pointers and counts out.  Pointers are followed as far as they stay in the
 // workgroup's elements: one that ends at a maximum here becomes that maximum's
 // number.
-template <int Q>
+template <int Q, int T = kThreads>
 __device__ __forceinline__ void assign_end(const BasinArgs& a, const SurfDev& S, const Assign& w,
                                            AssignShared<Q>& sh) {
   const int tid = threadIdx.x;
   __syncthreads();
   const int here = min(kBlockOf<Q>, w.V - w.vb0);
-  for (int i = tid; i < here; i += kThreads) {
+  for (int i = tid; i < here; i += T) {
     int p = sh.word[i];
     if (p == kNever) continue;
     while (p >= w.vb0 && p < w.vb0 + kBlockOf<Q>) p = sh.word[p - w.vb0];
     w.word[w.vb0 + i] = p;
   }
   int32_t* unit = a.unit + unit_of(a, w.br.s, w.br.lp) * kBasinUnitWords;
-  for (int i = tid; i < 2 * kBasinLevels; i += kThreads) {
+  for (int i = tid; i < 2 * kBasinLevels; i += T) {
     if (sh.hist[i]) atomicAdd(&unit[kBasinCur + i], sh.hist[i]);
     if (sh.pairs[i]) atomicAdd(&unit[kBasinEvCur + i], sh.pairs[i]);
   }
   if (tid < 3) block_counts<Q>(a, S, w.br.lp, w.br.j)[tid] = tid < 2 ? sh.nmax[tid] : sh.npairs;
+}
+
+typedef int Row __attribute__((ext_vector_type(4)));
+
+// The entries of a ring-packed row of element v; those past its end repeat the
+// first one (an empty row: the element).
+__device__ __forceinline__ void assign_ring_row(Row row, int v, int (&u)[kRingMaxDeg], unsigned& tail) {
+  ring_fields(make_int4(row.x, row.y, row.z, row.w), u, tail);
+  const int deg = (int)(tail >> 6);
+  if (__any(deg < kRingMaxDeg)) {
+    if (deg == 0) u[0] = v;
+#pragma unroll
+    for (int j = 1; j < kRingMaxDeg; ++j) u[j] = j < deg ? u[j] : u[0];
+  }
+}
+
+// Entry j of a ring-packed row: 18 bits from bit 18 j.
+__device__ __forceinline__ int ring_entry(Row row, int j) {
+  const int k = j >> 1;
+  int lo = row.x, hi = row.y;
+  lo = k == 1 ? row.y : lo;
+  hi = k == 1 ? row.z : hi;
+  lo = k == 2 ? row.z : lo;
+  hi = k == 2 ? row.w : hi;
+  return (int)(__builtin_amdgcn_alignbit((unsigned)hi, (unsigned)lo, 18 * (j & 1) + 4 * k) & (unsigned)kRingNone);
 }
 
 // Vertex pass 1 over ring-packed surfaces [s0, s1): four elements' rows and
@@ -355,64 +386,71 @@ __global__ __launch_bounds__(kThreads) void basin_assign_ring_kernel(BasinArgs a
   const SurfDev S = a.surfs[br.s];
   Assign w;
   assign_begin(a, S, br, w, sh);
-  const float* x = w.x;
   const int V = w.V;
-  const int4* tab = reinterpret_cast<const int4*>(S.nadj);
+  const char* xb = reinterpret_cast<const char*>(w.x);
+  const Global<Row> tab = (Global<Row>)S.nadj;
   for (int r = 0; r < kBlockOf<Q> / kThreads / kRound; ++r) {
     const int vb = w.vb0 + r * kRound * kThreads + tid;
     if (vb - tid >= V) break;
     float key[kRound];
     int g[kRound];
-    int4 row[kRound];
+    Row row[kRound];
     bool act[kRound];
 #pragma unroll
     for (int t = 0; t < kRound; ++t) {
-      const int v = vb + t * kThreads;
-      key[t] = v < V ? x[v] : __int_as_float(0x7fc00000);
-    }
-#pragma unroll
-    for (int t = 0; t < kRound; ++t) {
-      act[t] = assign_active(w, key[t], g[t], key[t]);
-      row[t] = act[t] ? tab[vb + t * kThreads] : make_int4(-1, -1, -1, -1);
+      const int v = min(vb + t * kThreads, V - 1);
+      key[t] = w.x[v];
+      row[t] = tab[v];
     }
     float nk[kRound][kRingMaxDeg];
 #pragma unroll
     for (int t = 0; t < kRound; ++t) {
+      const int v = vb + t * kThreads;
+      act[t] = assign_active(w, key[t], g[t], key[t]) && v < V;
       int u[kRingMaxDeg];
       unsigned tail;
-      ring_fields(row[t], u, tail);
+      assign_ring_row(row[t], min(v, V - 1), u, tail);
 #pragma unroll
-      for (int j = 0; j < kRingMaxDeg; ++j) nk[t][j] = u[j] != kRingNone ? x[u[j]] : __int_as_float(0x7fc00000);
+      for (int j = 0; j < kRingMaxDeg; ++j)
+        nk[t][j] = *reinterpret_cast<const float*>(xb + (unsigned)u[j] * 4u);
     }
 #pragma unroll
     for (int t = 0; t < kRound; ++t) {
       const int v = vb + t * kThreads;
-      int u[kRingMaxDeg];
-      unsigned tail;
-      ring_fields(row[t], u, tail);
+      const unsigned tail = ((unsigned)row[t].w >> 12) & 0x1ffu;
+      const int deg = (int)(tail >> 6);
       const float s = g[t] ? -1.0f : w.sgn[0];
-      // the earlier neighbours, the largest of them; equal values (index
-      // order) only where the wave meets any
-      unsigned up = 0;
-      bool tie = false;
-      float bk = key[t];
-      int best = v;
+      // the earlier neighbours by the signs of the differences and one of the
+      // largest (see basin_assign_wide_kernel); equal values (index order) and
+      // NaN only where the wave meets any
+      unsigned up = 0, far = 0;
+      bool odd = false;
 #pragma unroll
-      for (int j = 0; j < kRingMaxDeg; ++j) {
-        const float k = s * nk[t][j];
-        up |= k > key[t] ? 1u << j : 0u;
-        tie |= k == key[t];
-        best = k > bk ? u[j] : best;
-        bk = fmaxf(bk, k);
+      for (int j = kRingMaxDeg - 1; j >= 0; --j) {
+        const float d = fmaf(-s, nk[t][j], key[t]);
+        const unsigned bits = __float_as_uint(d);
+        up = __builtin_amdgcn_alignbit(up, bits, 31);
+        far = max(far, (bits & ~7u) | (unsigned)j);
+        odd |= !(d < 0.0f || d > 0.0f);
       }
-      if (__any(tie)) {
-#pragma unroll
-        for (int j = 0; j < kRingMaxDeg; ++j)
-          if (s * nk[t][j] == key[t] && u[j] < v) {
-            up |= 1u << j;
-            if (best == v) best = u[j];
+      if (__any(act[t] && odd)) {
+        up = 0;
+        far = 0;
+        float bk = -INFINITY;
+        for (int j = 0; j < deg; ++j) {
+          const int u = ring_entry(row[t], j);
+          const float k = s * w.x[u];
+          if (!(k > key[t] || (k == key[t] && u < v))) continue;
+          up |= 1u << j;
+          if (up == 1u << j || k > bk) {
+            far = (unsigned)j;
+            bk = k;
           }
+        }
       }
+      up = act[t] ? up & ((1u << deg) - 1u) : 0u;
+      const int bj = (int)(far & 7u);
+      const int best = ring_entry(row[t], bj < deg ? bj : 0);
       const int lev = act[t] ? assign_level(w, sh, g[t], key[t]) : kInactive;
       // local maxima numbered within the workgroup, per sign
       int32_t p = best;
@@ -424,13 +462,10 @@ __global__ __launch_bounds__(kThreads) void basin_assign_ring_kernel(BasinArgs a
       const int more = __popc(arcs) - 1;
       if (more > 0) {
         int at = assign_pairs(sh, lev, more);
-        int first = -1;
-#pragma unroll
-        for (int j = 0; j < kRingMaxDeg; ++j) {
-          if (!((arcs >> j) & 1u)) continue;
-          if (first < 0) first = u[j];
-          else put_pair(w, at++, lev, first, u[j]);
-        }
+        const int first = ring_entry(row[t], __ffs((int)arcs) - 1);
+#pragma unroll 1
+        for (unsigned rest = arcs & (arcs - 1u); rest; rest &= rest - 1u)
+          put_pair(w, at++, lev, first, ring_entry(row[t], __ffs((int)rest) - 1));
       }
     }
   }
@@ -460,11 +495,8 @@ __device__ __forceinline__ unsigned row_arcs(unsigned up, unsigned seed, unsigne
 }
 
 // Vertex pass 1 over surfaces with a fixed-width table of W entries per row.
-// W = 32 (26-connected volumes): groups of earlier neighbours by the full row
-// adjacency, whose masks come through the scalar cache where a whole wave has
-// the same masks (the interior of a volume); narrower tables by the adjacency
-// bytes within each eight entries (a group seen as two only adds a pair that
-// basin_resolve drops).
+// Groups of earlier neighbours by the adjacency bytes within each eight entries
+// (a group seen as two only adds a pair that basin_resolve drops).
 template <int W, int Q>
 __global__ __launch_bounds__(kThreads) void basin_assign_table_kernel(BasinArgs a, int s0, int s1) {
   __shared__ AssignShared<Q> sh;
@@ -530,30 +562,7 @@ __global__ __launch_bounds__(kThreads) void basin_assign_table_kernel(BasinArgs 
     // the groups of the earlier neighbours (one neighbour is one group)
     const bool many = (up & (up - 1u)) != 0u;
     unsigned arcs = 0u;
-    if (W == kEllMaxWidth && S.adjw) {
-      const int id = many ? (S.adjid ? (int)S.adjid[v] : v) : -1;
-      const unsigned long long who = __ballot(many);
-      if (who != 0ull) {
-        const int id0 = __builtin_amdgcn_readlane(id, __ffsll((long long)who) - 1);
-        const unsigned near = many ? S.adjw[(size_t)id * W + bj] : 0u;
-        if (__ballot(id == id0) == who) {
-          const uint32_t* m = S.adjw + (size_t)id0 * W;  // uniform: scalar loads
-          if (many) arcs = row_arcs<W>(up, 1u << bj, near, [&](int j) { return m[j]; });
-        } else if (many) {
-          unsigned m[W];
-          const uint4* mr = reinterpret_cast<const uint4*>(S.adjw + (size_t)id * W);
-#pragma unroll
-          for (int c = 0; c < W / 4; ++c) {
-            const uint4 q = mr[c];
-            m[4 * c] = q.x;
-            m[4 * c + 1] = q.y;
-            m[4 * c + 2] = q.z;
-            m[4 * c + 3] = q.w;
-          }
-          arcs = row_arcs<W>(up, 1u << bj, near, [&](int j) { return m[j]; });
-        }
-      }
-    } else if (many) {
+    if (many) {
       unsigned m[W];
       if (S.nadj) {
         const uint32_t* mr = reinterpret_cast<const uint32_t*>(S.nadj + (size_t)v * W);
@@ -577,6 +586,139 @@ __global__ __launch_bounds__(kThreads) void basin_assign_table_kernel(BasinArgs 
     }
   }
   assign_end(a, S, w, sh);
+}
+
+// Vertex pass 1 over surfaces with lists of up to NE entries in tiles of 64
+// elements (SurfDev.tile; 18- and 26-connected volumes, others of 17 to 32
+// neighbours).  Bound by the vector cache's lines: from rows of 32 entries a
+// wave's list took 512 of them and the masks of the grouping another 512, from
+// tiles 28 and one per step.  The groups of an element's earlier neighbours
+// grow from one of them, one mask per step, until they hold all: elements other
+// than saddles are done after the few masks that cover them.
+// 232k 26-connected voxels, 512 maps, both signs: 4.4 ms from rows; 2.6 from
+// tiles, of which a third went to gathering the values through the same cache,
+// so the workgroup keeps the map around its elements in LDS where that fits
+// (NEAR: every neighbour within kNearReach, launches of the larger workgroups,
+// two workgroups of 1,024 threads per compute unit up to 5,600): 2.1.  Small
+// workgroups would load ten times the map for it.
+template <bool NEAR>
+constexpr int kWideThreads = NEAR ? 1024 : kThreads;
+
+template <int NE, bool D16, int Q, bool NEAR>
+__global__ __launch_bounds__(kWideThreads<NEAR>) void basin_assign_wide_kernel(BasinArgs a, int s0, int s1) {
+  constexpr int T = kWideThreads<NEAR>;
+  extern __shared__ float s_near[];
+  __shared__ AssignShared<Q> sh;
+  const int tid = threadIdx.x;
+  const BlockRef br = decode_block<Q>(a, s0, s1);
+  const SurfDev S = a.surfs[br.s];
+  Assign w;
+  assign_begin<Q, T>(a, S, br, w, sh);
+  const int V = w.V;
+  constexpr int kWords = tile_words(NE, D16);
+  // byte offsets in 32 bits (V < 2^24) from a uniform address
+  const char* xb = reinterpret_cast<const char*>(w.x);
+  const Global<uint32_t> tile = (Global<uint32_t>)S.tile, adjw = (Global<uint32_t>)S.adjw;
+  const bool shared_rows = S.adjid != nullptr;
+  const int near0 = w.vb0 - S.reach;
+  if (NEAR) {
+    const int n = kBlockOf<Q> + 2 * S.reach;
+    for (int i = tid; i < n; i += T) s_near[i] = w.x[min(max(near0 + i, 0), V - 1)];
+    __syncthreads();
+  }
+  for (int r = 0; r < kBlockOf<Q> / T; ++r) {
+    const int v = w.vb0 + r * T + tid;
+    if (v - tid >= V) break;
+    const Global<uint32_t> tw = tile + (size_t)((unsigned)(v - tid) >> 6) * kWords * 64;
+    const unsigned lane0 = (unsigned)(tid >> 6) * kWords * 64 + (tid & 63);
+    float key = NEAR ? s_near[v - near0] : w.x[min(v, V - 1)];
+    uint32_t q[kWords];
+#pragma unroll
+    for (int i = 0; i < kWords; ++i) q[i] = tw[lane0 + i * 64];
+    int g;
+    bool act = assign_active(w, key, g, key);
+    act = act && v < V;
+    const float s = g ? -1.0f : w.sgn[0];
+    float nk[NE];
+#pragma unroll
+    for (int j = 0; j < NE; ++j) {
+      const int to = D16 ? ((j & 1) ? (int)q[j / 2] >> 16 : (int)(int16_t)q[j / 2]) : (int)q[j];
+      nk[j] = NEAR ? (s_near + (v - near0))[to]
+                   : *reinterpret_cast<const float*>(xb + (unsigned)(D16 ? v + to : to) * 4u);
+    }
+    // The earlier neighbours (bit j: entry j) by the signs of the differences
+    // (s * nk is exact, and a difference is zero only of equal values), one of
+    // the largest differences with its entry in the low bits.  Pointing at any
+    // earlier neighbour is right; a large one keeps the ways to the maxima
+    // short.  Equal values (index order) and NaN only where the wave meets any.
+    unsigned up = 0, far = 0;
+    bool odd = false;
+#pragma unroll
+    for (int j = NE - 1; j >= 0; --j) {
+      const float d = fmaf(-s, nk[j], key);
+      const unsigned bits = __float_as_uint(d);
+      up = __builtin_amdgcn_alignbit(up, bits, 31);
+      far = max(far, (bits & ~31u) | (unsigned)j);
+      odd |= !(d < 0.0f || d > 0.0f);
+    }
+    const int deg = (int)(q[kWords - 1] & 0xffffu);
+    const unsigned listed = deg < 32 ? (1u << deg) - 1u : ~0u;
+    const auto entry = [&](int j) {
+      return D16 ? v + (int)((Global<int16_t>)tw)[(lane0 + (j >> 1) * 64) * 2 + (j & 1)] : (int)tw[lane0 + j * 64];
+    };
+    if (__any(act && odd)) {
+      up = 0;
+      far = 0;
+      float bk = -INFINITY;
+      for (int j = 0; j < deg; ++j) {
+        const int u = entry(j);
+        const float k = s * w.x[u];
+        if (!(k > key || (k == key && u < v))) continue;
+        up |= 1u << j;
+        if (up == 1u << j || k > bk) {
+          far = (unsigned)j;
+          bk = k;
+        }
+      }
+    }
+    up &= listed;
+    // an entry past the list repeats entry 0
+    const int bj = (int)(far & 31u);
+    int best = 0;
+    if (act && up != 0u) best = entry(bj < deg ? bj : 0);
+    const int lev = act ? assign_level(w, sh, g, key) : kInactive;
+    int32_t p = kNever;
+    if (act) p = up == 0u ? ~atomicAdd(&sh.nmax[g], 1) : best;
+    if (v < V) w.code[v] = (uint16_t)lev;
+    sh.word[v - w.vb0] = p;
+    if (!act || (up & (up - 1u)) == 0u) continue;
+    unsigned arcs = up;
+    if (adjw) {
+      const Global<uint32_t> m = adjw + (size_t)(shared_rows ? q[kWords - 1] >> 16 : (unsigned)v) * kEllMaxWidth;
+      unsigned in = up & (0u - up), todo = in;
+      arcs = in;
+      while (in != up) {
+        if (todo == 0u) {  // the groups reached are complete: the next one
+          const unsigned rem = up & ~in;
+          todo = rem & (0u - rem);
+          arcs |= todo;
+          in |= todo;
+          continue;
+        }
+        const unsigned grown = up & ~in & m[__ffs((int)todo) - 1];
+        todo = (todo & (todo - 1u)) | grown;
+        in |= grown;
+      }
+    }
+    const int more = __popc(arcs) - 1;
+    if (more > 0) {
+      int slot = assign_pairs(sh, lev, more);
+      const int first = entry(__ffs((int)arcs) - 1);
+      for (unsigned rest = arcs & (arcs - 1u); rest; rest &= rest - 1u)
+        put_pair(w, slot++, lev, first, entry(__ffs((int)rest) - 1));
+    }
+  }
+  assign_end<Q, T>(a, S, w, sh);
 }
 
 // Exclusive scan over the workgroup's kThreads values; total in *tot.
@@ -695,6 +837,9 @@ __global__ __launch_bounds__(kThreads) void basin_resolve_kernel(BasinArgs a) {
   constexpr int kBlock = kBlockOf<Q>, kPer = kBlock / kThreads;
   __shared__ int s_cnt[2 * kBasinLevels];
   __shared__ int s_base[2 * kBaseMax];
+  __shared__ int s_loc[2 * kBasinLevels];
+  __shared__ int s_scan[kThreads / 64];
+  __shared__ uint32_t s_list[kBlock];
   const int tid = threadIdx.x;
   const BlockRef br = decode_block<Q>(a, a.s_first, a.n_surf);
   const SurfDev S = a.surfs[br.s];
@@ -726,24 +871,45 @@ __global__ __launch_bounds__(kThreads) void basin_resolve_kernel(BasinArgs a) {
 #pragma unroll
   for (int t = 0; t < kPer; ++t) cr[t] = cr[t] == kInactive ? -1 : cr[t] | atomicAdd(&s_cnt[cr[t]], 1) << 16;
   __syncthreads();
-  for (int i = tid; i < 2 * kBasinLevels; i += kThreads)
-    if (s_cnt[i]) s_cnt[i] = atomicAdd(&unit[kBasinCur + i], s_cnt[i]);
+  // the workgroup's elements in level order (s_loc: a level's first place
+  // here), and what takes a place to the level's entries in the list
+  static_assert(kBasinLevels <= kThreads, "two level codes per thread");
+  int total;
+  {
+    const bool mine = tid < kBasinLevels;
+    const int c0 = mine ? s_cnt[2 * tid] : 0, c1 = mine ? s_cnt[2 * tid + 1] : 0;
+    const int l0 = block_excl_scan(c0 + c1, s_scan, &total);
+    if (mine) {
+      s_loc[2 * tid] = l0;
+      s_loc[2 * tid + 1] = l0 + c0;
+      if (c0) s_cnt[2 * tid] = atomicAdd(&unit[kBasinCur + 2 * tid], c0) - l0;
+      if (c1) s_cnt[2 * tid + 1] = atomicAdd(&unit[kBasinCur + 2 * tid + 1], c1) - (l0 + c0);
+    }
+  }
   __syncthreads();
+  constexpr int kChase = kPer < 8 ? kPer : 8;
 #pragma unroll
-  for (int r = 0; r < kPer / kRound; ++r) {
-    int e[kRound], n[kRound];
+  for (int r = 0; r < kPer / kChase; ++r) {
+    int e[kChase], n[kChase];
 #pragma unroll
-    for (int t = 0; t < kRound; ++t) e[t] = cr[r * kRound + t] >= 0 ? vb + (r * kRound + t) * kThreads : -1;
-    chase<kRound>(word, e, n);
+    for (int t = 0; t < kChase; ++t) e[t] = cr[r * kChase + t] >= 0 ? vb + (r * kChase + t) * kThreads : -1;
+    chase<kChase>(word, e, n);
 #pragma unroll
-    for (int t = 0; t < kRound; ++t) {
-      const int c = cr[r * kRound + t];
+    for (int t = 0; t < kChase; ++t) {
+      const int c = cr[r * kChase + t];
       if (c < 0) continue;
       const int lc = c & 0xffff;
-      const uint16_t bn = (uint16_t)basin(e[t], lc >= kBasinLevels ? 1 : 0, n[t]);
-      list[s_cnt[lc] + (c >> 16)] = bn;
-      if (a.bas) a.bas[e0 + vb + (r * kRound + t) * kThreads] = bn;
+      const unsigned bn = (uint16_t)basin(e[t], lc >= kBasinLevels ? 1 : 0, n[t]);
+      s_list[s_loc[lc] + (c >> 16)] = bn | (unsigned)lc << 16;
+      if (a.bas) a.bas[e0 + vb + (r * kChase + t) * kThreads] = (uint16_t)bn;
     }
+  }
+  // out in level order: a wave writes a few runs, where each element for
+  // itself was a line per lane
+  __syncthreads();
+  for (int i = tid; i < total; i += kThreads) {
+    const uint32_t w = s_list[i];
+    list[s_cnt[w >> 16] + i] = (uint16_t)w;
   }
   // the workgroup's saddle pairs, placed in level order by one reservation
   // per level and kThreads pairs (a returning atomic on the level's cursor per
@@ -1261,6 +1427,28 @@ void launch_assign(const BasinArgs& a, const BasinGroup& g, hipStream_t stream) 
     hipLaunchKernelGGL((basin_assign_table_kernel<W, Q>), grid, dim3(kThreads), 0, stream, a, g.s0, g.s1);
 }
 
+template <int NE, bool D16, int Q, bool NEAR>
+hipError_t launch_wide(const BasinArgs& a, const BasinGroup& g, hipStream_t stream) {
+  const size_t lds = NEAR ? sizeof(float) * (kBlockOf<Q> + 2 * (size_t)g.reach) : 0;
+  if (lds + sizeof(AssignShared<Q>) > 65536) {
+    const hipError_t e =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(basin_assign_wide_kernel<NE, D16, Q, NEAR>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL((basin_assign_wide_kernel<NE, D16, Q, NEAR>), dim3((unsigned)((int64_t)g.blocks * Q * a.pc)),
+                     dim3(kWideThreads<NEAR>), lds, stream, a, g.s0, g.s1);
+  return hipSuccess;
+}
+
+template <int NE, int Q>
+hipError_t launch_wide(const BasinArgs& a, const BasinGroup& g, hipStream_t stream) {
+  if constexpr (Q == 1) {
+    if (g.width & kBasinNear) return launch_wide<NE, true, Q, true>(a, g, stream);
+  }
+  return (g.width & 1) ? launch_wide<NE, true, Q, false>(a, g, stream) : launch_wide<NE, false, Q, false>(a, g, stream);
+}
+
 template <int Q>
 hipError_t launch_basin(const BasinArgs& a, const BasinGroup* groups, int n_groups, hipStream_t stream) {
   const unsigned units = (unsigned)((a.n_surf - a.s_first) * a.pc);
@@ -1275,7 +1463,14 @@ hipError_t launch_basin(const BasinArgs& a, const BasinGroup* groups, int n_grou
       case 8: launch_assign<8, Q>(a, groups[i], stream); break;
       case 12: launch_assign<12, Q>(a, groups[i], stream); break;
       case 16: launch_assign<16, Q>(a, groups[i], stream); break;
-      default: launch_assign<32, Q>(a, groups[i], stream); break;
+      default: {
+        const int entries = ((groups[i].width & ~kBasinNear) - kBasinWide) / 2;
+        const hipError_t e = entries == 18   ? launch_wide<18, Q>(a, groups[i], stream)
+                             : entries == 26 ? launch_wide<26, Q>(a, groups[i], stream)
+                             : entries == 32 ? launch_wide<32, Q>(a, groups[i], stream)
+                                             : hipErrorInvalidValue;
+        if (e != hipSuccess) return e;
+      }
     }
   }
   hipLaunchKernelGGL(basin_scan_kernel, dim3(units), threads, 0, stream, a);

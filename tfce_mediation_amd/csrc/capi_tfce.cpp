@@ -41,6 +41,9 @@ struct tfce_adj {
   uint8_t* d_nadj = nullptr;    // [V][ell_width] adjacency among a row's neighbours (width <= 8)
   uint32_t* d_adjw = nullptr;   // [V or distinct rows][ell_width] full row adjacency, rows wider than kNposMaxWidth
   uint16_t* d_adjid = nullptr;  // [V] row of d_adjw per element when d_adjw holds distinct rows only
+  uint32_t* d_tile = nullptr;   // SurfDev.tile
+  int32_t tile_entries = 0;     // entries per element there; 0: none
+  int32_t reach = 0;            // SurfDev.reach
   int32_t ell_width = 0;
   double* d_sizepow = nullptr;  // (double)s^E for s in [0, V] when E != 1
   SurfDev* d_surf = nullptr;    // one descriptor, offset 0
@@ -237,6 +240,8 @@ static SurfDev describe(const tfce_adj* a, int64_t offset) {
   sd.nadj = a->d_nadj;
   sd.adjw = a->d_adjw;
   sd.adjid = a->d_adjid;
+  sd.tile = a->d_tile;
+  sd.reach = a->reach;
   sd.sizepow = a->d_sizepow;
   sd.offset = offset;
   sd.V = a->V;
@@ -250,7 +255,13 @@ static SurfDev describe(const tfce_adj* a, int64_t offset) {
 // table (ring-packed or of fixed width).  Others (one-sided lists, lists of
 // more than kEllMaxWidth neighbours) stay with the element-wise sweep.
 static bool basin_ok(const tfce_adj* a) { return a->pairs_max > 0; }
-static int32_t basin_width(const tfce_adj* a) { return (a->flags & kSurfRing) ? 0 : a->ell_width; }
+// Which kernel of basin_assign takes a surface: 0 ring-packed rows, a table's
+// width, or kBasinWide + the entries and form of its tiles.
+static int32_t basin_width(const tfce_adj* a) {
+  if (a->flags & kSurfRing) return 0;
+  if (!a->tile_entries) return a->ell_width;
+  return kBasinWide + 2 * a->tile_entries + (a->reach <= 32767 ? 1 : 0) + (a->reach <= kNearReach ? kBasinNear : 0);
+}
 
 // Appends a surface to the basin sweep's scratch layout.
 static void span_add(BasinSpan& p, const tfce_adj* a, SurfDev& sd) {
@@ -283,9 +294,10 @@ static void span_add(BasinSpan& p, const tfce_adj* a, SurfDev& sd) {
   p.sure_full = p.sure_full && (int64_t)a->basins_max * kBasinLevels <= b.tab_cap;
   const int32_t at = p.first + p.n++;
   if (p.groups.empty() || p.groups.back().width != basin_width(a))
-    p.groups.push_back(BasinGroup{basin_width(a), at, at, 0});
+    p.groups.push_back(BasinGroup{basin_width(a), at, at, 0, 0});
   p.groups.back().s1 = at + 1;
   p.groups.back().blocks += b.nblk;
+  p.groups.back().reach = std::max(p.groups.back().reach, a->reach);
 }
 
 extern "C" {
@@ -344,6 +356,7 @@ int tfce_adj_create_ex(const int32_t* row_ptr, const int32_t* col, int32_t V, in
     if (a->d_nadj) (void)hipFree(a->d_nadj);
     if (a->d_adjw) (void)hipFree(a->d_adjw);
     if (a->d_adjid) (void)hipFree(a->d_adjid);
+    if (a->d_tile) (void)hipFree(a->d_tile);
     if (a->d_sizepow) (void)hipFree(a->d_sizepow);
     if (a->d_surf) (void)hipFree(a->d_surf);
     delete a;
@@ -449,6 +462,31 @@ int tfce_adj_create_ex(const int32_t* row_ptr, const int32_t* col, int32_t V, in
           const bool plain = listed == nnz && 2 * earlier == listed;
           a->basins_max = (plain && deg_min > 0) ? (int32_t)((int64_t)V * arcs_max / (deg_min + arcs_max)) + 1 : V;
         } else {
+          if (width > kNposMaxWidth) {
+            // wide rows: the entries adjacent to most of the row first (the
+            // face neighbours of a volume), from which the groups of a row's
+            // entries are found in the fewest steps
+            std::vector<int32_t> mark(V, -1);
+            for (int32_t v = 0; v < V; ++v) {
+              int32_t* row = ell.data() + (size_t)v * width;
+              const int32_t deg = row_ptr[v + 1] - row_ptr[v];
+              for (int32_t j = 0; j < deg; ++j) mark[row[j]] = v;
+              std::pair<int32_t, int32_t> by[kEllMaxWidth];
+              for (int32_t j = 0; j < deg; ++j) {
+                int32_t n = 0;
+                for (int32_t e2 = row_ptr[row[j]]; e2 < row_ptr[row[j] + 1]; ++e2) n += mark[col[e2]] == v;
+                by[j] = std::make_pair(-n, row[j]);
+              }
+              std::stable_sort(by, by + deg,
+                               [](const std::pair<int32_t, int32_t>& x, const std::pair<int32_t, int32_t>& y) {
+                                 return x.first < y.first;
+                               });
+              for (int32_t j = 0; j < deg; ++j) row[j] = by[j].second;
+            }
+            if ((e = hipMemcpy(a->d_ell, ell.data(), sizeof(int32_t) * ell.size(), hipMemcpyHostToDevice)) !=
+                hipSuccess)
+              return cleanup(-(int)e, "upload reordered ell");
+          }
           std::vector<uint8_t> nadj((size_t)V * width, 0);
           for (int32_t v = 0; v < V; ++v)
             for (int32_t j = 0; j < width; ++j) {
@@ -527,6 +565,34 @@ int tfce_adj_create_ex(const int32_t* row_ptr, const int32_t* col, int32_t V, in
               if ((e = hipMemcpy(a->d_adjid, rid.data(), ibytes, hipMemcpyHostToDevice)) != hipSuccess)
                 return cleanup(-(int)e, "upload adjid");
             }
+            // the smallest number of entries the kernels are built for: 18- and
+            // 26-connected volumes, others
+            const int32_t entries = max_deg <= 18 ? 18 : max_deg <= 26 ? 26 : 32;
+            for (int32_t v = 0; v < V; ++v)
+              for (int32_t e2 = row_ptr[v]; e2 < row_ptr[v + 1]; ++e2)
+                a->reach = std::max(a->reach, std::abs(col[e2] - v));
+            const bool d16 = a->reach <= 32767;
+            const int32_t words = tile_words(entries, d16);
+            const int32_t rows = (V + kTileRows - 1) / kTileRows * kTileRows;
+            std::vector<uint32_t> tile((size_t)rows * words);
+            for (int32_t v = 0; v < rows; ++v) {
+              uint32_t* w = tile.data() + (size_t)(v >> 6) * words * 64 + (v & 63);
+              const int32_t deg = v < V ? row_ptr[v + 1] - row_ptr[v] : 0;
+              const int32_t* row = v < V ? ell.data() + (size_t)v * width : nullptr;
+              for (int32_t j = 0; j < entries; ++j) {
+                const int32_t u = deg ? row[j < deg ? j : 0] : std::min(v, V - 1);
+                if (d16)
+                  w[(j / 2) * 64] |= (uint32_t)(uint16_t)(u - v) << (16 * (j & 1));
+                else
+                  w[j * 64] = (uint32_t)u;
+              }
+              w[(words - 1) * 64] = (uint32_t)deg | (use_dict && v < V ? (uint32_t)rid[v] << 16 : 0u);
+            }
+            const size_t tbytes = tile.size() * sizeof(uint32_t);
+            if ((e = hipMalloc(&a->d_tile, tbytes)) != hipSuccess) return cleanup(-(int)e, "hipMalloc(tile)");
+            if ((e = hipMemcpy(a->d_tile, tile.data(), tbytes, hipMemcpyHostToDevice)) != hipSuccess)
+              return cleanup(-(int)e, "upload tile");
+            a->tile_entries = entries;
           }
         }
       }
@@ -538,7 +604,7 @@ int tfce_adj_create_ex(const int32_t* row_ptr, const int32_t* col, int32_t V, in
     if ((e = launch_sizepow(a->d_sizepow, V, E, nullptr)) != hipSuccess || (e = hipDeviceSynchronize()) != hipSuccess)
       return cleanup(-(int)e, "sizepow table");
   }
-  if (symmetric && a->d_ell && !(a->flags & kSurfRing)) {
+  if (symmetric && a->d_ell && !(a->flags & kSurfRing) && (a->ell_width <= kNposMaxWidth || a->d_tile)) {
     a->pairs_max = std::max(a->ell_width - 1, 1);
     a->basins_max = V;
   }
@@ -636,6 +702,7 @@ int tfce_adj_destroy(tfce_adj_t* a) {
   if (a->d_nadj) (void)hipFree(a->d_nadj);
   if (a->d_adjw) (void)hipFree(a->d_adjw);
   if (a->d_adjid) (void)hipFree(a->d_adjid);
+  if (a->d_tile) (void)hipFree(a->d_tile);
   if (a->d_sizepow) (void)hipFree(a->d_sizepow);
   (void)hipFree(a->d_surf);
   delete a;

@@ -84,6 +84,18 @@ constexpr int kBasinEvCur = kBasinCur + 2 * kBasinLevels;
 constexpr int kBasinCount = kBasinEvCur + 2 * kBasinLevels;
 constexpr int kBasinUnitWords = kBasinCount + 4;
 
+// Wide neighbour lists for the basin sweep: tiles of 64 elements, word i of the
+// 64 side by side, so that a wave reads a list entry of its elements from two
+// cache lines (rows of 32 entries: from 64).  Words 0 .. : the neighbours, in the
+// order of the surface's table, as 16-bit differences from the element (two per
+// word, low half first) or as indices; the rest of a list repeats its first entry
+// (an empty one: the element).  Last word: the list's length, and from bit 16
+// the element's row of adjw if rows are shared.  Whole workgroups of elements
+// (kTileRows) are present; those past the surface have empty lists of its last
+// element.
+constexpr int kTileRows = 256;
+constexpr int tile_words(int entries, bool d16) { return (d16 ? entries / 2 : entries) + 1; }
+
 struct SurfDev {
   const int32_t* row_ptr;  // V+1
   const int32_t* col;      // nnz (indices local to the surface)
@@ -96,6 +108,8 @@ struct SurfDev {
                            // neighbours j and k are adjacent; null if not built
   const uint16_t* adjid;   // [V] with adjw: the row of adjw that holds element v's masks (adjw then
                            // holds each distinct row once), or null: row v
+  const uint32_t* tile;    // lists of 17 to 32 entries for the basin sweep, null if none (kTileRows)
+  int32_t reach;           // with tile: largest difference between an element's index and a neighbour's
   const double* sizepow;   // [V+1] (double)s^E, null when E == 1
   int64_t offset;          // first element of this surface inside a map row
   int32_t V;
@@ -233,8 +247,13 @@ struct BasinArgs {
 };
 // Consecutive surfaces [s0, s1) of one table form: ring-packed (width 0) or a
 // fixed-width table; `blocks` workgroups of the vertex passes per map.
+// Surfaces with tiles: width kBasinWide + 2 * entries + (16-bit differences) +
+// kBasinNear if no neighbour is further off than kNearReach; reach: the
+// furthest of the group.
+constexpr int kBasinWide = 64, kBasinNear = 256;
+constexpr int kNearReach = 15000;
 struct BasinGroup {
-  int32_t width, s0, s1, blocks;
+  int32_t width, s0, s1, blocks, reach;
 };
 hipError_t launch_basin_batch(const BasinArgs& a, const BasinGroup* groups, int n_groups, hipStream_t stream);
 // The element-wise sweep over a list of items whose records are written
