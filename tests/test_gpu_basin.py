@@ -269,3 +269,23 @@ def test_wide_lists(near, far, P):
             x = (np.float32(sgn) * maps[p]).astype(np.float32)
             enh, _, _ = otfce.tfce(*csr, x, 2.0, 1.0, exact_pow=True)
             assert out[p, k] == np.float32(enh.max() * np.float32(x.max() / np.float32(100))), (p, k)
+
+
+@pytest.mark.parametrize("E", [0.5, 0.67, 2.0])
+@pytest.mark.parametrize("order", [4, 6, 7])
+def test_exponents(order, E):
+    """Gains by root, by table, over one basin per thread, fours in LDS and 16-bit
+    parents (white noise: 380, 5,900 and 23,400 basins).  Bar: 16 ulp, the sum of
+    100 increments each within one rounding of a power that the two sides take
+    from different libraries (E = 0.5: one correctly rounded root)."""
+    csr = synth.icosphere_csr(order)
+    import torch
+    from tfce_mediation_amd.tfce import Adjacency, SurfaceSet
+    V = len(csr[0]) - 1
+    x = np.random.default_rng(order).standard_normal((2, V)).astype(np.float32)
+    say(f"[gpu] basin sweep E={E} V={V}")
+    out = SurfaceSet([Adjacency(csr, 2.0, E)], [0]).batch(torch.from_numpy(x).cuda(), 1).cpu().numpy()[0]
+    for p in range(2):
+        enh, _, _ = otfce.tfce(*csr, x[p], 2.0, E, exact_pow=True)
+        exp = np.float32(enh.max() * np.float32(x[p].max() / np.float32(100)))
+        assert abs(int(np.float32(out[p, 0]).view(np.int32)) - int(exp.view(np.int32))) <= (0 if E == 0.5 else 16)

@@ -980,8 +980,10 @@ struct Parents {
       return seen;
     }
   }
-  // Roots of N basins (x[j] < 0: none), the chains' reads interleaved.
-  template <int N>
+  // Roots of N basins (x[j] < 0: none), the chains' reads interleaved.  SPLIT:
+  // every basin passed on the way is put under its grandparent (a basin that is
+  // no root may be written at any time: the hooks only change roots).
+  template <bool SPLIT, int N>
   __device__ __forceinline__ void roots(int (&x)[N]) const {
     int up[N];
 #pragma unroll
@@ -996,6 +998,7 @@ struct Parents {
       for (int j = 0; j < N; ++j) q[j] = up[j] >= 0 ? get(up[j]) : up[j];
 #pragma unroll
       for (int j = 0; j < N; ++j) {
+        if (SPLIT && q[j] != up[j]) const_cast<Parents*>(this)->set(x[j], q[j]);
         x[j] = up[j];
         up[j] = q[j];
       }
@@ -1003,7 +1006,7 @@ struct Parents {
   }
 };
 
-constexpr int kIlp = 4;  // basins or elements in flight per thread
+constexpr int kIlp = 4;  // elements in flight per thread
 
 // Adds the wave's active lanes' elements to their roots' sizes: those of the
 // first lane's root as one addition.
@@ -1019,18 +1022,25 @@ __device__ __forceinline__ void count_wave(int* size, int r) {
 // barrier:
 //   A  the level's saddle pairs hook roots (the larger under the smaller, by
 //      CAS).  Beside it every root gains the previous level's
-//      (float)(size^E * T^H), and a basin whose parent was hooked there moves up
-//      one step;
+//      (float)(size^E * T^H);
 //   B  every hooked root hands its size and its value (the larger one stays) to
 //      its final root, and the level's elements add to their roots' sizes.
 // A root's value is the largest TFCE among its members (members gain the same
 // increments once joined, and the earliest element has the most of them), so
 // the largest value over the roots is the image's maximum, bit for bit.
-// Bound by the instructions a wave issues per level, times about 100 levels:
-// an image of the batch has its own workgroup and its levels are a chain, so
-// the number of instructions on that chain counts, not the LDS operations.
-// Hence one basin and one element per thread where that is enough (N = 1) and
-// the level tables in registers, level l in lane l % 64.
+// Bound by the chain of a level (about 100 of them): LDS round trips and the
+// instructions around them, not the LDS operations.  Hence reads that do not
+// depend on each other are issued together (a basin's size, value and parent
+// beside the pair's parents; the roots of the hooked basin and of the element
+// together), the level tables are in registers, level l in lane l % 64, and the
+// gains take one basin per thread, or four neighbouring ones by 16-byte accesses
+// where there are more.  Basins are brought near their roots by one step up per
+// level (one per thread) or, where looking at all of them would cost more, by
+// splitting the paths that are walked.  1,024 images of 2,640 basins: 396 ->
+// 313 us; of 8,400: 1,230 -> 980; 16-bit parents, 23,400 basins: 3.7 -> 2.65 ms (its
+// values past the vector cache at workgroup scope: agent scope left the XCD's L2
+// at every level, 24 GB).  Slower: one wave per image of few basins (no barriers,
+// twice the instructions per wave), three fours in flight (registers).
 // P16: 16-bit parents and the values in global memory (the map's dead saddle
 // candidates), for images of more basins.
 // FULL: no values; every level's gain of every basin's component goes to the
@@ -1038,7 +1048,7 @@ __device__ __forceinline__ void count_wave(int* size, int r) {
 // per element.
 template <int T, bool P16, bool FULL>
 __global__ __launch_bounds__(T) void basin_sweep_kernel(BasinArgs a, int nb_lo, int nb_hi) {
-  extern __shared__ int s_dyn[];
+  extern __shared__ __attribute__((aligned(16))) int s_dyn[];
   __shared__ float s_red[T / 64];
   // a surface's images are consecutive workgroups: those of one LDS size are
   // spread over the XCDs (with the surfaces innermost, two large surfaces of
@@ -1054,7 +1064,7 @@ __global__ __launch_bounds__(T) void basin_sweep_kernel(BasinArgs a, int nb_lo, 
   const int status = rec[kPrepL];
   const int L = status > 0 ? status : 0;
   const int tid = threadIdx.x;
-  // (nb_hi is even)
+  // (nb_hi is a multiple of eight)
   Parents<P16> par{reinterpret_cast<typename Parents<P16>::type*>(s_dyn)};
   int* size = s_dyn + (P16 ? nb_hi / 2 : nb_hi);
   float* val = reinterpret_cast<float*>(size + nb_hi);
@@ -1064,89 +1074,127 @@ __global__ __launch_bounds__(T) void basin_sweep_kernel(BasinArgs a, int nb_lo, 
   float* tab = FULL ? a.tab + ((int64_t)lp * a.n_signs + g) * a.tab_total + S.basin.tab0 : nullptr;
   auto val_get = [&](int c) -> float {
     if constexpr (FULL) return 0.0f;
-    else if constexpr (P16) return __hip_atomic_load(val + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else if constexpr (P16) return __hip_atomic_load(val + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     else return val[c];
   };
   auto val_set = [&](int c, float v) {
     if constexpr (FULL) return;
-    else if constexpr (P16) __hip_atomic_store(val + c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else if constexpr (P16) __hip_atomic_store(val + c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     else val[c] = v;
+  };
+  // values in global memory are read and written past the vector cache (the
+  // last argument: sc0), which the maxima of hand_over do not pass through
+  typedef unsigned Words __attribute__((ext_vector_type(4)));
+  const __amdgpu_buffer_rsrc_t val_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(val, 0, P16 ? 4 * ((nb + 3) & ~3) : 0, 0x00027000);
+  auto four_get = [&](int c, float (&v)[4]) {
+    if constexpr (P16) {
+      const Words x = __builtin_amdgcn_raw_buffer_load_b128(val_rsrc, 4 * c, 0, 1);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(x[i]);
+    } else {
+      const float4 x = *reinterpret_cast<const float4*>(val + c);
+      v[0] = x.x;
+      v[1] = x.y;
+      v[2] = x.z;
+      v[3] = x.w;
+    }
+  };
+  auto four_set = [&](int c, const float (&v)[4]) {
+    if constexpr (P16) {
+      Words x;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = __float_as_uint(v[i]);
+      __builtin_amdgcn_raw_buffer_store_b128(x, val_rsrc, 4 * c, 0, 1);
+    } else {
+      *reinterpret_cast<float4*>(val + c) = make_float4(v[0], v[1], v[2], v[3]);
+    }
   };
   auto level_barrier = [&]() {
     if constexpr (P16 && !FULL) __syncthreads();
     else lds_barrier();
   };
-  for (int c = tid; c < nb; c += T) {
-    par.set(c, c);
+  for (int c = tid; c < ((nb + 3) & ~3); c += T) {
+    if (c < nb) par.set(c, c);
     size[c] = 0;
-    val_set(c, 0.0f);
+    if (c < nb || !P16) val_set(c, 0.0f);
   }
   __syncthreads();
   const uint16_t* list = a.list + (int64_t)lp * a.elt_total + S.basin.elt0;
   uint32_t* ev = a.ev + (int64_t)lp * a.ev_total + S.basin.ev0;
-  // gains of level l for basins c0 + j T; a basin that is no root, or not yet
-  // reached, has size 0
-  auto gain = [&](float HH, int l) {
-    if constexpr (FULL) {
-      float* out = tab + (int64_t)(l >> 3) * nb * 8 + (l & 7);
-      for (int c0 = tid; c0 < nb; c0 += kIlp * T) {
-        int r[kIlp], sz[kIlp];
-#pragma unroll
-        for (int j = 0; j < kIlp; ++j) r[j] = c0 + j * T < nb ? c0 + j * T : -1;
-        par.roots(r);
-#pragma unroll
-        for (int j = 0; j < kIlp; ++j) sz[j] = size[max(r[j], 0)];
-#pragma unroll
-        for (int j = 0; j < kIlp; ++j)
-          if (r[j] >= 0) out[(unsigned)(c0 + j * T) * 8u] = tfce_inc(sz[j], HH, S.E, S.sizepow);
+  const bool one = nb <= T;  // a basin per thread
+  const int own = min(tid, nb - 1);
+  // FULL: gains of level l, and every basin put under its root
+  auto gain_full = [&](float HH, int l) {
+    float* out = tab + (int64_t)(l >> 3) * nb * 8 + (l & 7);
+    if (one) {
+      int r[1] = {own};
+      par.template roots<false>(r);
+      const float inc = tfce_inc(size[r[0]], HH, S.E, S.sizepow);
+      if (tid < nb) {
+        if (r[0] != tid) par.set(tid, r[0]);
+        out[(unsigned)tid * 8u] = inc;
       }
-      return;
-    }
-    if (nb <= T) {
-      const int c = min(tid, nb - 1);
-      const int sz = size[c];
-      const float v = val_get(c);
-      if (sz && tid < nb) val_set(c, v + tfce_inc(sz, HH, S.E, S.sizepow));
       return;
     }
     for (int c0 = tid; c0 < nb; c0 += kIlp * T) {
-      int sz[kIlp];
-      float v[kIlp];
+      int r[kIlp], sz[kIlp];
+#pragma unroll
+      for (int j = 0; j < kIlp; ++j) r[j] = c0 + j * T < nb ? c0 + j * T : -1;
+      par.template roots<false>(r);
+#pragma unroll
+      for (int j = 0; j < kIlp; ++j) sz[j] = size[max(r[j], 0)];
 #pragma unroll
       for (int j = 0; j < kIlp; ++j) {
-        const int c = min(c0 + j * T, nb - 1);
-        sz[j] = size[c];
-        if (!P16) v[j] = val_get(c);
+        const int c = c0 + j * T;
+        if (r[j] < 0) continue;
+        if (r[j] != c) par.set(c, r[j]);
+        out[(unsigned)c * 8u] = tfce_inc(sz[j], HH, S.E, S.sizepow);
       }
-      if (P16) {
-#pragma unroll
-        for (int j = 0; j < kIlp; ++j) v[j] = sz[j] ? val_get(min(c0 + j * T, nb - 1)) : 0.0f;
-      }
-#pragma unroll
-      for (int j = 0; j < kIlp; ++j)
-        if (sz[j] && c0 + j * T < nb) val_set(c0 + j * T, v[j] + tfce_inc(sz[j], HH, S.E, S.sizepow));
     }
   };
-  // one step up for basins whose parent was hooked; a basin that is no root
-  // has its parent written by its own thread only
-  auto move_up = [&]() {
-    for (int c0 = tid; c0 < nb; c0 += 2 * T) {
-      const int c1 = min(c0 + T, nb - 1);
-      const int p0 = par.get(c0), p1 = par.get(c1);
-      const int q0 = par.get(p0), q1 = par.get(p1);
-      if (q0 != p0) par.set(c0, q0);
-      if (q1 != p1 && c0 + T < nb) par.set(c1, q1);
+  // the gain HH of a level for all basins, four neighbouring ones at a time
+  // (sizes and values lie on 16 bytes); a basin that is no root, or not yet
+  // reached, has size 0
+  auto gain_fours = [&](auto inc) {
+    for (int c0 = 4 * tid; c0 < nb; c0 += 4 * T) {
+      const int4 z = *reinterpret_cast<const int4*>(size + c0);
+      if ((z.x | z.y | z.z | z.w) == 0) continue;
+      const int zs[4] = {z.x, z.y, z.z, z.w};
+      float v[4], w[4];
+      four_get(c0, v);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[i] = inc(zs[i]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = zs[i] ? v[i] + w[i] : v[i];
+      four_set(c0, v);
     }
   };
-  auto hand_over = [&](int c) {
-    const int sz = size[c];
-    int r[1] = {c};
-    par.roots(r);
+  const Global<double> sizepow = (Global<double>)S.sizepow;
+  auto gain_all = [&](float HH) {
+    if (S.E == 1.0f) gain_fours([&](int z) { return __fmul_rn((float)z, HH); });
+    else if (S.E == 0.5f) gain_fours([&](int z) { return __double2float_rn(sqrt_pos((double)z) * (double)HH); });
+    else gain_fours([&](int z) { return __double2float_rn(sizepow[z] * (double)HH); });
+  };
+  auto hand_over = [&](int c, int r, int sz, float v) {
     if (sz) {  // 0: a basin reached at this level
-      atomicAdd(&size[r[0]], sz);
-      if constexpr (!FULL) atomicMax(reinterpret_cast<int*>(val) + r[0], __float_as_int(val_get(c)));
+      atomicAdd(&size[r], sz);
+      if constexpr (!FULL)
+        (void)__hip_atomic_fetch_max(reinterpret_cast<int*>(val) + r, __float_as_int(v), __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_WORKGROUP);
       size[c] = 0;
     }
+  };
+  // the larger of two roots under the smaller; the one hooked, -1 if they were one
+  auto join = [&](int p, int q) -> int {
+    while (p != q) {
+      const int hi = max(p, q), lo = min(p, q);
+      const int seen = par.hook(hi, lo);
+      if (seen == hi) return hi;
+      p = seen;  // hi was no root: its parent (smaller) takes its place
+      q = lo;
+    }
+    return -1;
   };
   bool moved = false;  // roots were hooked at the last level
   float HH = 0.0f;     // its T^H
@@ -1176,57 +1224,89 @@ __global__ __launch_bounds__(T) void basin_sweep_kernel(BasinArgs a, int nb_lo, 
       // A
       int mine = -1;  // the root that this thread's first pair hooked
       const bool pairs = e1 > e0;
+      // one basin per thread: its reads are issued beside those of the pair
+      int sz = 0, up = own, up2 = own;
+      float v = 0.0f;
+      if (one && !FULL) {
+        sz = size[own];
+        v = val_get(own);
+        if (moved) up = par.get(own);
+      }
+      int p = 0, q = 0;
       if (pairs) {
-        for (int k = e0 + tid; k < e1; k += T) {
-          const uint32_t w = k == e0 + tid ? evw : ev[k];
-          int p = par.get((int)(w & 0xffffu)), q = par.get((int)(w >> 16));
-          int hit = -1;
-          while (p != q) {
-            const int hi = max(p, q), lo = min(p, q);
-            const int seen = par.hook(hi, lo);
-            if (seen == hi) {
-              hit = hi;
-              break;
-            }
-            p = seen;  // hi was no root: its parent (smaller) takes its place
-            q = lo;
+        p = par.get((int)(evw & 0xffffu));
+        q = par.get((int)(evw >> 16));
+      }
+      if (one && !FULL && moved) up2 = par.get(up);
+      if (pairs) {
+        if (e0 + tid < e1) {
+          if (!one) {
+            int r[2] = {p, q};
+            par.template roots<true>(r);
+            p = r[0];
+            q = r[1];
           }
+          mine = join(p, q);
+        }
+        for (int k = e0 + T + tid; k < e1; k += T) {
+          const uint32_t w = ev[k];
+          int r[2] = {(int)(w & 0xffffu), (int)(w >> 16)};
+          par.template roots<true>(r);
           // a thread's later pairs leave the root they hooked in their place
-          if (k == e0 + tid) mine = hit;
-          else ev[k] = (uint32_t)(hit + 1);
+          ev[k] = (uint32_t)(join(r[0], r[1]) + 1);
         }
       }
-      if constexpr (!FULL) gain(HH, 0);
-      if (moved) move_up();
+      if constexpr (!FULL) {
+        if (one) {
+          if (tid < nb) {
+            if (sz) val_set(tid, v + tfce_inc(sz, HH, S.E, S.sizepow));
+            // one step up for a basin whose parent was hooked
+            if (up2 != up) par.set(tid, up2);
+          }
+        } else {
+          gain_all(HH);
+        }
+      }
       moved = pairs;
       HH = __int_as_float(__builtin_amdgcn_readlane(t_HH, l));
       level_barrier();
       // B
-      if (pairs) {
-        if (mine >= 0) hand_over(mine);
-        for (int k = e0 + T + tid; k < e1; k += T) {
-          const int c = (int)ev[k] - 1;
-          if (c >= 0) hand_over(c);
+      {
+        const bool some = b0 + tid < b1;
+        const int m = max(mine, 0);
+        const int zm = pairs ? size[m] : 0;
+        const float vm = pairs ? val_get(m) : 0.0f;
+        if (pairs) {
+          int r[2] = {mine, some ? el : -1};
+          par.template roots<true>(r);
+          if (mine >= 0) hand_over(mine, r[0], zm, vm);
+          if (some) count_wave(size, r[1]);
+          for (int k = e0 + T + tid; k < e1; k += T) {
+            const int c = (int)ev[k] - 1;
+            int rc[1] = {c};
+            if (c < 0) continue;
+            par.template roots<true>(rc);
+            hand_over(c, rc[0], size[c], val_get(c));
+          }
+        } else if (some) {
+          int r[1] = {el};
+          par.template roots<true>(r);
+          count_wave(size, r[0]);
         }
-      }
-      if (b0 + tid < b1) {
-        int r[1] = {el};
-        par.roots(r);
-        count_wave(size, r[0]);
       }
       // more than one element per thread: kIlp at a time
       for (int k0 = b0 + T + tid; k0 < b1; k0 += kIlp * T) {
         int r[kIlp];
 #pragma unroll
         for (int j = 0; j < kIlp; ++j) r[j] = k0 + j * T < b1 ? (int)list[(unsigned)(k0 + j * T)] : -1;
-        par.roots(r);
+        par.template roots<true>(r);
 #pragma unroll
         for (int j = 0; j < kIlp; ++j)
           if (r[j] >= 0) count_wave(size, r[j]);
       }
       level_barrier();
       if constexpr (FULL) {  // before the next level's unions
-        gain(HH, lb + l);
+        gain_full(HH, lb + l);
         level_barrier();
       }
       b0 = nb0;
@@ -1236,7 +1316,7 @@ __global__ __launch_bounds__(T) void basin_sweep_kernel(BasinArgs a, int nb_lo, 
     }
   }
   if constexpr (FULL) return;
-  if (L > 0) gain(HH, 0);
+  if (L > 0) gain_all(HH);
   __syncthreads();
   float best = 0.0f;
   for (int c = tid; c < nb; c += T) best = fmaxf(best, val_get(c));
@@ -1405,7 +1485,7 @@ __global__ void basin_clear_kernel(int32_t* rest, int32_t* queue) {
 // Images of at most `hi` basins and more than *lo, which becomes hi.
 template <int T, bool P16, bool FULL>
 hipError_t launch_sweep(const BasinArgs& a, unsigned units, int* lo, int hi, hipStream_t stream) {
-  hi = std::min(hi, (a.nb_max + 1) & ~1);
+  hi = std::min(hi, (a.nb_max + 7) & ~7);
   if (hi <= *lo) return hipSuccess;
   const size_t lds = (size_t)hi * (P16 ? 6 : (FULL ? 8 : 12));
   if (lds > 65536) {

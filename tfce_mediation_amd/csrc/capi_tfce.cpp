@@ -45,7 +45,7 @@ struct tfce_adj {
   int32_t tile_entries = 0;     // entries per element there; 0: none
   int32_t reach = 0;            // SurfDev.reach
   int32_t ell_width = 0;
-  double* d_sizepow = nullptr;  // (double)s^E for s in [0, V] when E != 1
+  double* d_sizepow = nullptr;  // (double)s^E for s in [0, V], null when E is 1 or 0.5
   SurfDev* d_surf = nullptr;    // one descriptor, offset 0
   int32_t basins_max = 0;       // most local maxima an image can have
   int32_t pairs_max = 0;        // most saddle pairs of one element (basin sweep); 0: not taken
@@ -598,7 +598,7 @@ int tfce_adj_create_ex(const int32_t* row_ptr, const int32_t* col, int32_t V, in
       }
     }
   }
-  if (E != 1.0f) {
+  if (E != 1.0f && E != 0.5f) {
     if ((e = hipMalloc(&a->d_sizepow, sizeof(double) * ((size_t)V + 1))) != hipSuccess)
       return cleanup(-(int)e, "hipMalloc(sizepow)");
     if ((e = launch_sizepow(a->d_sizepow, V, E, nullptr)) != hipSuccess || (e = hipDeviceSynchronize()) != hipSuccess)

@@ -1,14 +1,19 @@
 // Device helpers shared by the TFCE kernels.
 #pragma once
+#include "sqrt_pos.h"
 #include "tfce_internal.h"
 
 namespace tfcehip {
 
 // (float)(s^E * HH) for one component: E == 1 is one correctly rounded float
-// product (exact in double, as fast_tfce.hpp:77 computes it); otherwise the
-// per-adjacency table holds (double)s^E.
+// product (exact in double, as fast_tfce.hpp:77 computes it).  E == 0.5 takes
+// the root itself (the hardware's reciprocal root and two residual corrections:
+// equal to the library's sqrt for every whole number up to 2^24, checked one by
+// one) instead of a random 8 bytes of global memory; any other exponent has
+// (double)s^E in the per-adjacency table.
 __device__ __forceinline__ float tfce_inc(int size, float HH, float E, const double* sizepow) {
   if (E == 1.0f) return __fmul_rn((float)size, HH);
+  if (E == 0.5f) return size > 0 ? __double2float_rn(sqrt_pos((double)size) * (double)HH) : 0.0f;
   return __double2float_rn(sizepow[size] * (double)HH);
 }
 

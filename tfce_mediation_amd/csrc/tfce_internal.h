@@ -110,7 +110,7 @@ struct SurfDev {
                            // holds each distinct row once), or null: row v
   const uint32_t* tile;    // lists of 17 to 32 entries for the basin sweep, null if none (kTileRows)
   int32_t reach;           // with tile: largest difference between an element's index and a neighbour's
-  const double* sizepow;   // [V+1] (double)s^E, null when E == 1
+  const double* sizepow;   // [V+1] (double)s^E, null when E is 1 or 0.5
   int64_t offset;          // first element of this surface inside a map row
   int32_t V;
   int32_t flags;
@@ -164,7 +164,7 @@ constexpr int kPrepWords = kPrepT + 2 * kMaxLevels;
 struct TfceCoopArgs {
   const int32_t* row_ptr;  // V+1
   const int32_t* col;
-  const double* sizepow;   // null when E == 1
+  const double* sizepow;   // null when E is 1 or 0.5
   float E;
   int32_t V;
   const float* x;          // image [V]

@@ -1814,8 +1814,7 @@ __global__ __launch_bounds__(kTfceThreads) void shared_T0_kernel(TfceBatchArgs a
 __global__ void sizepow_kernel(double* out, int32_t n, double E) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i > n) return;
-  const double s = (double)i;
-  out[i] = (E == 0.5) ? sqrt(s) : pow(s, E);
+  out[i] = pow((double)i, E);
 }
 
 __global__ void fill_f32_kernel(float* p, int64_t n, float v) {
