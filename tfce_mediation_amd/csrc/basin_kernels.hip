@@ -56,6 +56,7 @@ constexpr uint16_t kInactive = 0xffff;
 // compute unit, not threads per image, fill it: 2,640-basin images took 398 us
 // a launch of 1,024 with four workgroups of 256 threads per compute unit, 493
 // with four of 512.
+constexpr int64_t kWideMinV = 16384;
 constexpr int kBasinTiny = 1696, kBasinSmall = 3400, kBasinMid = 6800, kBasinMax12 = 13600;
 
 // A pointer read from a descriptor, known to be global memory.
@@ -1529,6 +1530,17 @@ hipError_t launch_wide(const BasinArgs& a, const BasinGroup& g, hipStream_t stre
   return (g.width & 1) ? launch_wide<NE, true, Q, false>(a, g, stream) : launch_wide<NE, false, Q, false>(a, g, stream);
 }
 
+// Launches of at most two images per compute unit over large surfaces: 1,024
+// threads per image, for nothing else would fill the unit and an image's levels
+// have elements and basins for them (300 images of 25k voxels: 268 -> 203 us;
+// one image of 163,842 vertices 384 -> 353 us in all).  Below kWideMinV elements a
+// level is shorter than the barriers of 16 waves (64 maps of 2,562 vertices stay
+// with 256 threads).
+bool few_large_images(const BasinArgs& a, unsigned units) {
+  const int64_t surfaces = a.n_surf - a.s_first;
+  return (int64_t)units * a.n_signs <= 512 && a.elt_total > kWideMinV * surfaces;
+}
+
 template <int Q>
 hipError_t launch_basin(const BasinArgs& a, const BasinGroup* groups, int n_groups, hipStream_t stream) {
   const unsigned units = (unsigned)((a.n_surf - a.s_first) * a.pc);
@@ -1557,8 +1569,10 @@ hipError_t launch_basin(const BasinArgs& a, const BasinGroup* groups, int n_grou
   hipLaunchKernelGGL(basin_resolve_kernel<Q>, grid, threads, 0, stream, a);
   int lo = -1;
   hipError_t e = hipSuccess;
+  const bool wide = few_large_images(a, units);
   if (a.tab) {
-    e = launch_sweep<256, false, true>(a, units, &lo, kBasinTiny, stream);
+    if (wide) e = launch_sweep<1024, false, true>(a, units, &lo, kBasinMid, stream);
+    else e = launch_sweep<256, false, true>(a, units, &lo, kBasinTiny, stream);
     if (e == hipSuccess) e = launch_sweep<512, false, true>(a, units, &lo, kBasinMid, stream);
     if (e == hipSuccess) e = launch_sweep<1024, true, true>(a, units, &lo, kBasinMax, stream);
     if (e != hipSuccess) return e;
@@ -1566,7 +1580,8 @@ hipError_t launch_basin(const BasinArgs& a, const BasinGroup* groups, int n_grou
     hipLaunchKernelGGL(basin_final_kernel, dim3(units * a.n_signs), dim3(64), 0, stream, a);
     return hipGetLastError();
   }
-  e = launch_sweep<256, false, false>(a, units, &lo, kBasinTiny, stream);
+  if (wide) e = launch_sweep<1024, false, false>(a, units, &lo, kBasinMid, stream);
+  if (e == hipSuccess) e = launch_sweep<256, false, false>(a, units, &lo, kBasinTiny, stream);
   if (e == hipSuccess) e = launch_sweep<256, false, false>(a, units, &lo, kBasinSmall, stream);
   if (e == hipSuccess) e = launch_sweep<512, false, false>(a, units, &lo, kBasinMid, stream);
   if (e == hipSuccess) e = launch_sweep<1024, false, false>(a, units, &lo, kBasinMax12, stream);
