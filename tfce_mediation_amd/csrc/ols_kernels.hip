@@ -143,51 +143,75 @@ __global__ __launch_bounds__(256) void ols_fixed_kernel(OlsFixedArgs a) {
   a.r0[v] = a.yy[v] - ss;
 }
 
-// One workgroup per permutation: Gram matrix of X_p = [F, Z[perm]], its
+// One workgroup (a wave) per permutation: Gram matrix of X_p = [F, Z[perm]], its
 // Cholesky factor and the inverse factor (FP64), stored as float for the
-// epilogue, plus [(X'X)^-1]_cc per contrast in FP64.
+// epilogue, plus [(X'X)^-1]_cc per contrast in FP64.  Bound by latency: the rows
+// that the permutation picks are brought to LDS by the whole wave, kFactorRows at
+// a time (one lane per sum reading them itself waited for memory twice per row),
+// and the factors lie in LDS, a lane per row or column.  Every sum is one chain
+// in row order.  250 rows, 4 fixed and 2 permuted columns, 128 permutations: 103 -> 15 us.
+constexpr int kFactorRows = 64;
+
 __global__ __launch_bounds__(64) void ols_factor_kernel(OlsFactorArgs a) {
   __shared__ double C[kOlsMaxK * kOlsMaxK];
+  __shared__ double sF[kFactorRows][kOlsMaxK], sZ[kFactorRows][kOlsMaxK];
+  __shared__ double L[kOlsMaxK][kOlsMaxK], Li[kOlsMaxK][kOlsMaxK];
   const int p = blockIdx.x;
   const int tid = threadIdx.x;
   const int32_t* perm = a.perm ? a.perm + (int64_t)p * a.n : nullptr;
-  if (tid < a.f * a.m) {
-    const int q = tid / a.m, b = tid % a.m;
-    double s = 0.0;
-    for (int i = 0; i < a.n; ++i) {
-      int src = perm ? perm[i] : i;
-      if (src < 0 || src >= a.n) { s = NAN; break; }
-      s += a.F[i * a.f + q] * a.Z[src * a.m + b];
-    }
-    C[q * kOlsMaxK + b] = s;
-  }
-  __syncthreads();
-  if (tid != 0) return;
   const int k = a.f + a.m;
-  double G[kOlsMaxK][kOlsMaxK], L[kOlsMaxK][kOlsMaxK], Li[kOlsMaxK][kOlsMaxK];
-  for (int i = 0; i < k; ++i)
-    for (int j = 0; j < k; ++j) {
-      double g;
-      if (i < a.f && j < a.f) g = a.FF[i * a.f + j];
-      else if (i < a.f) g = C[i * kOlsMaxK + (j - a.f)];
-      else if (j < a.f) g = C[j * kOlsMaxK + (i - a.f)];
-      else g = a.ZZ[(i - a.f) * a.m + (j - a.f)];
-      G[i][j] = g;
-      L[i][j] = 0.0;
-      Li[i][j] = 0.0;
+  const bool cross = tid < a.f * a.m;
+  const int cq = cross ? tid / a.m : 0, cb = cross ? tid % a.m : 0;
+  double cs = 0.0;
+  for (int i0 = 0; a.f > 0 && a.m > 0 && i0 < a.n; i0 += kFactorRows) {
+    const int i = i0 + tid;
+    if (i < a.n) {
+      const int src = perm ? perm[i] : i;
+      const bool ok = src >= 0 && src < a.n;  // NaN from there on if not
+      for (int q = 0; q < a.f; ++q) sF[tid][q] = a.F[i * a.f + q];
+      for (int b = 0; b < a.m; ++b) sZ[tid][b] = ok ? a.Z[src * a.m + b] : NAN;
     }
-  for (int j = 0; j < k; ++j) {
-    double d = G[j][j];
-    for (int q = 0; q < j; ++q) d -= L[j][q] * L[j][q];
-    d = d > 0.0 ? sqrt(d) : NAN;
-    L[j][j] = d;
-    for (int i = j + 1; i < k; ++i) {
-      double s = G[i][j];
-      for (int q = 0; q < j; ++q) s -= L[i][q] * L[j][q];
-      L[i][j] = s / d;
+    __syncthreads();
+    if (cross) {
+      const int rows = min(kFactorRows, a.n - i0);
+#pragma unroll 8
+      for (int r = 0; r < rows; ++r) cs += sF[r][cq] * sZ[r][cb];
+    }
+    __syncthreads();
+  }
+  if (cross) C[cq * kOlsMaxK + cb] = cs;
+  L[tid / kOlsMaxK][tid % kOlsMaxK] = 0.0;
+  Li[tid / kOlsMaxK][tid % kOlsMaxK] = 0.0;
+  __syncthreads();
+  const auto gram = [&](int i, int j) -> double {
+    if (i < a.f && j < a.f) return a.FF[i * a.f + j];
+    if (i < a.f) return C[i * kOlsMaxK + (j - a.f)];
+    if (j < a.f) return C[j * kOlsMaxK + (i - a.f)];
+    return a.ZZ[(i - a.f) * a.m + (j - a.f)];
+  };
+  const int row = tid < k ? tid : 0;
+  double g[kOlsMaxK];
+#pragma unroll
+  for (int j = 0; j < kOlsMaxK; ++j) g[j] = j < k ? gram(row, j) : 0.0;
+#pragma unroll
+  for (int j = 0; j < kOlsMaxK; ++j) {
+    if (j < k) {
+      if (tid == j) {
+        double d = g[j];
+        for (int q = 0; q < j; ++q) d -= L[j][q] * L[j][q];
+        L[j][j] = d > 0.0 ? sqrt(d) : NAN;
+      }
+      __syncthreads();
+      if (tid > j && tid < k) {
+        double s = g[j];
+        for (int q = 0; q < j; ++q) s -= L[tid][q] * L[j][q];
+        L[tid][j] = s / L[j][j];
+      }
+      __syncthreads();
     }
   }
-  for (int j = 0; j < k; ++j) {
+  if (tid < k) {
+    const int j = tid;
     Li[j][j] = 1.0 / L[j][j];
     for (int i = j + 1; i < k; ++i) {
       double s = 0.0;
@@ -195,20 +219,20 @@ __global__ __launch_bounds__(64) void ols_factor_kernel(OlsFactorArgs a) {
       Li[i][j] = -s / L[i][i];
     }
   }
+  __syncthreads();
   float* out = a.Linv + (int64_t)p * 64;
-  for (int i = 0; i < 8; ++i)
-    for (int j = 0; j < 8; ++j) out[i * 8 + j] = (i < k && j < k) ? (float)Li[i][j] : 0.0f;
-  for (int c = 0; c < kOlsMaxContrasts; ++c) {
+  out[tid] = (float)Li[tid / kOlsMaxK][tid % kOlsMaxK];
+  if (tid < kOlsMaxContrasts) {
     double s = 0.0;
-    if (c < a.n_con)
-      for (int j = a.con[c]; j < k; ++j) s += Li[j][a.con[c]] * Li[j][a.con[c]];
-    a.dc[(int64_t)p * kOlsMaxContrasts + c] = s;
+    if (tid < a.n_con)
+      for (int j = a.con[tid]; j < k; ++j) s += Li[j][a.con[tid]] * Li[j][a.con[tid]];
+    a.dc[(int64_t)p * kOlsMaxContrasts + tid] = s;
   }
   // Block b with columns B: beta = Li' h, and the extra sum of squares of B
   // given the other columns is beta_B' [(X'X)^-1_BB]^-1 beta_B = |C^-1 beta_B|^2
   // with C C' = (X'X)^-1_BB = (Li' Li)_BB; row r of Rb is sum_s C^-1[r][s]
   // Li[.][B_s], so |Rb h|^2 is that sum of squares.
-  for (int b = 0; b < a.n_blk && a.Rb; ++b) {
+  for (int b = tid; b < a.n_blk && a.Rb; b += 64) {
     int B[kOlsMaxK], w = 0;
     for (int j = 0; j < k; ++j)
       if ((a.blk_mask[b] >> j) & 1u) B[w++] = j;
