@@ -289,3 +289,29 @@ def test_exponents(order, E):
         enh, _, _ = otfce.tfce(*csr, x[p], 2.0, E, exact_pow=True)
         exp = np.float32(enh.max() * np.float32(x[p].max() / np.float32(100)))
         assert abs(int(np.float32(out[p, 0]).view(np.int32)) - int(exp.view(np.int32))) <= (0 if E == 0.5 else 16)
+
+
+@pytest.mark.parametrize("gname", ["loop", "ico4_cut", "plane8", "grid26"])
+def test_self_loops_and_repeats(gname):
+    """Lists that hold the element itself and a neighbour twice: ring-packed rows,
+    tables and tiles give the maxima of the clean graph."""
+    import torch
+    from tfce_mediation_amd.tfce import Adjacency, SurfaceSet
+    rp, col = {"loop": lambda: loop(777), "ico4_cut": lambda: adjacency.induced_subgraph(
+        *synth.icosphere_csr(4), np.random.default_rng(1).random(2562) < 0.5),
+        "plane8": lambda: grid26((1, 30, 41)), "grid26": lambda: grid26((11, 13, 9))}[gname]()
+    V = len(rp) - 1
+    lists = [list(col[rp[v]:rp[v + 1]]) for v in range(V)]
+    for v in range(V):
+        if lists[v] and len(lists[v]) <= 28:
+            if v % 3 == 0:
+                lists[v].insert(len(lists[v]) // 2, v)
+            if v % 5 < 2:
+                lists[v].append(lists[v][0])
+    x = np.random.default_rng(6).standard_normal((3, V)).astype(np.float32)
+    x[1] = np.round(2 * x[1]) / 2
+    d = torch.from_numpy(x).cuda()
+    out = [SurfaceSet([Adjacency(c, 2.0, 1.0)], [0]).batch(d, 3).cpu().numpy()
+           for c in ((rp, col), adjacency.to_csr(lists))]
+    np.testing.assert_array_equal(out[0], out[1])
+    say(f"[gpu] basin sweep, self loops and repeats {gname}")
