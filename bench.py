@@ -516,14 +516,14 @@ def main():
         log(f"[bench] GPU vs CPU null values: max rel diff {rel.max():.2e}, median {np.median(rel):.2e}")
 
     # ---- roofline of the dominant kernel (TFCE sweep) -----------------------
-    # Touch-once algorithmic bytes of the incremental sweep, per image (one
-    # surface, one permutation, one sign) with V elements, A of them active at
-    # the last level and d = nnz / V neighbours on average:
-    #   read the map 4V; write and read each element's activation position 8V;
-    #   read each active element's neighbour list 4dA and gather its
-    #   neighbours' positions 4dA; write and read one union-find node
-    #   {parent, size, value} per active element 24A.
-    #   B = 12 V + (8 d + 24) A
+    # Touch-once algorithmic bytes of the sweep (all its kernels), per image
+    # (one surface, one permutation, one sign) with V elements, A of them active
+    # at the last level and d = nnz / V neighbours on average:
+    #   read the map 4V, once for both signs; write and read each active
+    #   element's pointer (8), its level (4) and its place in the level order
+    #   (4); the neighbour lists, 4 nnz, once per launch.
+    #   B = 4 V / signs + 16 A
+    # (The basins' union-find stays in LDS.)
     # A is counted on the maps of the first timed step with the reference's
     # float32 level sequence (the last threshold >= 0).
     maps = eng.tvalues(perm_batches[args.warmup])
@@ -533,11 +533,11 @@ def main():
     images = 0
     for (rp, col), off in zip(eng.csrs, cfg["offsets"]):
         V_s, nnz_s = len(rp) - 1, len(col)
-        d = nnz_s / V_s
+        touch_bytes += 4.0 * nnz_s
         for sgn in signs:
             x = sgn * maps[:, int(off):int(off) + V_s]
             A = active_counts(x)
-            touch_bytes += float((12.0 * V_s + (8.0 * d + 24.0) * A).sum())
+            touch_bytes += float((4.0 * V_s / n_signs + 16.0 * A).sum())
             level_model_bytes += float(P * (N_THR * (4 * (V_s + 1) + 4 * nnz_s + 8 * V_s) + 8 * V_s))
             images += P
     del maps
@@ -572,8 +572,8 @@ def main():
             "precision": args.precision,
             "plain_fp32_perms_per_s": None if plain is None else round(plain, 3),
             "plain_path": "per permutation, the reference's call structure: one FP32 t map, then one "
-                          "single-image CreateAdjSet.run per surface and sign (tfce_run: the whole-GPU "
-                          "level sweep for surfaces of 32,768 elements and more, one workgroup below)",
+                          "single-image CreateAdjSet.run per surface and sign (tfce_run: the basin sweep "
+                          "of one image)",
             "batched_over_plain": None if plain is None else round(value / plain, 2),
             "batched_fp32_perms_per_s": None if "fp32" not in alt_rate else round(alt_rate["fp32"], 1),
             "batched_over_batched_fp32": None if "fp32" not in alt_rate else round(value / alt_rate["fp32"], 3),
@@ -593,7 +593,7 @@ def main():
             "contraction_frac_of_dense_peak": round(gemm_flops / (gemm_ms * 1e-3) / 1e12 / BF16_PEAK_TFLOPS, 4),
         },
         "roofline": {
-            "kernel": (traffic_kernel or "tfce_batch_kernel") + " (persistent TFCE sweep)",
+            "kernel": (traffic_kernel or "basin_sweep") + " (TFCE sweep, all kernels of a launch)",
             "bound": "hbm",
             "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBS,
@@ -606,8 +606,8 @@ def main():
             "traffic_frac_of_peak": None if traffic is None else round(traffic / (tfce_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
             "algorithmic_bytes_per_launch": int(touch_bytes),
             "images_per_launch": images,
-            "byte_model": "touch-once: B = 12 V + (8 d + 24) A per image (V elements, A active at the last "
-                          "level, d neighbours per element)",
+            "byte_model": "touch-once: B = 4 V / signs + 16 A per image (V elements, A active at the last "
+                          "level) and the neighbour lists once per launch",
             "level_sweep_model_frac": round(level_model_bytes / (tfce_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 3),
         },
         "cpu_baseline": None if cpu is None else {

@@ -119,9 +119,11 @@ int tfce_geodesic_destroy(tfce_geodesic_t *pairs);
  * enhn += TFCE(image) over V float32 elements (accumulate != 0), or
  * enhn = TFCE(image) (accumulate == 0).  dh == 0 gives the reference's step
  * fl(max/100); dh > 0 an explicit step.  minT is 0 as in tfce.pyx:45.  A
- * symmetric surface of 32,768 elements or more is swept over the whole GPU
- * (a cooperative launch, levels in lock step), a smaller one by one
- * workgroup; tfce_set_single_image_mode changes the choice, not the values. */
+ * symmetric surface is swept through the basins of the image's local maxima
+ * (dh == 0; with an explicit step, or more basins than LDS holds: element by
+ * element, from 32,768 elements on over the whole GPU in a cooperative launch,
+ * levels in lock step); tfce_set_single_image_mode changes the choice, not the
+ * values. */
 int tfce_run(tfce_adj_t *adj, const float *d_image, float *d_enhn, float dh, int accumulate,
              hipStream_t stream);
 
@@ -359,29 +361,29 @@ int tfce_batch_ex(const tfce_surfset_t *set, const float *d_maps, int64_t map_st
                   float *d_own, int32_t *d_status, hipStream_t stream);
 
 /* How tfce_run / tfce_run_ex sweep one image of a symmetric surface: mode -1
- * (default) over the whole GPU for surfaces of at least 32,768 elements and in
- * one workgroup below that, 0 always in one workgroup, 1 always over the whole
- * GPU; max_workgroups > 0 caps the whole-GPU grid (0: one workgroup per
- * compute unit).  Both give the same values bit for bit; the labels debug
- * output of tfce_run_ex always takes the one-workgroup sweep.  Process-wide.
- * No counterpart in the reference. */
+ * (default) through the basins of its local maxima, 0 element by element in
+ * one workgroup, 1 element by element over the whole GPU; max_workgroups > 0
+ * caps the whole-GPU grid (0: one workgroup per compute unit).  All give the
+ * same values bit for bit; the labels debug output of tfce_run_ex always takes
+ * the one-workgroup sweep, and an image of more basins than LDS holds the
+ * whole-GPU one.  Process-wide.  No counterpart in the reference. */
 int tfce_set_single_image_mode(int32_t mode, int32_t max_workgroups);
 
 /* Number of resident workgroups per CU used by the TFCE sweep (autotuner knob). */
 int tfce_set_occupancy(int32_t wgs_per_cu);
 
-/* Batched maxima (tfce_batch*, tfce_batch_max*) of symmetric surfaces of at
- * most 13,248 elements with a neighbour table run in an LDS-resident sweep
- * (the whole union-find of an image in one compute unit's LDS) unless this
- * process-wide knob is 0; the maxima are the same bit for bit either way.
- * No counterpart in the reference. */
+/* Element-wise maxima (tfce_batch_max_noalloc, whose scratch has no room for
+ * the basin sweep) of symmetric surfaces of at most 13,248 elements with a
+ * neighbour table run in an LDS-resident sweep (the whole union-find of an image
+ * in one compute unit's LDS) unless this process-wide knob is 0; the maxima are
+ * the same bit for bit either way.  No counterpart in the reference. */
 int tfce_set_lds_sweep(int32_t enable);
 
-/* Batched maxima of both signs (sign_mask 3) over ring-packed surfaces (closed
- * triangle meshes of at most six neighbours per vertex) run both signs of a map
- * in one workgroup, sharing one pass over the map and the vertices, unless
- * this process-wide knob is 0; the maxima are the same bit for bit either way.
- * No counterpart in the reference. */
+/* Element-wise maxima of both signs (sign_mask 3; as above) over ring-packed
+ * surfaces (closed triangle meshes of at most six neighbours per vertex) run
+ * both signs of a map in one workgroup, sharing one pass over the map and the
+ * vertices, unless this process-wide knob is 0; the maxima are the same bit for
+ * bit either way.  No counterpart in the reference. */
 int tfce_set_pair_sweep(int32_t enable);
 
 /* ---------------------------------------------------- learned early stop */

@@ -3,14 +3,13 @@
 * the workgroup tile of the split-precision contraction
   (``tfce_ols_set_tile``: 256 x 128, 512 x 64, 512 x 128 or 256 x 256 rows x
   elements);
-* the number of resident sweep workgroups per compute unit
-  (``tfce_set_occupancy``): more hide more latency, fewer keep more of each
-  slot's scratch in cache;
-* whether surfaces of at most 13,248 elements take the LDS-resident sweep
-  (``tfce_set_lds_sweep``; one workgroup per compute unit holding both signs
-  of a map) or the global-memory sweep, and whether ring-packed surfaces
-  sweep both signs of a map in one workgroup (``tfce_set_pair_sweep``); each
-  alternative must give the same maxima bit for bit, and the faster is kept.
+* the number of resident workgroups per compute unit of the element-wise sweep
+  (``tfce_set_occupancy``), whether it takes surfaces of at most 13,248
+  elements in LDS (``tfce_set_lds_sweep``) and both signs of a map in one
+  workgroup (``tfce_set_pair_sweep``).  The batched maxima of symmetric
+  surfaces go through the basin sweep, which has no knobs: on a workload of
+  such surfaces these candidates time the same kernels, and any choice is as
+  good.  Each alternative must give the same maxima bit for bit.
 
 Each candidate is timed with HIP events on the real workload (one batch of P
 permutations of an engine), the contraction and the sweep separately since

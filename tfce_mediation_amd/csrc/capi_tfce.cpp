@@ -81,8 +81,9 @@ static std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
 static int g_wgs_per_cu = 4;
 static bool g_lds_sweep = true;  // small surfaces in the LDS-resident sweep
 static bool g_pair_sweep = true;  // both signs of a map in one workgroup (ring-packed MAX sweeps)
-// tfce_run on one image: -1 the whole-GPU sweep for symmetric surfaces of at
-// least kCoopMinV elements, 0 never, 1 for every symmetric surface
+// tfce_run on one image: -1 the basin sweep, with the whole-GPU sweep behind it
+// for symmetric surfaces of at least kCoopMinV elements; 0 one workgroup; 1 the
+// whole-GPU sweep for every symmetric surface
 static int g_coop_mode = -1;
 static int g_coop_grid = 0;
 constexpr int32_t kCoopMinV = 32768;
