@@ -107,3 +107,45 @@ def test_single_design_in_fp64(n, k, V):
     for name, ref in (("coef", coef), ("resid", res), ("sse", (res ** 2).sum(0)), ("sumyy", (y ** 2).sum(0))):
         assert np.linalg.norm(got[name] - ref) <= 1e-10 * np.linalg.norm(ref), name
     assert np.abs(got["sumy"] - y.sum(0)).max() <= 1e-10 * np.abs(y).sum(0).max()
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 129])
+def test_factors_around_the_rows_in_lds(n):
+    """Permuted columns beside two covariates that stay (a Gram matrix per
+    permutation), row counts around the 64 that the factor kernel holds."""
+    import torch
+    from tfce_mediation_amd.ols import PermutedOLS
+    rng = np.random.default_rng(n)
+    V, P = 150, 6
+    X = np.column_stack([np.ones(n), rng.standard_normal((n, 4))]).astype(np.float32).astype(np.float64)
+    Y = rng.standard_normal((n, V)).astype(np.float32)
+    perms = np.stack([rng.permutation(n) for _ in range(P)]).astype(np.int32)
+    model = PermutedOLS(torch.from_numpy(Y).cuda(), X, contrasts=[4, 3], perm_columns=[3, 4])
+    t = model.t(torch.from_numpy(perms).cuda()).cpu().numpy().astype(np.float64)
+    ref = np.stack([t64(X, Y.astype(np.float64), p, [3, 4], [4, 3]) for p in perms], 1)
+    assert np.linalg.norm(t - ref) <= 1e-5 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("P", [1, 96, 192, 193, 300])
+@pytest.mark.parametrize("V", [700, 70001])
+def test_mediation_tiles_agree(V, P):
+    """The tile that the mediation's contraction takes by its size against the
+    others: the same z bit for bit (the k order does not depend on the tile)."""
+    import torch
+    from tfce_mediation_amd import _lib
+    from tfce_mediation_amd.randomise import MediationModel
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(P)
+    n = 40
+    rng = np.random.default_rng(P)
+    Y = torch.randn((n, V), generator=gen, device="cuda")
+    perms = torch.from_numpy(np.stack([rng.permutation(n) for _ in range(P)]).astype(np.int32)).cuda()
+    model = MediationModel(Y, rng.standard_normal(n), rng.standard_normal(n), "I")
+    lib = _lib.lib()
+    auto = model.z(perms).clone()
+    try:
+        for tile in (1, 2, 3):
+            _lib.check(lib.tfce_ols_set_tile(tile))
+            assert torch.equal(auto, model.z(perms)), tile
+    finally:
+        _lib.check(lib.tfce_ols_set_tile(0))
